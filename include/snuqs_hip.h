@@ -153,10 +153,16 @@ int sq_program_destroy(void *program);
  * have finished.  A captured hipGraph is dropped (recaptured on the next
  * sq_program_run_graph); tuned launch shapes are kept. */
 int sq_program_set_matrices(void *program, const double *matrices, void *stream);
-/* Number of kernels a run launches and its algorithmic HBM bytes
+/* Number of gate sweeps of a run (one kernel launch each when the gates run
+ * one by one, as in sq_program_run_timed; sq_program_run applies several gates
+ * to a pass over the state where it can) and their algorithmic HBM bytes
  * (2 x touched amplitudes x itemsize, summed over the gates). */
 int sq_program_stats(void *program, uint64_t *num_launches,
                      double *algorithmic_bytes);
+/* Apply every gate (asynchronous on `stream`).  Gates are grouped at creation
+ * into passes: the gates of a pass act inside chunks of up to 2^13 amplitudes
+ * held on chip, so the state is read and written once per pass.  Gates are
+ * reordered only past gates they share no target with. */
 int sq_program_run(void *program, void *sv, uint64_t num_elems, void *stream);
 /* sq_program_run through a hipGraph (no reference counterpart; the reference
  * launches one kernel per Python call, simulation.py:274-284): the launch
@@ -164,8 +170,8 @@ int sq_program_run(void *program, void *sv, uint64_t num_elems, void *stream);
  * calls with the same state; another state (or sq_program_tune) recaptures.
  * Asynchronous on `stream` like sq_program_run. */
 int sq_program_run_graph(void *program, void *sv, uint64_t num_elems, void *stream);
-/* Measurement variant of sq_program_run: records a HIP event before every
- * launch and one after the last on `stream`, waits for completion and writes
+/* Measurement variant of sq_program_run: every gate as a launch of its own
+ * kernel, with a HIP event recorded before each and one after the last on `stream`, waits for completion and writes
  * each gate's elapsed time to ms_per_gate[num_gates] (0 for gates that
  * launch nothing). */
 int sq_program_run_timed(void *program, void *sv, uint64_t num_elems,
@@ -192,7 +198,8 @@ int sq_program_gate_info(void *program, uint32_t gate, int *kernel_class,
  * One gate structure, num_sets parameter sets: the states are num_sets
  * consecutive blocks of num_elems = 2^num_qubits amplitudes in one device
  * buffer (state y at states + y * num_elems), and every gate of the batch
- * runs as ONE launch over all of them, each state with its own matrix.
+ * (or pass of several gates, as in sq_program_run) runs as ONE launch over all
+ * of them, each state with its own matrices.
  * `matrices` holds set 0's gate matrices in the layout of sq_program_create,
  * then set 1's, and so on; the sets must use the same targets per gate.  A
  * gate whose sets' matrices fall into different classes (e.g. an angle of 0
@@ -213,7 +220,8 @@ int sq_batch_run(void *batch, void *states, uint64_t num_elems, void *stream);
  * and replayed on later calls with the same states. */
 int sq_batch_run_graph(void *batch, void *states, uint64_t num_elems,
                        void *stream);
-/* Launches per run and algorithmic HBM bytes per run (all states). */
+/* Gate sweeps per run (as sq_program_stats) and their algorithmic HBM bytes,
+ * all states. */
 int sq_batch_stats(void *batch, uint64_t *num_launches,
                    double *algorithmic_bytes);
 /* |0...0> in each of num_sets consecutive states (one launch). */

@@ -25,7 +25,9 @@ ARCH = "gfx950"
 
 HIP_SOURCES = [
     "gate_plan.cpp",
+    "pass_plan.cpp",
     "kernels_gate.hip",
+    "kernels_pass.hip",
     "kernels_reduce.hip",
     "kernels_sample.hip",
     "kernels_qaoa.hip",

@@ -20,6 +20,7 @@
 #include "kernels_qaoa.hpp"
 #include "kernels_cbatch.hpp"
 #include "kernels_reduce.hpp"
+#include "pass_plan.hpp"
 
 namespace sq {
 const std::string &last_error();
@@ -295,6 +296,62 @@ int sq_apply(void *sv, sq_dtype_t dt, uint64_t n, uint32_t num_qubits,
 // ---- programs -----------------------------------------------------------------
 namespace sq {
 
+// The steps of a program or batch (plan_passes) and where each pass's device
+// data sits: descriptors at `desc`, set y's matrices at `image + y * stride`.
+struct PassSet {
+  std::vector<Step> steps;
+  std::vector<PassPlan> plans;
+  std::vector<PassGeom> geoms;
+  std::vector<std::vector<PassBlock>> blocks;
+  std::vector<size_t> desc, image, stride;  // bytes
+  size_t total = 0;                         // bytes of descriptors and nsets images
+};
+
+// Plan the passes of a gate list.  The plan depends on the targets and on
+// the plans' touched fractions at creation; later matrices of the same gates
+// run on the same steps.
+static void plan_pass_set(int nq, sq_dtype_t dt, uint32_t nsets, const std::vector<int> &nt,
+                          const std::vector<size_t> &toff, const std::vector<uint32_t> &targets,
+                          const std::vector<double> &touched, PassSet *ps) {
+  std::vector<uint64_t> masks(nt.size(), 0);
+  for (size_t g = 0; g < nt.size(); ++g)
+    for (int t = 0; t < nt[g]; ++t) masks[g] |= 1ull << (nq - 1 - (int)targets[toff[g] + t]);
+  *ps = PassSet{};
+  plan_passes(nq, dt, masks, touched, &ps->steps, &ps->plans);
+  for (const PassPlan &p : ps->plans) {
+    size_t bytes;
+    ps->geoms.push_back(pass_geom(p));
+    ps->blocks.push_back(pass_blocks(p, dt, &bytes));
+    ps->desc.push_back(ps->total);
+    ps->total += (ps->blocks.back().size() * sizeof(PassBlock) + 255) / 256 * 256;
+    ps->image.push_back(ps->total);
+    ps->stride.push_back(bytes);
+    ps->total += nsets * bytes;
+  }
+}
+
+// Host image of a pass set: `gates.matrices` is set 0's matrices, set y's lie
+// set_doubles further on.
+static void pass_set_image(const PassSet &ps, sq_dtype_t dt, uint32_t nsets, PassGates gates,
+                           size_t set_doubles, char *img) {
+  const double *m0 = gates.matrices;
+  for (size_t i = 0; i < ps.plans.size(); ++i) {
+    std::memcpy(img + ps.desc[i], ps.blocks[i].data(), ps.blocks[i].size() * sizeof(PassBlock));
+    for (uint32_t y = 0; y < nsets; ++y) {
+      gates.matrices = m0 + y * set_doubles;
+      pass_image(ps.plans[i], ps.blocks[i], dt, gates, img + ps.image[i] + y * ps.stride[i]);
+    }
+  }
+}
+
+static int launch_pass_step(const PassSet &ps, int i, sq_dtype_t dt, void *sv, uint64_t nelems,
+                            uint32_t nsets, const void *dev, hipStream_t st) {
+  const char *d = (const char *)dev;
+  return launch_pass(ps.plans[i], ps.geoms[i], dt, sv, nelems, nsets,
+                     (const PassBlock *)(d + ps.desc[i]), (int)ps.blocks[i].size(),
+                     d + ps.image[i], ps.stride[i], st);
+}
+
 struct Program {
   sq_dtype_t dt;
   int nq;
@@ -311,6 +368,8 @@ struct Program {
   size_t dev_cap = 0;                  // bytes of dev_mats
   uint64_t launches = 0;
   double bytes = 0.0;
+  PassSet passes;                      // the forward run's steps
+  void *dev_pass = nullptr;            // pass descriptors and matrices
   // hipGraph of the forward launch sequence on one state (sq_program_run_graph)
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
@@ -428,6 +487,35 @@ static std::vector<char> program_image(Program *p) {
   return img;
 }
 
+// The passes' descriptors and matrices, from the program's matrices.
+static int upload_passes(Program *p, hipStream_t st) {
+  if (!p->passes.total) return SQ_OK;
+  std::vector<char> img(p->passes.total);
+  pass_set_image(p->passes, p->dt, 1,
+                 PassGates{p->mats.data(), &p->moffs, &p->toff, &p->targets, &p->nt, p->nq}, 0,
+                 img.data());
+  SQ_HIP(hipMemcpyAsync(p->dev_pass, img.data(), img.size(), hipMemcpyHostToDevice, st));
+  SQ_HIP(hipStreamSynchronize(st));
+  return SQ_OK;
+}
+
+// The program's forward launches: its steps, or every gate on its own kernel
+// where the state is not on the 16-byte boundary that the passes need.
+static int program_launches(Program *p, void *sv, uint64_t n, hipStream_t st) {
+  if ((uintptr_t)sv & 15) {
+    for (size_t g = 0; g < p->fwd.size(); ++g)
+      SQ_TRY(launch_plan(p->fwd[g], sv, p->dt, n, st, p->fwd_dev[g]));
+    return SQ_OK;
+  }
+  for (const Step &s : p->passes.steps) {
+    if (s.pass >= 0)
+      SQ_TRY(launch_pass_step(p->passes, s.pass, p->dt, sv, n, 1, p->dev_pass, st));
+    else
+      SQ_TRY(launch_plan(p->fwd[s.gate], sv, p->dt, n, st, p->fwd_dev[s.gate]));
+  }
+  return SQ_OK;
+}
+
 }  // namespace sq
 
 extern "C" {
@@ -471,6 +559,23 @@ int sq_program_create(void **program, sq_dtype_t dt, uint32_t nq, uint32_t ng,
       return fail(SQ_ERR_HIP, "program matrices: upload failed");
     }
   }
+  std::vector<double> touched;
+  for (const GatePlan &g : prog->fwd) touched.push_back(g.touched);
+  plan_pass_set(prog->nq, dt, 1, prog->nt, prog->toff, prog->targets, touched, &prog->passes);
+  if (prog->passes.total) {
+    if (hipMalloc(&prog->dev_pass, prog->passes.total) != hipSuccess) {
+      (void)hipGetLastError();  // no room for the passes' matrices: gate by gate
+      prog->dev_pass = nullptr;
+      prog->passes = PassSet{};
+      for (uint32_t g = 0; g < ng; ++g) prog->passes.steps.push_back({(int)g, -1});
+    }
+    const int rc = upload_passes(prog.get(), nullptr);
+    if (rc != SQ_OK) {
+      if (prog->dev_pass) (void)hipFree(prog->dev_pass);
+      if (prog->dev_mats) (void)hipFree(prog->dev_mats);
+      return rc;
+    }
+  }
   *program = prog.release();
   return SQ_OK;
 }
@@ -489,13 +594,14 @@ int sq_program_set_matrices(void *program, const double *matrices, void *stream)
     SQ_HIP(hipMemcpyAsync(p->dev_mats, img.data(), p->dev_cap, hipMemcpyHostToDevice, st));
     SQ_HIP(hipStreamSynchronize(st));
   }
-  return SQ_OK;
+  return upload_passes(p, st);
 }
 
 int sq_program_destroy(void *program) {
   Program *p = (Program *)program;
   if (!p) return SQ_OK;
   drop_graph(p);
+  if (p->dev_pass) SQ_HIP(hipFree(p->dev_pass));
   if (p->dev_mats) SQ_HIP(hipFree(p->dev_mats));
   delete p;
   return SQ_OK;
@@ -700,8 +806,7 @@ int sq_program_run_graph(void *program, void *sv, uint64_t n, void *stream) {
     int rc = SQ_OK;
     if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess)
       rc = fail(SQ_ERR_HIP, "hipStreamBeginCapture failed");
-    for (size_t g = 0; g < p->fwd.size() && rc == SQ_OK; ++g)
-      rc = launch_plan(p->fwd[g], sv, p->dt, n, cs, p->fwd_dev[g]);
+    if (rc == SQ_OK) rc = program_launches(p, sv, n, cs);
     hipGraph_t gr = nullptr;
     if (hipStreamEndCapture(cs, &gr) != hipSuccess && rc == SQ_OK)
       rc = fail(SQ_ERR_HIP, "hipStreamEndCapture failed");
@@ -735,10 +840,7 @@ int sq_program_run(void *program, void *sv, uint64_t n, void *stream) {
   if (n != (1ull << p->nq))
     return fail(SQ_ERR_INVALID, "program built for " + std::to_string(p->nq) +
                                     " qubits, state has " + std::to_string(n) + " amplitudes");
-  hipStream_t st = (hipStream_t)stream;
-  for (size_t g = 0; g < p->fwd.size(); ++g)
-    SQ_TRY(launch_plan(p->fwd[g], sv, p->dt, n, st, p->fwd_dev[g]));
-  return SQ_OK;
+  return program_launches(p, sv, n, (hipStream_t)stream);
 }
 
 // ---- results ----------------------------------------------------------------
@@ -1996,6 +2098,9 @@ struct Batch {
     uint64_t gstride = 0;         // elements between two sets' blocks
   };
   std::vector<Gate> gates;
+  PassSet passes;             // planned once, at creation
+  size_t pass_off = 0;        // their device data in `dev`
+  std::vector<char> in_pass;  // gates that run inside a pass: no tables of their own
   void *dev = nullptr;
   size_t dev_cap = 0;
   uint64_t launches = 0;
@@ -2033,7 +2138,7 @@ static bool same_structure(const GatePlan &a, const GatePlan &b) {
 // block matrices, and its size.  A gate whose sets' matrices fall into
 // different classes (e.g. RotY(0) = identity next to RotY(0.3)) is planned as
 // a dense gate on all its targets in every set.
-static int plan_batch(Batch *b, const double *matrices, std::vector<char> *img) {
+static int plan_batch(Batch *b, const double *matrices, bool create, std::vector<char> *img) {
   const uint64_t n = 1ull << b->nq;
   const size_t ng = b->nt.size();
   std::vector<Batch::Gate> gates(ng);
@@ -2063,11 +2168,24 @@ static int plan_batch(Batch *b, const double *matrices, std::vector<char> *img) 
         const double *m = matrices + y * b->set_doubles + b->moffs[g];
         SQ_TRY(make_plan(m, t, k, b->nq, b->nq, &P[y], kPlanDense));
       }
-    std::vector<const GatePlan *> pp(b->nsets);
-    for (uint32_t y = 0; y < b->nsets; ++y) {
-      pp[y] = &P[y];
+    for (uint32_t y = 0; y < b->nsets; ++y)
       bytes += 2.0 * P[y].touched * (double)n * itemsize(b->dt);
-    }
+    ++launches;
+  }
+  if (create) {
+    std::vector<double> touched(ng, 0.0);
+    for (size_t g = 0; g < ng; ++g)
+      if (!gates[g].plans.empty()) touched[g] = gates[g].plans[0].touched;
+    plan_pass_set(b->nq, b->dt, b->nsets, b->nt, b->toff, b->targets, touched, &b->passes);
+    b->in_pass.assign(ng, 1);
+    for (const Step &s : b->passes.steps)
+      if (s.gate >= 0) b->in_pass[s.gate] = 0;
+  }
+  for (size_t g = 0; g < ng; ++g) {
+    const std::vector<GatePlan> &P = gates[g].plans;
+    if (P.empty() || b->in_pass[g]) continue;
+    std::vector<const GatePlan *> pp(b->nsets);
+    for (uint32_t y = 0; y < b->nsets; ++y) pp[y] = &P[y];
     tab.resize((tab.size() + 255) / 256 * 256);
     gates[g].tab_off = tab.size();
     SQ_TRY(batch_gate_table(pp.data(), b->nsets, b->dt, n, &tab));
@@ -2078,11 +2196,14 @@ static int plan_batch(Batch *b, const double *matrices, std::vector<char> *img) 
       for (uint32_t y = 0; y < b->nsets; ++y) blocks.push_back({blk_total + y * bb, &P[y]});
       blk_total += b->nsets * bb;
     }
-    ++launches;
   }
-  // image: tables, then blocks (256-byte aligned)
+  // image: tables, blocks, passes (256-byte aligned)
   const size_t tab_bytes = (tab.size() + 255) / 256 * 256;
-  img->assign(tab_bytes + blk_total, 0);
+  b->pass_off = tab_bytes + blk_total;
+  img->assign(b->pass_off + b->passes.total, 0);
+  pass_set_image(b->passes, b->dt, b->nsets,
+                 PassGates{matrices, &b->moffs, &b->toff, &b->targets, &b->nt, b->nq},
+                 b->set_doubles, img->data() + b->pass_off);
   std::memcpy(img->data(), tab.data(), tab.size());
   std::vector<const GatePlan *> bp;
   std::vector<size_t> bo;
@@ -2120,9 +2241,14 @@ static int upload_batch(Batch *b, const std::vector<char> &img, hipStream_t st) 
 
 static int batch_launches(Batch *b, void *states, hipStream_t st) {
   const uint64_t n = 1ull << b->nq;
-  for (auto &gt : b->gates) {
+  const char *d = (const char *)b->dev;
+  for (const Step &s : b->passes.steps) {
+    if (s.pass >= 0) {
+      SQ_TRY(launch_pass_step(b->passes, s.pass, b->dt, states, n, b->nsets, d + b->pass_off, st));
+      continue;
+    }
+    const Batch::Gate &gt = b->gates[s.gate];
     if (gt.plans.empty()) continue;
-    const char *d = (const char *)b->dev;
     SQ_TRY(launch_batch_gate(gt.plans[0], b->dt, n, b->nsets, states, d + gt.tab_off,
                              gt.blk_off == (size_t)-1 ? nullptr : d + gt.blk_off, gt.gstride,
                              st));
@@ -2170,7 +2296,7 @@ int sq_batch_create(void **batch, sq_dtype_t dt, uint32_t nq, uint32_t nsets, ui
   }
   b->set_doubles = moff;
   std::vector<char> img;
-  SQ_TRY(plan_batch(b.get(), matrices, &img));
+  SQ_TRY(plan_batch(b.get(), matrices, true, &img));
   SQ_TRY(upload_batch(b.get(), img, nullptr));
   *batch = b.release();
   return SQ_OK;
@@ -2181,7 +2307,7 @@ int sq_batch_set_matrices(void *batch, const double *matrices, void *stream) {
   if (!b) return fail(SQ_ERR_INVALID, "null batch");
   if (!matrices && !b->nt.empty()) return fail(SQ_ERR_INVALID, "null matrices");
   std::vector<char> img;
-  SQ_TRY(plan_batch(b, matrices, &img));
+  SQ_TRY(plan_batch(b, matrices, false, &img));
   drop_batch_graph(b);
   // work already queued on `stream` may still read the old tables: the new
   // image is copied behind it

@@ -1,0 +1,391 @@
+// pass_plan.cpp -- host side of the multi-gate passes (no device code).
+#include "pass_plan.hpp"
+
+#include <algorithm>
+#include <array>
+#include <cstring>
+
+namespace sq {
+
+// LDS slot of chunk index e: the XOR of slot weights of e's bits.  Weight i
+// is 1 << i with the low bits (5 for complex64: 32 8-byte slots span the
+// banks; 4 for complex128: 16 16-byte slots) replaced by these values, so
+// that the group bits of (nearly) every choice of block targets map onto all
+// banks: any 8 of the 13 complex64 values span the 5 low bits in all but 5 of
+// the 1287 cases, any 7 of the 12 complex128 values always span the 4.
+static const uint32_t kHash64[kPassMaxBits] = {1, 2, 4, 8, 16, 15, 23, 14, 5, 25, 6, 19, 26};
+static const uint32_t kHash128[12] = {1, 2, 4, 8, 3, 9, 14, 7, 6, 12, 13, 11};
+
+static uint32_t slot_weight(sq_dtype_t dt, int i) {
+  if (dt == SQ_COMPLEX64) return (i < 5 ? 0u : 1u << i) | kHash64[i];
+  return (i < 4 ? 0u : 1u << i) | kHash128[i];
+}
+
+namespace {
+
+// Next unplaced gate of each bit (position in Planner::perbit).
+using Front = std::array<int, 64>;
+
+struct Planner {
+  const std::vector<uint64_t> &masks;
+  std::vector<std::vector<int>> perbit;  // gates on each bit, program order
+  Front ptr;
+
+  bool ready(const Front &p, int g) const {
+    for (uint64_t m = masks[g]; m; m &= m - 1) {
+      const int b = __builtin_ctzll(m);
+      if (perbit[b][p[b]] != g) return false;
+    }
+    return true;
+  }
+  int head(const Front &p, int b) const {
+    return p[b] < (int)perbit[b].size() ? perbit[b][p[b]] : -1;
+  }
+  void take(Front &p, int g) const {
+    for (uint64_t m = masks[g]; m; m &= m - 1) p[__builtin_ctzll(m)]++;
+  }
+  // Place every ready gate inside `set`.
+  void absorb(Front &p, uint64_t set, std::vector<int> *out) const {
+    bool progress = true;
+    while (progress) {
+      progress = false;
+      for (uint64_t m = set; m; m &= m - 1) {
+        const int g = head(p, __builtin_ctzll(m));
+        if (g < 0 || (masks[g] & ~set) || !ready(p, g)) continue;
+        take(p, g);
+        out->push_back(g);
+        progress = true;
+      }
+    }
+  }
+};
+
+}  // namespace
+
+// Blocks of a pass: each gate joins the last block that holds one of its bits
+// (or an earlier-made later block) if their union stays within 4 targets or
+// inside a block of 5; gates on 5 targets open their own.
+static void make_blocks(const std::vector<int> &gates, const std::vector<uint64_t> &masks,
+                        uint64_t local, std::vector<PassBlockPlan> *out) {
+  struct B {
+    uint64_t m;
+    std::vector<int> g;
+  };
+  std::vector<B> bl;
+  for (int g : gates) {
+    const uint64_t m = masks[g];
+    int lo = -1;
+    for (int b = (int)bl.size() - 1; b >= 0 && lo < 0; --b)
+      if (bl[b].m & m) lo = b;
+    int best = -1, grow = 99;
+    for (int b = std::max(lo, 0); b < (int)bl.size(); ++b) {
+      const uint64_t u = bl[b].m | m;
+      const int k = __builtin_popcountll(u);
+      if (u != bl[b].m && u != m && k > 4) continue;
+      if (k > kMaxK) continue;
+      const int gr = k - __builtin_popcountll(bl[b].m);
+      if (gr < grow) {
+        grow = gr;
+        best = b;
+      }
+    }
+    if (best < 0) {
+      bl.push_back({m, {g}});
+    } else {
+      bl[best].m |= m;
+      bl[best].g.push_back(g);
+    }
+  }
+  for (auto &b : bl) {
+    // at least 4 bits: identity on the lowest local bits not in the block
+    for (uint64_t f = local & ~b.m; f && __builtin_popcountll(b.m) < 4; f &= f - 1)
+      b.m |= f & -f;
+    PassBlockPlan p;
+    for (uint64_t m = b.m; m; m &= m - 1) p.bits[p.k++] = __builtin_ctzll(m);
+    p.gates = std::move(b.g);
+    out->push_back(std::move(p));
+  }
+}
+
+void plan_passes(int nq, sq_dtype_t dt, const std::vector<uint64_t> &masks,
+                 const std::vector<double> &touched, std::vector<Step> *steps,
+                 std::vector<PassPlan> *passes) {
+  steps->clear();
+  passes->clear();
+  const int ng = (int)masks.size();
+  const bool c64 = dt == SQ_COMPLEX64;
+  const int cmin = c64 ? 10 : 9;      // one 5-target tile
+  const int cmax = c64 ? 13 : 12;     // 64 KiB
+  // Larger chunks hold more gates per pass; from 21 qubits on the chunks
+  // still fill the chip (layered circuits of depth 10, fused: 22 qubits 295 us
+  // with the largest chunk, 356 us with the next smaller; 16 qubits 124 against
+  // 91 us).
+  const int cb = std::min(nq, nq >= 21 ? cmax : cmax - 1);
+  if (nq < cmin) {
+    for (int g = 0; g < ng; ++g) steps->push_back({g, -1});
+    return;
+  }
+  const int run = c64 ? 4 : 3;        // 128-byte runs at least
+  const uint64_t low = (1ull << run) - 1;
+  Planner pl{masks, std::vector<std::vector<int>>(nq), Front{}};
+  std::vector<int> phases;
+  int left = 0;
+  for (int g = 0; g < ng; ++g) {
+    if (!masks[g]) {
+      phases.push_back(g);  // commutes with everything
+      continue;
+    }
+    ++left;
+    for (uint64_t m = masks[g]; m; m &= m - 1) pl.perbit[__builtin_ctzll(m)].push_back(g);
+  }
+  bool phases_placed = phases.empty();
+  std::vector<int> t2, btaken;
+  while (left) {
+    // seed: the earliest ready gate
+    int seed = ng;
+    for (int b = 0; b < nq; ++b) {
+      const int g = pl.head(pl.ptr, b);
+      if (g >= 0 && g < seed && pl.ready(pl.ptr, g)) seed = g;
+    }
+    uint64_t set = low | masks[seed];
+    Front ptr = pl.ptr;
+    std::vector<int> taken;
+    pl.absorb(ptr, set, &taken);
+    while (true) {
+      // grow by the ready gate that brings the most gates per added bit
+      double best = 0.0;
+      uint64_t bset = 0;
+      Front bptr;
+      btaken.clear();
+      for (int b = 0; b < nq; ++b) {
+        const int g = pl.head(ptr, b);
+        if (g < 0 || b != __builtin_ctzll(masks[g]) || !pl.ready(ptr, g)) continue;
+        const uint64_t s2 = set | masks[g];
+        const int add = __builtin_popcountll(s2) - __builtin_popcountll(set);
+        if (__builtin_popcountll(s2) > cb) continue;
+        Front p2 = ptr;
+        t2.clear();
+        pl.absorb(p2, s2, &t2);
+        const double score = (double)t2.size() / add;
+        if (score > best) {
+          best = score;
+          bset = s2;
+          bptr = p2;
+          btaken.swap(t2);
+        }
+      }
+      if (best == 0.0) break;
+      set = bset;
+      ptr = bptr;
+      taken.insert(taken.end(), btaken.begin(), btaken.end());
+    }
+    double sweeps = 0.0;
+    for (int g : taken) sweeps += touched[g];
+    if (taken.size() >= 2 && sweeps > 1.0) {
+      PassPlan p;
+      for (int b = 0; b < nq && __builtin_popcountll(set) < cb; ++b) set |= 1ull << b;
+      p.local = set;
+      p.cb = cb;
+      make_blocks(taken, masks, set, &p.blocks);
+      if (!phases_placed) {
+        p.blocks[0].gates.insert(p.blocks[0].gates.end(), phases.begin(), phases.end());
+        phases_placed = true;
+      }
+      steps->push_back({-1, (int)passes->size()});
+      passes->push_back(std::move(p));
+    } else {
+      for (int g : taken) steps->push_back({g, -1});
+    }
+    pl.ptr = ptr;
+    left -= (int)taken.size();
+  }
+  if (!phases_placed)
+    for (int g : phases) steps->push_back({g, -1});
+}
+
+PassGeom pass_geom(const PassPlan &p) {
+  PassGeom g{};
+  int i = 0;
+  for (uint64_t m = p.local; m; m &= m - 1) g.addr[i++] = m & -m;
+  while ((p.local >> g.shift) & 1) ++g.shift;
+  for (uint64_t m = p.local >> g.shift; m; m &= m - 1) g.lowmask[g.nins++] = (m & -m) - 1;
+  return g;
+}
+
+std::vector<PassBlock> pass_blocks(const PassPlan &p, sq_dtype_t dt, size_t *image_bytes) {
+  const bool c64 = dt == SQ_COMPLEX64;
+  const int ncol = c64 ? 5 : 4;
+  const uint32_t item = c64 ? 8 : 16, banks = c64 ? 31 : 15;
+  std::vector<PassBlock> out;
+  size_t off = 0;
+  for (const PassBlockPlan &b : p.blocks) {
+    PassBlock d{};
+    int chunk_bit[64];
+    int n = 0;
+    for (uint64_t m = p.local; m; m &= m - 1) chunk_bit[__builtin_ctzll(m)] = n++;
+    uint64_t used = 0;
+    for (int j = 0; j < b.k; ++j) {
+      const int i = chunk_bit[b.bits[j]];
+      used |= 1ull << i;
+      d.row[j] = (uint16_t)(slot_weight(dt, i) * item);
+    }
+    // group bits: the lowest bits whose bank images are independent (no two
+    // groups of a row in one bank), topped up if there are not enough
+    uint32_t basis[5];
+    int nb = 0, nc = 0;
+    for (int i = 0; i < p.cb && nc < ncol; ++i) {
+      if ((used >> i) & 1) continue;
+      uint32_t v = slot_weight(dt, i) & banks;
+      for (int q = 0; q < nb; ++q) v = std::min(v, v ^ basis[q]);
+      if (!v) continue;
+      basis[nb++] = v;
+      d.col[nc++] = (uint16_t)(slot_weight(dt, i) * item);
+      used |= 1ull << i;
+    }
+    int nw = 0;
+    for (int i = 0; i < p.cb; ++i) {
+      if ((used >> i) & 1) continue;
+      const uint16_t w = (uint16_t)(slot_weight(dt, i) * item);
+      if (nc < ncol) d.col[nc++] = w; else d.wave[nw++] = w;
+    }
+    d.k = (uint16_t)b.k;
+    const size_t bytes = b.k == 5 ? 16384 : (c64 ? 4096 : 8192);
+    d.n16 = (uint16_t)(bytes / 16);
+    d.goff = (uint32_t)(off / 16);
+    off += bytes;
+    out.push_back(d);
+  }
+  *image_bytes = off;
+  return out;
+}
+
+// The block's complex128 matrix (local index bit j = bits[j]), row-major, real
+// and imaginary parts apart.
+struct BlockMatrix {
+  alignas(64) double re[32 * 32], im[32 * 32];
+};
+
+static void block_matrix(const PassBlockPlan &b, const PassGates &pg, BlockMatrix *M) {
+  const int d = 1 << b.k;
+  bool first = true;
+  alignas(64) double xr[32 * 32], xi[32 * 32];
+  for (int g : b.gates) {
+    const double *m = pg.matrices + (*pg.moffs)[g];
+    const int k = (*pg.nt)[g], dk = 1 << k;
+    // local offset of the gate's index r (reference order: targets[0] the MSB)
+    int off[1 << kMaxK] = {0}, mask = 0;
+    for (int t = 0; t < k; ++t) {
+      const int bit = pg.nq - 1 - (int)(*pg.targets)[(*pg.toff)[g] + t];
+      int j = 0;
+      while (b.bits[j] != bit) ++j;
+      mask |= 1 << j;
+      for (int r = 0; r < dk; ++r)
+        if ((r >> (k - 1 - t)) & 1) off[r] |= 1 << j;
+    }
+    if (first) {  // the gate itself, the identity on the other bits
+      first = false;
+      std::fill(M->re, M->re + d * d, 0.0);
+      std::fill(M->im, M->im + d * d, 0.0);
+      for (int base = 0; base < d; ++base) {
+        if (base & mask) continue;
+        for (int r = 0; r < dk; ++r)
+          for (int s = 0; s < dk; ++s) {
+            M->re[(base | off[r]) * d + (base | off[s])] = m[2 * (r * dk + s)];
+            M->im[(base | off[r]) * d + (base | off[s])] = m[2 * (r * dk + s) + 1];
+          }
+      }
+      continue;
+    }
+    bool diag = true;
+    for (int r = 0; r < dk && diag; ++r)
+      for (int s = 0; s < dk && diag; ++s)
+        diag = r == s || (m[2 * (r * dk + s)] == 0.0 && m[2 * (r * dk + s) + 1] == 0.0);
+    if (diag) {
+      for (int base = 0; base < d; ++base) {
+        if (base & mask) continue;
+        for (int r = 0; r < dk; ++r) {
+          const double mr = m[2 * (r * dk + r)], mi = m[2 * (r * dk + r) + 1];
+          double *yr = M->re + (base | off[r]) * d, *yi = M->im + (base | off[r]) * d;
+          for (int c = 0; c < d; ++c) {
+            const double a = yr[c];
+            yr[c] = mr * a - mi * yi[c];
+            yi[c] = mr * yi[c] + mi * a;
+          }
+        }
+      }
+      continue;
+    }
+    for (int base = 0; base < d; ++base) {
+      if (base & mask) continue;
+      for (int s = 0; s < dk; ++s) {
+        std::memcpy(xr + s * d, M->re + (base | off[s]) * d, d * sizeof(double));
+        std::memcpy(xi + s * d, M->im + (base | off[s]) * d, d * sizeof(double));
+      }
+      for (int r = 0; r < dk; ++r) {
+        double *yr = M->re + (base | off[r]) * d, *yi = M->im + (base | off[r]) * d;
+        for (int c = 0; c < d; ++c) yr[c] = yi[c] = 0.0;
+        for (int s = 0; s < dk; ++s) {
+          const double mr = m[2 * (r * dk + s)], mi = m[2 * (r * dk + s) + 1];
+          if (mr == 0.0 && mi == 0.0) continue;
+          const double *ar = xr + s * d, *ai = xi + s * d;
+          for (int c = 0; c < d; ++c) {
+            yr[c] += mr * ar[c] - mi * ai[c];
+            yi[c] += mr * ai[c] + mi * ar[c];
+          }
+        }
+      }
+    }
+  }
+}
+
+void pass_image(const PassPlan &p, const std::vector<PassBlock> &blocks, sq_dtype_t dt,
+                const PassGates &pg, char *img) {
+  const bool c64 = dt == SQ_COMPLEX64;
+  BlockMatrix M;
+  for (size_t i = 0; i < blocks.size(); ++i) {
+    const PassBlockPlan &b = p.blocks[i];
+    block_matrix(b, pg, &M);
+    const int d = 1 << b.k;
+    char *dst = img + (size_t)blocks[i].goff * 16;
+    if (b.k == 5) {
+      // entry (o, r): {Re, Im, Re + Im, 0} (complex64), {Re, Im} (complex128)
+      for (int o = 0; o < d; ++o)
+        for (int r = 0; r < d; ++r) {
+          const double re = M.re[r * d + o], im = M.im[r * d + o];
+          if (c64) {
+            float *e = (float *)dst + 4 * (o * d + r);
+            e[0] = (float)re;
+            e[1] = (float)im;
+            e[2] = (float)(re + im);
+            e[3] = 0.f;
+          } else {
+            double *e = (double *)dst + 2 * (o * d + r);
+            e[0] = re;
+            e[1] = im;
+          }
+        }
+      continue;
+    }
+    // real form: row 2r + c, column 2o + c', column-major
+    for (int o = 0; o < d; ++o)
+      for (int r = 0; r < d; ++r) {
+        const double re = M.re[r * d + o], im = M.im[r * d + o];
+        const int e0 = 2 * o * 32 + 2 * r, e1 = e0 + 32;
+        if (c64) {
+          float *f = (float *)dst;
+          f[e0] = (float)re;
+          f[e0 + 1] = (float)im;
+          f[e1] = (float)-im;
+          f[e1 + 1] = (float)re;
+        } else {
+          double *f = (double *)dst;
+          f[e0] = re;
+          f[e0 + 1] = im;
+          f[e1] = -im;
+          f[e1 + 1] = re;
+        }
+      }
+  }
+}
+
+}  // namespace sq

@@ -1,0 +1,89 @@
+// pass_plan.hpp -- grouping of a gate list into multi-gate passes.
+//
+// A pass applies several gates of a program in one sweep over the state: a
+// workgroup holds a chunk of 2^cb amplitudes (the pass's local bits vary, the
+// others are fixed) in LDS, applies every gate of the pass there and writes
+// the chunk back, so the state crosses HBM once per pass instead of once per
+// gate.  No reference counterpart (the reference sweeps the state once per
+// gate, gate_operations_impl_cuda.cu:13-175).
+#pragma once
+
+#include <cstdint>
+#include <vector>
+
+#include "sq_common.hpp"
+
+namespace sq {
+
+constexpr int kPassMaxBits = 13;  // largest chunk: 2^13 complex64 amplitudes = 64 KiB of LDS
+
+// One matrix of a pass: the product of `gates` (program order) on the state
+// bits bits[0..k-1] (ascending, k = 4 or 5).
+struct PassBlockPlan {
+  int k = 0;
+  int bits[kMaxK] = {0};
+  std::vector<int> gates;
+};
+
+struct PassPlan {
+  uint64_t local = 0;  // state bits that vary inside a chunk
+  int cb = 0;          // their number
+  std::vector<PassBlockPlan> blocks;
+};
+
+// A program as a sequence of steps: one gate on its own kernel, or one pass.
+struct Step {
+  int gate = -1;
+  int pass = -1;
+};
+
+// Steps of a gate list on an nq-bit state.  masks[g]: the state bits gate g
+// acts on (0 for a global phase); touched[g]: the fraction of the amplitudes
+// it changes.  Gates are reordered only past gates they share no bit with.
+void plan_passes(int nq, sq_dtype_t dt, const std::vector<uint64_t> &masks,
+                 const std::vector<double> &touched, std::vector<Step> *steps,
+                 std::vector<PassPlan> *passes);
+
+// Device form of one block: byte offsets in the chunk's LDS image that the
+// block's column (group), wave and row (amplitude) index bits stand for; an
+// element's offset is the XOR of its bits' entries.
+struct PassBlock {
+  uint16_t col[5];
+  uint16_t wave[4];
+  uint16_t row[5];
+  uint16_t k;
+  uint16_t n16;   // 16-byte units of the block's matrix image
+  uint32_t goff;  // its offset in the pass's matrix image, 16-byte units
+};
+
+// Geometry of a pass's chunks.
+struct PassGeom {
+  uint64_t addr[kPassMaxBits];     // address stride (amplitudes) of chunk bit i
+  uint64_t lowmask[kPassMaxBits];  // chunk index -> base: insert zero bits here
+  int nins;
+  int shift;                       // local bits 0..shift-1 are inserted by a shift
+};
+
+PassGeom pass_geom(const PassPlan &p);
+// The blocks' device descriptors and, per block, the bytes of its matrix.
+std::vector<PassBlock> pass_blocks(const PassPlan &p, sq_dtype_t dt, size_t *image_bytes);
+// Matrix image of a pass: `matrix(g)` gives gate g's row-major complex128
+// matrix and `targets(g)` / `nt(g)` its targets in the reference's order.
+struct PassGates {
+  const double *matrices;            // all gates' matrices
+  const std::vector<size_t> *moffs;  // gate -> offset in matrices (doubles)
+  const std::vector<size_t> *toff;   // gate -> offset in targets
+  const std::vector<uint32_t> *targets;
+  const std::vector<int> *nt;
+  int nq;
+};
+void pass_image(const PassPlan &p, const std::vector<PassBlock> &blocks, sq_dtype_t dt,
+                const PassGates &g, char *img);
+
+// Launch a pass over nsets states of nelems amplitudes (state y at
+// sv + y * nelems, its matrices at image + y * gstride bytes).
+int launch_pass(const PassPlan &p, const PassGeom &geom, sq_dtype_t dt, void *sv,
+                uint64_t nelems, uint32_t nsets, const PassBlock *blocks, int nblocks,
+                const void *image, uint64_t gstride, hipStream_t stream);
+
+}  // namespace sq

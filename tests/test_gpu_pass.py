@@ -1,0 +1,95 @@
+"""Programs whose gates run several to a pass (kernels_pass.hip): every chunk
+size and the state sizes around it, against the CPU oracle."""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+from helpers import device_state, random_state, run_oracle, to_np
+
+pytestmark = pytest.mark.gpu
+
+# the bars of the gate tests: max-abs error of a unit-norm state
+TOL = {"complex128": 1e-12, "complex64": 1e-5}
+
+
+def _circuit(n, rng, gates):
+    """Random gates of 0-5 targets: all kinds, dense blocks of 4 and 5 targets
+    on random qubits, global phases, controls."""
+    from snuqs_amd.circuits import haar_unitary, random_gate_list
+    from snuqs_amd._C.operation import gate_operations as g
+
+    ops = []
+    for op in random_gate_list(n, gates, rng, with_unitary=True):
+        ops.append(op)
+        if rng.random() < 0.15:
+            k = int(rng.integers(4, 6))
+            ops.append(g.Unitary([int(q) for q in rng.permutation(n)[:k]], haar_unitary(1 << k, rng)))
+    return ops + [g.RotX([int(q) for q in rng.permutation(n)[:3]], 0.7, ctrl_modifiers=[1, 0]),
+                  g.GPhase([], 0.9)]
+
+
+# 8 / 9: below the smallest chunk of complex128 / complex64; 9-13: the state is
+# one chunk; 20 / 21: the largest chunk starts at 21 qubits
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n", [8, 9, 10, 11, 12, 13, 14, 17, 20, 21])
+def test_program_passes_vs_oracle(C, dtype, n):
+    rng = np.random.default_rng(1000 + n)
+    ops = _circuit(n, rng, 60)
+    init = random_state(n, rng, np.complex64 if dtype == "complex64" else np.complex128)
+    ref = run_oracle(n, ops, init.astype(np.complex128))
+    prog = C.functionals.Program(n, ops, dtype=dtype)
+    for use_graph in (False, True):
+        sv = device_state(C, n, dtype, init)
+        prog.run(sv, use_graph=use_graph)
+        assert np.abs(to_np(C, sv) - ref).max() <= TOL[dtype], use_graph
+
+
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+def test_set_gates_from_identities(C, dtype):
+    """A program made with all angles 0 (every gate the identity) runs the
+    gates that later matrices make of it."""
+    from snuqs_amd.circuits import hea_ansatz
+
+    n = 14
+    th = np.random.default_rng(4).uniform(0, 2 * np.pi, 4 * n)
+    prog = C.functionals.Program(n, hea_ansatz(n, 2, 0 * th)[0], dtype=dtype)
+    ops = hea_ansatz(n, 2, th)[0]
+    prog.set_gates(ops)
+    sv = device_state(C, n, dtype)
+    prog.run(sv)
+    assert np.abs(to_np(C, sv) - run_oracle(n, ops)).max() <= TOL[dtype]
+
+
+def test_unaligned_complex64_state(C):
+    """A complex64 state at an odd amplitude (8 bytes past a 16-byte
+    boundary), as a C caller may hold it, gets the same result."""
+    L = ctypes.CDLL(os.path.join(os.path.dirname(C.__file__), "libsnuqs_hip.so"))
+    n = 14
+    rng = np.random.default_rng(6)
+    ops = _circuit(n, rng, 30)
+    init = random_state(n, rng, np.complex64)
+    buf = C.result_types.StateVector(C.DeviceType.CUDA, n + 1, dtype="complex64")
+    host = np.zeros(2 << n, np.complex64)
+    host[1:1 + (1 << n)] = init
+    P = ctypes.c_void_p
+    nt = np.array([len(op.targets) for op in ops], np.uint32)
+    tg = np.array([q for op in ops for q in op.targets], np.uint32)
+    ms = np.concatenate([np.asarray(op.matrix(), np.complex128).ravel() for op in ops])
+    prog = P()
+    L.sq_memcpy_h2d.argtypes = [P, P, ctypes.c_size_t, P]
+    L.sq_program_create.argtypes = [ctypes.POINTER(P), ctypes.c_int, ctypes.c_uint32,
+                                    ctypes.c_uint32, P, P, P]
+    L.sq_program_run.argtypes = [P, P, ctypes.c_uint64, P]
+    L.sq_program_destroy.argtypes = [P]
+    assert L.sq_memcpy_h2d(buf.data_ptr, host.ctypes.data, host.nbytes, None) == 0
+    assert L.sq_program_create(ctypes.byref(prog), 0, n, len(ops), nt.ctypes.data, tg.ctypes.data,
+                               ms.ctypes.data) == 0
+    assert L.sq_program_run(prog, buf.data_ptr + 8, 1 << n, None) == 0
+    C.core.cuda.device_synchronize()
+    out = np.array(buf.cpu(), copy=True)
+    L.sq_program_destroy(prog)
+    got = out[1:1 + (1 << n)].astype(np.complex128)
+    assert np.abs(got - run_oracle(n, ops, init.astype(np.complex128))).max() <= TOL["complex64"]
+    assert out[0] == 0 and not out[1 + (1 << n):].any()  # nothing beside the state

@@ -340,6 +340,13 @@ int sq_apply_pauli_sum(const void *in, void *out, sq_dtype_t dtype,
 int sq_sample(const double *probs, uint64_t num_elems, const double *uniforms,
               uint64_t shots, int exact, int64_t *out, void *stream);
 
+/* sq_sample with p = |sv[i]|^2 of a state (divided by the state's norm^2 when
+ * normalize != 0: the values of sq_probabilities / sq_probabilities_normalized,
+ * formed where they are used instead of stored). */
+int sq_sample_state(const void *sv, sq_dtype_t dtype, uint64_t num_elems,
+                    int normalize, const double *uniforms, uint64_t shots,
+                    int exact, int64_t *out, void *stream);
+
 /* ---- adjoint differentiation (new; no reference counterpart).
  * For the program U = G_{m-1}...G_0 and observable H = sum_t c_t P_t the
  * call runs the forward pass itself (sv <- U|0..0>), returns the energy

@@ -1176,33 +1176,71 @@ int sq_apply_pauli_sum(const void *in, void *out, sq_dtype_t dt, uint64_t n, uin
   return SQ_OK;
 }
 
-int sq_sample(const double *probs, uint64_t n, const double *uniforms, uint64_t shots,
-              int exact, int64_t *out, void *stream) {
-  if (!probs || !is_pow2(n)) return fail(SQ_ERR_INVALID, "bad probabilities");
+// Samples from `probs`, or from the state `sv` when that is given.
+static int sample_from(const double *probs, const void *sv, sq_dtype_t dt, int normalize,
+                       uint64_t n, const double *uniforms, uint64_t shots, int exact,
+                       int64_t *out, void *stream) {
   if (shots == 0) return SQ_OK;
   if (!uniforms || !out) return fail(SQ_ERR_INVALID, "null uniforms or output");
   int dev;
   SQ_TRY(current_device(&dev));
   std::lock_guard<std::mutex> lk(g_ws_mutex[dev]);
   const size_t cdf_b = n * sizeof(double) + 256;
-  const size_t scr_b = sample_scratch_bytes(n, exact != 0) + 256;
   const size_t io_b = shots * 16 + 512;
-  Workspace *w;
-  SQ_TRY(ws_reserve(dev, cdf_b + scr_b + io_b + 1024, io_b, &w));
+  const size_t red_b = (kRedBlocks + 64) * sizeof(double) + 256;
   hipStream_t st = (hipStream_t)stream;
-  char *d = (char *)w->dev;
-  double *cdf = (double *)d;
-  char *scr = al(d + cdf_b);
-  double *du = (double *)al(scr + scr_b);
-  int64_t *dout = (int64_t *)al((char *)du + shots * 8);
-  SQ_TRY(sample_cdf(probs, n, cdf, exact != 0, scr, scr_b, st));
-  std::memcpy(w->host, uniforms, shots * 8);
-  SQ_HIP(hipMemcpyAsync(du, w->host, shots * 8, hipMemcpyHostToDevice, st));
-  SQ_TRY(launch_search(cdf, n, du, shots, dout, st));
-  SQ_HIP(hipMemcpyAsync(w->host, dout, shots * 8, hipMemcpyDeviceToHost, st));
-  SQ_HIP(hipStreamSynchronize(st));
+  Workspace *w;
+  // route 0: exact samples by tiles; 1: a cdf over all elements (fast mode, and
+  // exact mode on entries that are negative or not finite)
+  for (int route = exact ? 0 : 1; route < 2; ++route) {
+    const size_t scr_b =
+        (route ? sample_scratch_bytes(n, exact != 0) : sample_exact_scratch_bytes(n)) + 256;
+    const size_t prob_b = route && sv ? n * sizeof(double) + 256 : 0;
+    SQ_TRY(ws_reserve(dev, cdf_b + scr_b + red_b + prob_b + io_b + 1024, io_b, &w));
+    char *d = (char *)w->dev;
+    double *cdf = (double *)d;
+    char *scr = al(d + cdf_b);
+    double *red = (double *)al(scr + scr_b);
+    double *pr = (double *)al((char *)red + red_b);
+    double *du = (double *)al((char *)pr + prob_b);
+    int64_t *dout = (int64_t *)al((char *)du + shots * 8);
+    int bad = 0;
+    std::memcpy(w->host, uniforms, shots * 8);
+    SQ_HIP(hipMemcpyAsync(du, w->host, shots * 8, hipMemcpyHostToDevice, st));
+    if (sv && normalize) SQ_TRY(launch_norm2(sv, dt, n, red + 32, red, st));
+    if (route == 0) {
+      const int *bad_dev;
+      if (sv)
+        SQ_TRY(sample_exact_state(sv, dt, normalize ? red : nullptr, n, cdf, du, shots, dout, scr,
+                                  &bad_dev, st));
+      else
+        SQ_TRY(sample_exact(probs, n, cdf, du, shots, dout, scr, &bad_dev, st));
+      SQ_HIP(hipMemcpyAsync(&bad, bad_dev, sizeof(int), hipMemcpyDeviceToHost, st));
+    } else {
+      if (sv && normalize) SQ_TRY(launch_probabilities_div(sv, dt, n, pr, red, st));
+      else if (sv) SQ_TRY(launch_probabilities(sv, dt, n, pr, st));
+      SQ_TRY(sample_cdf(sv ? pr : probs, n, cdf, exact != 0, scr, scr_b, st));
+      SQ_TRY(launch_search(cdf, n, du, shots, dout, st));
+    }
+    SQ_HIP(hipMemcpyAsync(w->host, dout, shots * 8, hipMemcpyDeviceToHost, st));
+    SQ_HIP(hipStreamSynchronize(st));
+    if (!bad) break;
+  }
   std::memcpy(out, w->host, shots * 8);
   return SQ_OK;
+}
+
+int sq_sample(const double *probs, uint64_t n, const double *uniforms, uint64_t shots,
+              int exact, int64_t *out, void *stream) {
+  if (!probs || !is_pow2(n)) return fail(SQ_ERR_INVALID, "bad probabilities");
+  return sample_from(probs, nullptr, SQ_COMPLEX64, 0, n, uniforms, shots, exact, out, stream);
+}
+
+int sq_sample_state(const void *sv, sq_dtype_t dt, uint64_t n, int normalize,
+                    const double *uniforms, uint64_t shots, int exact, int64_t *out,
+                    void *stream) {
+  SQ_TRY(check_state(sv, dt, n));
+  return sample_from(nullptr, sv, dt, normalize, n, uniforms, shots, exact, out, stream);
 }
 
 // ---- adjoint ----------------------------------------------------------------

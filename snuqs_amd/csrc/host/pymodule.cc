@@ -299,18 +299,14 @@ py::array_t<double> probabilities(StateVector &sv, bool normalize, std::shared_p
 py::array_t<int64_t> sample(StateVector &sv, py::array_t<double, py::array::c_style> uniforms,
                             bool exact, bool normalize, std::shared_ptr<Stream> stream) {
   sv.require_device("sample");
-  const size_t n = sv.num_elems();
-  void *d;
-  check(sq_malloc(&d, n * sizeof(double)));
-  std::unique_ptr<void, int (*)(void *)> g(d, sq_free);
   py::array_t<int64_t> out(uniforms.size());
   const double *u = uniforms.data();
   int64_t *o = out.mutable_data();
   const size_t shots = uniforms.size();
   {
     py::gil_scoped_release nogil;
-    check(probs_into(sv, (double *)d, normalize, stream));
-    check(sq_sample((const double *)d, n, u, shots, exact ? 1 : 0, o, sraw(stream)));
+    check(sq_sample_state(sv.ptr(), sv.dtype(), sv.num_elems(), normalize ? 1 : 0, u, shots,
+                          exact ? 1 : 0, o, sraw(stream)));
   }
   return out;
 }

@@ -12,10 +12,23 @@
 // binade [2^e, 2^(e+1)) every value is an integer multiple of u = 2^(e-52), so
 // fl(c + p) = (C + d) u with d = p/u rounded to nearest; the increments d do
 // not depend on c except at exact ties (p/u = k + 1/2, broken towards the even
-// result, i.e. by the parity of C), which are rare and resolved in order.  An
-// epoch is therefore an int64 prefix sum: the chain runs binade by binade, the
-// element that leaves the binade is added with one ordinary double add, and
-// the fast FP64 scan bounds where each binade ends.
+// result, i.e. by the parity of C).  A run of elements inside one binade is
+// therefore a map C -> C + D(parity of C), and such maps compose.
+//
+// The elements are cut into tiles of 4096.  A fast FP64 scan of the tile sums
+// bounds c at each tile's start, which leaves one or two candidate binades; one
+// pass forms each tile's map for them.  One workgroup then walks the tiles,
+// 1024 maps per scan; where a scan shows that c leaves the binade inside a
+// tile, that tile's elements are gone through (the crossing element is added
+// with one ordinary double add).  That gives the exact c at every tile's
+// start; a last pass writes the cdf inside the tiles that some uniform falls
+// into.  Nothing waits for the host.  The state is read four times (norm, sums,
+// maps, cdf) and the cdf written once: 2.7 GB at 2^26 complex64 amplitudes,
+// 0.4 ms at copy rate; measured 1.1 ms (norm 0.12, sums 0.09, maps 0.13, chain
+// 0.28, a serial chain of some 70 scans, cdf 0.24, search 0.03), 20 ms with an
+// epoch of launches and host reads per binade.  Inputs that are not finite and
+// non-negative take the older route, an epoch of launches per binade driven by
+// the host.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -256,6 +269,571 @@ int launch_search(const double *cdf, uint64_t n, const double *u_dev, uint64_t s
   return SQ_OK;
 }
 
+// ---- exact mode by tiles -----------------------------------------------------
+constexpr int kTileThreads = 1024;
+constexpr int kTileItems = 4;
+constexpr int kTile = kTileThreads * kTileItems;
+constexpr double kTop = 9007199254740992.0;  // 2^53: C has left the binade
+
+// What a tile does to C (integers held as doubles: exact below 2^53, and sums
+// that reach 2^53 stay there): C -> C + d[C & 1] in binade e, C + d[2 + (C & 1)]
+// in binade e + 1 (both only where kHasNext).
+struct TileMap {
+  double d[4];
+  int e;
+  int flags;
+};
+enum { kAllZero = 1, kHasNext = 2, kTies = 4 };
+
+__device__ __forceinline__ bool odd(double x) {
+  const double h = x * 0.5;
+  return h != floor(h);
+}
+__device__ __forceinline__ int binade(double c) {
+  const int e = (int)((__double_as_longlong(c) >> 52) & 0x7ff) - 1023;
+  return e < -1022 ? -1022 : e;  // subnormals share the first binade's ulp
+}
+// x 2^k, exact unless it leaves the range of doubles (k uniform): one product
+// where 2^k is a normal double, and ldexp beyond.
+struct Scale {
+  double f;
+  int k;
+  __device__ explicit Scale(int k_)
+      : f(k_ >= -1022 && k_ <= 1023 ? __longlong_as_double((int64_t)(k_ + 1023) << 52) : 0.0),
+        k(k_) {}
+  __device__ __forceinline__ double operator()(double x) const { return f != 0.0 ? x * f : ldexp(x, k); }
+};
+// Increments of p (in ulps of the binade that `up` scales by) for C even / odd.
+__device__ __forceinline__ void increments(double p, const Scale &up, double &d0, double &d1) {
+  const double q = up(p);
+  const double r = (q + 0x1p52) - 0x1p52;  // nearest integer, ties to even
+  d0 = d1 = q < 0x1p52 ? r : q;
+  if (fabs(q - d0) == 0.5) {
+    const double k = floor(q), o = odd(k) ? 1.0 : 0.0;
+    d0 = k + o;
+    d1 = k + (1.0 - o);
+  }
+}
+// (a0, a1) followed by (b0, b1).
+__device__ __forceinline__ void then(double &a0, double &a1, double b0, double b1) {
+  a0 += odd(a0) ? b1 : b0;
+  a1 += odd(a1) ? b0 : b1;
+}
+
+// Exclusive scan over the workgroup of the maps (d0, d1): on return (d0, d1) is
+// the composition of the maps of all lower threads, (t0, t1) that of all.
+__device__ __forceinline__ void scan_maps(double &d0, double &d1, double &t0, double &t1) {
+  constexpr int W = kTileThreads / 64;
+  __shared__ double w0[W], w1[W];
+  __shared__ int wp[W];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool wpairs = __any(d0 != d1);
+  double i0 = d0, i1 = d1;
+  if (!wpairs) {  // no ties in this wave: plain sums
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double p0 = __shfl_up(i0, o);
+      if (lane >= o) i0 += p0;
+    }
+    i1 = i0;
+  } else {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      double p0 = __shfl_up(i0, o), p1 = __shfl_up(i1, o);
+      if (lane >= o) {
+        then(p0, p1, i0, i1);
+        i0 = p0;
+        i1 = p1;
+      }
+    }
+  }
+  double e0 = __shfl_up(i0, 1), e1 = wpairs ? __shfl_up(i1, 1) : e0;
+  if (lane == 0) e0 = e1 = 0.0;
+  __syncthreads();  // an earlier call's reads are done
+  if (lane == 63) {
+    w0[wave] = i0;
+    w1[wave] = i1;
+    wp[wave] = wpairs;
+  }
+  __syncthreads();
+  int pairs = 0;
+#pragma unroll
+  for (int v = 0; v < W; ++v) pairs |= wp[v];
+  double a0 = 0.0, a1 = 0.0, s0 = 0.0, s1 = 0.0;
+  if (!pairs) {
+#pragma unroll
+    for (int v = 0; v < W; ++v) {
+      if (v == wave) s0 = a0;
+      a0 += w0[v];
+    }
+    t0 = t1 = a0;
+    d0 = d1 = s0 + e0;
+    return;
+  }
+  for (int v = 0; v < W; ++v) {
+    if (v == wave) {
+      s0 = a0;
+      s1 = a1;
+    }
+    then(a0, a1, w0[v], w1[v]);
+  }
+  t0 = a0;
+  t1 = a1;
+  then(s0, s1, e0, e1);
+  d0 = s0;
+  d1 = s1;
+}
+
+// Smallest of the threads' values.
+__device__ __forceinline__ int block_min(int v) {
+  __shared__ int m[kTileThreads / 64];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) m[threadIdx.x >> 6] = v;
+  __syncthreads();
+  int r = m[0];
+#pragma unroll
+  for (int w = 1; w < kTileThreads / 64; ++w) r = min(r, m[w]);
+  return r;
+}
+
+// The recurrence over one tile's elements (thread t holds items 4t .. 4t + 3,
+// cnt in all) from c; writes the cdf to out unless it is null and returns c
+// after the tile.  Every round of the loop ends the tile or passes one
+// element that starts a binade.
+__device__ __forceinline__ double walk_tile(const double (&x)[kTileItems], int cnt, double c,
+                                            double *__restrict__ out) {
+  __shared__ double sc;
+  const int i0 = threadIdx.x * kTileItems;
+  int s = 0;  // elements before s are done
+  while (s < cnt) {
+    double v[kTileItems], start = 0.0;  // C (0 while c is 0) after each item
+    int f = kTile, first = kTile;
+    const int e = binade(c);
+    const Scale down(e - 52);
+    if (c == 0.0) {
+#pragma unroll
+      for (int j = kTileItems - 1; j >= 0; --j) {
+        v[j] = 0.0;
+        if (i0 + j >= s && i0 + j < cnt && x[j] > 0.0) f = i0 + j;
+      }
+      first = block_min(f);
+    } else {
+      if (!(c > 0.0 && c < __builtin_inf())) return c;  // not a probability: given up
+      const Scale up(52 - e);
+      const double C0 = up(c);
+      double d0[kTileItems], d1[kTileItems];
+      double t0 = 0.0, t1 = 0.0, a0, a1;
+      bool pairs = false;
+#pragma unroll
+      for (int j = 0; j < kTileItems; ++j) {
+        d0[j] = d1[j] = 0.0;
+        if (i0 + j >= s && i0 + j < cnt) increments(x[j], up, d0[j], d1[j]);
+        pairs |= d0[j] != d1[j];
+      }
+      if (!pairs) {
+        t0 = t1 = d0[0] + d0[1] + d0[2] + d0[3];
+      } else {
+#pragma unroll
+        for (int j = 0; j < kTileItems; ++j) then(t0, t1, d0[j], d1[j]);
+      }
+      scan_maps(t0, t1, a0, a1);
+      const bool o = odd(C0);
+      start = C0 + (o ? t1 : t0);
+      double C = start;
+#pragma unroll
+      for (int j = 0; j < kTileItems; ++j) {
+        C += pairs && odd(C) ? d1[j] : d0[j];
+        v[j] = C;
+      }
+      if (C0 + (o ? a1 : a0) >= kTop) {  // leaves the binade in this tile
+#pragma unroll
+        for (int j = kTileItems - 1; j >= 0; --j)
+          if (v[j] >= kTop) f = i0 + j;
+        first = block_min(f);
+      }
+    }
+    if (out) {
+#pragma unroll
+      for (int j = 0; j < kTileItems; ++j)
+        if (i0 + j >= s && i0 + j < cnt && i0 + j < first) out[i0 + j] = down(v[j]);
+    }
+    const bool last = first >= cnt;  // stays in the binade to the tile's end
+    if (last ? (int)threadIdx.x == (cnt - 1) / kTileItems : f == first) {
+      double l = start, px = 0.0;  // C before (after, at the end) the element
+#pragma unroll
+      for (int j = kTileItems - 1; j >= 0; --j) {
+        if (last) {
+          if (i0 + j == cnt - 1) l = v[j];
+        } else if (i0 + j == first) {
+          px = x[j];
+          if (j) l = v[j - 1];
+        }
+      }
+      sc = down(l) + px;
+      if (out && !last) out[first] = sc;
+    }
+    __syncthreads();
+    c = sc;
+    __syncthreads();
+    s = first + 1;
+  }
+  return c;
+}
+
+// Where the probabilities come from: an array, or |a|^2 of a state's amplitudes
+// in FP64 without contraction, divided by *norm2 unless that is null (the
+// values of k_probabilities and k_probabilities_div).
+struct FromArray {
+  const double *p;
+  __device__ __forceinline__ double one(uint64_t i) const { return p[i]; }
+  __device__ __forceinline__ void four(uint64_t i, double (&x)[kTileItems]) const {
+    if (((uintptr_t)p & 15) == 0) {
+      const double2 a = *reinterpret_cast<const double2 *>(p + i);
+      const double2 b = *reinterpret_cast<const double2 *>(p + i + 2);
+      x[0] = a.x;
+      x[1] = a.y;
+      x[2] = b.x;
+      x[3] = b.y;
+    } else {
+#pragma unroll
+      for (int j = 0; j < kTileItems; ++j) x[j] = p[i + j];
+    }
+  }
+};
+template <typename T>
+struct FromState {
+  const T *sv;
+  const double *norm2;
+  __device__ __forceinline__ double prob(double re, double im) const {
+#pragma clang fp contract(off)
+    const double q = re * re + im * im;
+    return norm2 ? q / *norm2 : q;
+  }
+  __device__ __forceinline__ double one(uint64_t i) const { return prob(sv[i].x, sv[i].y); }
+  __device__ __forceinline__ void four(uint64_t i, double (&x)[kTileItems]) const {
+    T a[kTileItems];
+    if (sizeof(T) == 8 && ((uintptr_t)sv & 15) == 0) {
+      const float4 *q = reinterpret_cast<const float4 *>(sv + i);
+      const float4 u = q[0], v = q[1];
+      a[0].x = u.x, a[0].y = u.y, a[1].x = u.z, a[1].y = u.w;
+      a[2].x = v.x, a[2].y = v.y, a[3].x = v.z, a[3].y = v.w;
+    } else {
+#pragma unroll
+      for (int j = 0; j < kTileItems; ++j) a[j] = sv[i + j];
+    }
+#pragma unroll
+    for (int j = 0; j < kTileItems; ++j) x[j] = prob(a[j].x, a[j].y);
+  }
+};
+
+// This thread's items of a tile and the tile's element count.
+template <typename S>
+__device__ __forceinline__ int load_tile(const S &src, uint64_t n, uint64_t tile,
+                                         double (&x)[kTileItems]) {
+  const uint64_t base = tile * kTile;
+  const int cnt = (int)(n - base < (uint64_t)kTile ? n - base : (uint64_t)kTile);
+  const int i0 = threadIdx.x * kTileItems;
+  if (cnt == kTile) {
+    src.four(base + i0, x);
+  } else {
+#pragma unroll
+    for (int j = 0; j < kTileItems; ++j) x[j] = i0 + j < cnt ? src.one(base + i0 + j) : 0.0;
+  }
+  return cnt;
+}
+
+// Sum of each tile (any order: it only bounds c); *bad is set by an element
+// that is negative or not finite.
+template <typename S>
+__global__ void __launch_bounds__(kTileThreads)
+    k_tile_sums(S src, uint64_t n, double *__restrict__ sums, int *__restrict__ bad) {
+  __shared__ double w[kTileThreads / 64];
+  double x[kTileItems];
+  load_tile(src, n, blockIdx.x, x);
+  double s = 0.0;
+  bool b = false;
+#pragma unroll
+  for (int j = 0; j < kTileItems; ++j) {
+    b |= !(x[j] >= 0.0 && x[j] < __builtin_inf());
+    s += x[j];
+  }
+  if (b) *bad = 1;
+  s = wave_sum_d(s);
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    s = 0.0;
+    for (int v = 0; v < kTileThreads / 64; ++v) s += w[v];
+    sums[blockIdx.x] = s;
+  }
+}
+
+// Each tile's map for the binades that c may be in at its start: the scanned
+// sums' error and the recurrence's own are each below (n + 16) 2^-53 of c.
+template <typename S>
+__global__ void __launch_bounds__(kTileThreads, 8)
+    k_tile_maps(S src, uint64_t n, const double *__restrict__ scanned, TileMap *__restrict__ maps) {
+  constexpr int W = kTileThreads / 64;
+  __shared__ double w[2][W];
+  __shared__ int wf[W];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double x[kTileItems];
+  load_tile(src, n, blockIdx.x, x);
+  const double a = blockIdx.x ? scanned[blockIdx.x - 1] : 0.0;
+  const double slack = (double)(n + 16) * 0x1p-51;
+  TileMap m{};
+  m.e = binade(a * (1.0 - slack));
+  if (binade(a * (1.0 + slack)) != m.e) m.flags = kHasNext;
+  // increments in both binades (the second is rarely needed), without regard
+  // to ties; f bit 0: an element is not zero, bit 1: a tie
+  const Scale up0(52 - m.e), up1(51 - m.e);
+  double t0 = 0.0, t1 = 0.0;
+  int f = 0;
+#pragma unroll
+  for (int j = 0; j < kTileItems; ++j) {
+    double d0, d1;
+    increments(x[j], up0, d0, d1);
+    f |= (x[j] != 0.0) | (d0 != d1 ? 2 : 0);
+    t0 += d0;
+    if (m.flags) {
+      increments(x[j], up1, d0, d1);
+      f |= d0 != d1 ? 2 : 0;
+      t1 += d0;
+    }
+  }
+  t0 = wave_sum_d(t0);
+  if (m.flags) t1 = wave_sum_d(t1);
+  f = (__any(f & 1) ? 1 : 0) | (__any(f & 2) ? 2 : 0);
+  if (lane == 0) {
+    w[0][wave] = t0;
+    w[1][wave] = t1;
+    wf[wave] = f;
+  }
+  __syncthreads();
+  f = 0;
+  t0 = t1 = 0.0;
+#pragma unroll
+  for (int v = 0; v < W; ++v) {
+    f |= wf[v];
+    t0 += w[0][v];
+    t1 += w[1][v];
+  }
+  m.d[0] = m.d[1] = t0;
+  m.d[2] = m.d[3] = t1;
+  if (!(f & 1)) m.flags |= kAllZero;
+  if (f & 2) m.flags |= kTies;
+  if (threadIdx.x == 0) maps[blockIdx.x] = m;
+}
+
+// The maps of the tiles that hold ties, which depend on the parity of C.
+template <typename S>
+__global__ void __launch_bounds__(kTileThreads)
+    k_tile_tie_maps(S src, uint64_t n, TileMap *__restrict__ maps) {
+  const int flags = maps[blockIdx.x].flags, e = maps[blockIdx.x].e;
+  if (!(flags & kTies)) return;
+  double x[kTileItems];
+  load_tile(src, n, blockIdx.x, x);
+  for (int k = 0; k < ((flags & kHasNext) ? 2 : 1); ++k) {
+    const Scale up(52 - e - k);
+    double d0, d1, s0 = 0.0, s1 = 0.0;
+#pragma unroll
+    for (int j = 0; j < kTileItems; ++j) {
+      increments(x[j], up, d0, d1);
+      then(s0, s1, d0, d1);
+    }
+    scan_maps(s0, s1, d0, d1);
+    if (threadIdx.x == 0) {
+      maps[blockIdx.x].d[2 * k] = d0;
+      maps[blockIdx.x].d[2 * k + 1] = d1;
+    }
+  }
+}
+
+// One workgroup: the exact c before every tile, tile_in[t], and after the
+// last, tile_in[nt]; the cdf of the tiles it goes through.
+template <typename S>
+__global__ void __launch_bounds__(kTileThreads)
+    k_tile_chain(S src, uint64_t n, uint64_t nt, const TileMap *__restrict__ maps,
+                 double *__restrict__ tile_in, double *__restrict__ cdf, int *bad) {
+  if (*bad) return;
+  __shared__ double sc;
+  const int tid = threadIdx.x;
+  double c = 0.0;
+  TileMap m{}, next{};
+  if ((uint64_t)tid < nt) next = maps[tid];
+  for (uint64_t t0 = 0; t0 < nt; t0 += kTileThreads) {
+    const uint64_t t = t0 + tid;
+    m = next;
+    if (t + kTileThreads < nt) next = maps[t + kTileThreads];
+    for (int s = 0; s < kTileThreads;) {  // tiles before t0 + s are done
+      double d0 = 0.0, d1 = 0.0;
+      const int e = binade(c);
+      const Scale up(52 - e), down(e - 52);
+      const double C0 = up(c);
+      if (t < nt && tid >= s && !(m.flags & kAllZero)) {
+        if (c > 0.0 && e == m.e) {
+          d0 = m.d[0];
+          d1 = m.d[1];
+        } else if (c > 0.0 && (m.flags & kHasNext) && e == m.e + 1) {
+          d0 = m.d[2];
+          d1 = m.d[3];
+        } else {
+          d0 = d1 = kTop;  // no map for this binade: gone through below
+        }
+      }
+      double s0 = d0, s1 = d1, a0, a1;
+      scan_maps(s0, s1, a0, a1);
+      const bool o = odd(C0);
+      const double start = C0 + (o ? s1 : s0);
+      const double all = C0 + (o ? a1 : a0);
+      if (all < kTop) {
+        if (t < nt && tid >= s) tile_in[t] = down(start);
+        c = down(all);
+        break;
+      }
+      const double end = start + (odd(start) ? d1 : d0);
+      const int f = block_min(end >= kTop ? tid : kTileThreads);
+      if (t < nt && tid >= s && tid <= f) tile_in[t] = down(start);
+      if (tid == f) sc = down(start);
+      __syncthreads();
+      c = sc;
+      double x[kTileItems];
+      const int cnt = load_tile(src, n, t0 + f, x);
+      c = walk_tile(x, cnt, c, cdf + (t0 + f) * kTile);
+      s = f + 1;
+    }
+  }
+  if (tid == 0) {
+    tile_in[nt] = c;
+    if (!(c < __builtin_inf())) *bad = 1;  // the sum overflows
+  }
+}
+
+// The tile of each uniform: the first whose end is above it (the entries
+// before a tile's end are searched by k_tile_search), marked as needed.
+__global__ void __launch_bounds__(kBlock)
+    k_tile_find(const double *__restrict__ tile_in, uint64_t nt, const double *__restrict__ u,
+                uint64_t shots, int64_t *__restrict__ out, int *__restrict__ need,
+                const int *__restrict__ bad) {
+  if (*bad) return;
+  const double total = tile_in[nt];
+  for (uint64_t s = (uint64_t)blockIdx.x * kBlock + threadIdx.x; s < shots;
+       s += (uint64_t)gridDim.x * kBlock) {
+    const double v = u[s];
+    uint64_t lo = 0, hi = nt;
+    while (lo < hi) {
+      const uint64_t mid = lo + ((hi - lo) >> 1);
+      if (tile_in[mid + 1] / total <= v) lo = mid + 1; else hi = mid;
+    }
+    out[s] = (int64_t)lo;
+    if (lo < nt) need[lo] = 1;
+  }
+}
+
+// How a needed tile gets its cdf: by one plain scan, by a scan with ties, or not
+// here (c leaves its binade there: k_tile_chain has written it).
+enum class TileCdf { kDone, kPlain, kTied };
+__device__ __forceinline__ TileCdf tile_cdf(const double *tile_in, const TileMap *maps, uint64_t t) {
+  const double c = tile_in[t];
+  if (!(c > 0.0) || binade(c) != binade(tile_in[t + 1]))
+    return c == 0.0 && tile_in[t + 1] == 0.0 ? TileCdf::kTied : TileCdf::kDone;
+  return maps[t].flags & kTies ? TileCdf::kTied : TileCdf::kPlain;
+}
+
+// The cdf of the needed tiles, written where k_tile_search looks: the plain
+// ones (few registers, so two workgroups share a CU) and the others.
+template <typename S>
+__global__ void __launch_bounds__(kTileThreads, 8)
+    k_tile_cdf(S src, uint64_t n, const double *__restrict__ tile_in,
+               const TileMap *__restrict__ maps, const int *__restrict__ need,
+               double *__restrict__ cdf, const int *__restrict__ bad) {
+  constexpr int W = kTileThreads / 64;
+  __shared__ double w[W];
+  if (*bad || !need[blockIdx.x] || tile_cdf(tile_in, maps, blockIdx.x) != TileCdf::kPlain)
+    return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double x[kTileItems];
+  const int cnt = load_tile(src, n, blockIdx.x, x);
+  const double c = tile_in[blockIdx.x];
+  const int e = binade(c);
+  const Scale up(52 - e), down(e - 52);
+  double d1;
+#pragma unroll
+  for (int j = 0; j < kTileItems; ++j) {
+    increments(x[j], up, x[j], d1);
+    if (j) x[j] += x[j - 1];
+  }
+  double i = x[kTileItems - 1];
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double p = __shfl_up(i, o);
+    if (lane >= o) i += p;
+  }
+  if (lane == 63) w[wave] = i;
+  __syncthreads();
+  double start = up(c) + (i - x[kTileItems - 1]);
+#pragma unroll
+  for (int v = 0; v < W; ++v)
+    if (v < wave) start += w[v];
+  double *out = cdf + (uint64_t)blockIdx.x * kTile + threadIdx.x * kTileItems;
+#pragma unroll
+  for (int j = 0; j < kTileItems; ++j) x[j] = down(start + x[j]);
+  if (cnt == kTile) {
+    *reinterpret_cast<double2 *>(out) = make_double2(x[0], x[1]);
+    *reinterpret_cast<double2 *>(out + 2) = make_double2(x[2], x[3]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < kTileItems; ++j)
+      if ((int)threadIdx.x * kTileItems + j < cnt) out[j] = x[j];
+  }
+}
+
+template <typename S>
+__global__ void __launch_bounds__(kTileThreads)
+    k_tile_cdf_walk(S src, uint64_t n, uint64_t nt, const double *__restrict__ tile_in,
+                    const TileMap *__restrict__ maps, const int *__restrict__ need,
+                    double *__restrict__ cdf, const int *__restrict__ bad) {
+  if (*bad) return;
+  for (uint64_t t = blockIdx.x; t < nt; t += gridDim.x) {
+    if (!need[t] || tile_cdf(tile_in, maps, t) != TileCdf::kTied) continue;
+    double x[kTileItems];
+    const int cnt = load_tile(src, n, t, x);
+    walk_tile(x, cnt, tile_in[t], cdf + t * kTile);
+  }
+}
+
+// out[s]: the uniform's tile on entry, its element on return.
+__global__ void __launch_bounds__(kBlock)
+    k_tile_search(const double *__restrict__ cdf, uint64_t n, const double *__restrict__ tile_in,
+                  uint64_t nt, const double *__restrict__ u, uint64_t shots,
+                  int64_t *__restrict__ out, const int *__restrict__ bad) {
+  if (*bad) return;
+  const double total = tile_in[nt];
+  for (uint64_t s = (uint64_t)blockIdx.x * kBlock + threadIdx.x; s < shots;
+       s += (uint64_t)gridDim.x * kBlock) {
+    const uint64_t tile = (uint64_t)out[s];
+    uint64_t lo = tile * kTile, hi = lo + kTile;
+    if (tile >= nt) lo = n;
+    if (hi > n) hi = n;
+    const double v = u[s];
+    while (lo < hi) {
+      const uint64_t mid = lo + ((hi - lo) >> 1);
+      if (cdf[mid] / total <= v) lo = mid + 1; else hi = mid;
+    }
+    out[s] = (int64_t)lo;
+  }
+}
+
+static uint64_t tile_count(uint64_t n) { return (n + kTile - 1) / kTile; }
+
+size_t sample_exact_scratch_bytes(uint64_t n) {
+  const uint64_t nt = tile_count(n);
+  return nt * (sizeof(double) + sizeof(TileMap) + sizeof(int)) + (nt + 1) * sizeof(double) +
+         scan_scratch<double>(nt) + 8 * 256;
+}
+
 // ---- host driver -----------------------------------------------------------
 size_t sample_scratch_bytes(uint64_t n, bool exact) {
   size_t b = scan_scratch<double>(n) + 4096;
@@ -270,6 +848,60 @@ size_t sample_scratch_bytes(uint64_t n, bool exact) {
 
 static inline char *align_up(char *p) {
   return (char *)(((uintptr_t)p + 255) & ~(uintptr_t)255);
+}
+
+template <typename S>
+static int sample_exact_t(const S &src, uint64_t n, double *cdf, const double *u_dev,
+                          uint64_t shots, int64_t *out_dev, void *scratch, const int **bad_dev,
+                          hipStream_t st) {
+  const uint64_t nt = tile_count(n);
+  char *w = align_up((char *)scratch);
+  int *need = (int *)w;  // nt flags, then *bad
+  w = align_up(w + (nt + 1) * sizeof(int));
+  double *sums = (double *)w;
+  w = align_up(w + nt * sizeof(double));
+  double *tile_in = (double *)w;
+  w = align_up(w + (nt + 1) * sizeof(double));
+  TileMap *maps = (TileMap *)w;
+  w = align_up(w + nt * sizeof(TileMap));
+  int *bad = need + nt;
+  SQ_HIP(hipMemsetAsync(need, 0, (nt + 1) * sizeof(int), st));
+  const dim3 g((unsigned)nt), b(kTileThreads);
+  hipLaunchKernelGGL(k_tile_sums<S>, g, b, 0, st, src, n, sums, bad);
+  SQ_HIP(hipGetLastError());
+  SQ_TRY(scan_inplace<double>(sums, nt, (double *)w, st));
+  hipLaunchKernelGGL(k_tile_maps<S>, g, b, 0, st, src, n, (const double *)sums, maps);
+  hipLaunchKernelGGL(k_tile_tie_maps<S>, g, b, 0, st, src, n, maps);
+  hipLaunchKernelGGL(k_tile_chain<S>, dim3(1), b, 0, st, src, n, nt, (const TileMap *)maps,
+                     tile_in, cdf, bad);
+  hipLaunchKernelGGL(k_tile_find, sweep_grid(shots, kBlock), dim3(kBlock), 0, st,
+                     (const double *)tile_in, nt, u_dev, shots, out_dev, need, (const int *)bad);
+  hipLaunchKernelGGL(k_tile_cdf<S>, g, b, 0, st, src, n, (const double *)tile_in,
+                     (const TileMap *)maps, (const int *)need, cdf, (const int *)bad);
+  hipLaunchKernelGGL(k_tile_cdf_walk<S>, dim3((unsigned)std::min<uint64_t>(nt, 1024)), b, 0, st,
+                     src, n, nt, (const double *)tile_in, (const TileMap *)maps,
+                     (const int *)need, cdf, (const int *)bad);
+  hipLaunchKernelGGL(k_tile_search, sweep_grid(shots, kBlock), dim3(kBlock), 0, st,
+                     (const double *)cdf, n, (const double *)tile_in, nt, u_dev, shots, out_dev,
+                     (const int *)bad);
+  SQ_HIP(hipGetLastError());
+  *bad_dev = bad;
+  return SQ_OK;
+}
+
+int sample_exact(const double *p, uint64_t n, double *cdf, const double *u_dev, uint64_t shots,
+                 int64_t *out_dev, void *scratch, const int **bad_dev, hipStream_t st) {
+  return sample_exact_t(FromArray{p}, n, cdf, u_dev, shots, out_dev, scratch, bad_dev, st);
+}
+
+int sample_exact_state(const void *sv, sq_dtype_t dt, const double *norm2_dev, uint64_t n,
+                       double *cdf, const double *u_dev, uint64_t shots, int64_t *out_dev,
+                       void *scratch, const int **bad_dev, hipStream_t st) {
+  if (dt == SQ_COMPLEX64)
+    return sample_exact_t(FromState<float2>{(const float2 *)sv, norm2_dev}, n, cdf, u_dev, shots,
+                          out_dev, scratch, bad_dev, st);
+  return sample_exact_t(FromState<double2>{(const double2 *)sv, norm2_dev}, n, cdf, u_dev, shots,
+                        out_dev, scratch, bad_dev, st);
 }
 
 int sample_cdf(const double *p, uint64_t n, double *cdf, bool exact, void *scratch,

@@ -10,17 +10,18 @@
 // in e's bits (pass_plan.cpp), so an address is a per-lane constant XOR a
 // uniform term.
 //
-// Bound: a 5-target block takes 1.3 ms of FP32 MFMA at 2^30 complex64
-// amplitudes and the sweep 2.7 ms of HBM time at copy rate, so one block hides
-// under the sweep and from the second on the matrix cores share the time.
-// Measured at 2^30 complex64, local bits of four shapes: 0 blocks 3.1-3.9 ms,
-// 1 block 3.2-4.3, 2 blocks 4.5-5.8, 3 blocks 5.9-6.6, 4 blocks 7.3-7.7, where
-// one block per launch takes 3.1 ms each.  Layered 30-qubit circuit of depth
-// 10 in 50 blocks: 155 -> 110 ms; 25-qubit mixed circuit of 175 gates unfused:
-// 12.4 -> 1.6 ms.  A loop over several chunks per workgroup with the next
-// chunk's loads issued ahead of the products (4 waves, 2 tiles each) measured
-// 5-10% slower than one chunk per workgroup: the two workgroups of a CU
-// already overlap one's loads with the other's products.
+// Bound: the sweep takes 2.7 ms of HBM time at 2^30 complex64 amplitudes at copy
+// rate; a complex64 5-target block 0.7 ms of bf16 MFMA at 2.4 GHz (1.3 ms on
+// the FP32 instructions), and the clock falls with the matrix work (2.4 GHz
+// with none, 2.0 with two blocks, 1.7 with four).  Measured there, local bits
+// 0-3, 6, 10, 12, ..., 28: no block 3.5 ms, 1 block 3.6, 2 blocks 3.9, 3 blocks
+// 4.9, 4 blocks 6.1 (FP32 instructions: 3.4, 3.6, 4.7, 5.9, 7.4), where one
+// block per launch takes 3.1 ms each.  Layered 30-qubit circuit of depth 10 in
+// 48 blocks: 148 -> 69 ms; 25-qubit mixed circuit of 175 gates unfused: 12.4 ->
+// 1.1 ms.  A loop over several chunks per workgroup with the next chunk's loads
+// issued ahead of the products (4 waves, 2 tiles each) measured 5-10% slower
+// than one chunk per workgroup: the two workgroups of a CU already overlap
+// one's loads with the other's products.
 #include <algorithm>
 
 #include "kernels.hpp"
@@ -64,64 +65,120 @@ __device__ __forceinline__ uint32_t xor_lane(const uint16_t *w, uint32_t v) {
   return r;
 }
 
-// One 5-target block on this wave's tile (complex64): three real products per
-// complex one, operands as in k_mfma5_c64.
-__device__ __forceinline__ void pass_block5(char *X, const float4 *As, const PassBlock &b, int lane,
-                                            uint32_t lb) {
-  const int col = lane & 31, half = lane >> 5;
-  const uint32_t rd = lb ^ (half ? b.row[0] : 0u), wr = lb ^ (half ? b.row[2] : 0u);
-  float2 x[16];
+// complex64 products run on the bf16 matrix instructions (16 times the FP32
+// rate) with every FP32 operand split in three bf16 parts, x = x0 + x1 + x2 to
+// 2^-27 of x: the six products of parts i + j <= 2 are summed in FP32, and the
+// dropped ones are below 2^-26 of |g x|, under the rounding of an FP32 product.
+// The matrix parts come from its FP64 entries (pass_image).  Error of a layered
+// circuit against 64 bits (2-norm): 14 qubits 6.3e-7 -> 3.6e-7, 23 qubits 7.4e-7
+// -> 4.3e-7, 30 qubits 7.9e-7 -> 4.7e-7 against the FP32 instructions with three
+// real products per complex one.
+typedef __bf16 pbf2 __attribute__((ext_vector_type(2)));
+typedef __bf16 pbf8 __attribute__((ext_vector_type(8)));
+typedef float pf2 __attribute__((ext_vector_type(2)));
+
+// Parts of eight operands of this lane.
+struct Split8 {
+  pbf8 p[3];
+};
+__device__ __forceinline__ void split2(Split8 &s, int i, float a, float b) {
+  pf2 x = {a, b};
 #pragma unroll
-  for (int s = 0; s < 16; ++s)
-    x[s] = *reinterpret_cast<const float2 *>(X + (rd ^ xor_bits<4>(b.row + 1, s)));
+  for (int k = 0; k < 3; ++k) {
+    const pbf2 h = __builtin_convertvector(x, pbf2);
+    s.p[k][2 * i] = h[0];
+    s.p[k][2 * i + 1] = h[1];
+    if (k < 2) {
+      const pf2 f = __builtin_convertvector(h, pf2);
+      x[0] -= f[0];
+      x[1] -= f[1];
+    }
+  }
+}
+// One 5-target block on this wave's tile (complex64): T1 = Gr Xr, T2 = Gi Xi,
+// T3 = Gi Xr + Gr Xi.  Fragment (m, part, t) of the matrix image (m = 0: Gr,
+// 1: Gi) holds lane l's G[l%32][16t + 8(l/32) + j], j = 0..7; the state operand
+// of lane l is amplitude 16t + 8(l/32) + j of group l%32.
+__device__ __forceinline__ void pass_block5(char *X, const pbf8 *As, const PassBlock &b, int lane,
+                                            uint32_t lb) {
+  const int half = lane >> 5;
+  const uint32_t rd = lb ^ (half ? b.row[3] : 0u), wr = lb ^ (half ? b.row[2] : 0u);
   pfloatx16 t1, t2, t3;
 #pragma unroll
   for (int v = 0; v < 16; ++v) t1[v] = t2[v] = t3[v] = 0.f;
+  float2 u[2][8];
 #pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    const float4 a = As[(2 * s + half) * 32 + col];
-    t1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, x[s].x, t1, 0, 0, 0);
-    t2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, x[s].y, t2, 0, 0, 0);
-    t3 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, x[s].x + x[s].y, t3, 0, 0, 0);
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      u[t][j] = *reinterpret_cast<const float2 *>(
+          X + (rd ^ (t ? b.row[4] : 0u) ^ xor_bits<3>(b.row, j)));
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    Split8 xr, xi;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      split2(xr, i, u[t][2 * i].x, u[t][2 * i + 1].x);
+      split2(xi, i, u[t][2 * i].y, u[t][2 * i + 1].y);
+    }
+    // part p of the matrix against parts 2 - p, ..., 0 of the state
+#pragma unroll
+    for (int p = 2; p >= 0; --p) {
+      const pbf8 gr = As[(2 * p + t) * 64 + lane], gi = As[(2 * (3 + p) + t) * 64 + lane];
+#pragma unroll
+      for (int x = 2 - p; x >= 0; --x) {
+        t1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gr, xr.p[x], t1, 0, 0, 0);
+        t3 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gi, xr.p[x], t3, 0, 0, 0);
+        t2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gi, xi.p[x], t2, 0, 0, 0);
+        t3 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gr, xi.p[x], t3, 0, 0, 0);
+      }
+    }
   }
   // C layout: lane l, register v -> group l%32, amplitude 8(v/4) + 4(l/32) + v%4
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
     const uint32_t o = xor_bits<2>(b.row, v & 3) ^ xor_bits<2>(b.row + 3, v >> 2);
-    *reinterpret_cast<float2 *>(X + (wr ^ o)) = make_float2(t1[v] - t2[v], t3[v] - t1[v] - t2[v]);
+    *reinterpret_cast<float2 *>(X + (wr ^ o)) = make_float2(t1[v] - t2[v], t3[v]);
   }
 }
 
-// A-operand registers of a 4-target block's real 32x32 form.
-__device__ __forceinline__ void pass_a4(float (&a)[16], const float *As, int lane) {
-#pragma unroll
-  for (int s = 0; s < 16; ++s) a[s] = As[(2 * s + (lane >> 5)) * 32 + (lane & 31)];
-}
-__device__ __forceinline__ void pass_a4(double (&a)[16], const double *As, int lane) {
-#pragma unroll
-  for (int s = 0; s < 16; ++s) a[s] = As[(4 * (s >> 1) + (lane >> 4)) * 32 + 16 * (s & 1) + (lane & 15)];
-}
-
-// One 4-target block on two tiles (complex64): the real 32x32 form, operands
-// as in k_mfma4_c64.
-__device__ __forceinline__ void pass_block4(char *X, const float (&a)[16], const PassBlock &b,
-                                            int lane, uint32_t lb, uint32_t tile2) {
+// One 4-target block on two tiles (complex64) in its real 32x32 form (row
+// 2r + c, column 2o + c').  Fragment (part, t) holds lane l's entries of row
+// l%32, columns 16t + 8(l/32) + j; the state operand is component j%2 of
+// amplitude 8t + 4(l/32) + j/2.
+__device__ __forceinline__ void pass_block4(char *X, const pbf8 *As, const PassBlock &b, int lane,
+                                            uint32_t lb, uint32_t tile2) {
   const int half = lane >> 5;
-  float x0[16], x1[16];
-  const uint32_t rd = lb | (half ? 4u : 0u);
-#pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    const uint32_t o = xor_bits<4>(b.row, s);
-    x0[s] = *reinterpret_cast<const float *>(X + (rd ^ o));
-    x1[s] = *reinterpret_cast<const float *>(X + (rd ^ o ^ tile2));
-  }
+  const uint32_t rd = lb ^ (half ? b.row[2] : 0u);
   pfloatx16 t0, t1;
 #pragma unroll
   for (int v = 0; v < 16; ++v) t0[v] = t1[v] = 0.f;
+  float2 u[2][4], v[2][4];
 #pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    t0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], x0[s], t0, 0, 0, 0);
-    t1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], x1[s], t1, 0, 0, 0);
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t o = rd ^ (t ? b.row[3] : 0u) ^ xor_bits<2>(b.row, i);
+      u[t][i] = *reinterpret_cast<const float2 *>(X + o);
+      v[t][i] = *reinterpret_cast<const float2 *>(X + (o ^ tile2));
+    }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    Split8 x0, x1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      split2(x0, i, u[t][i].x, u[t][i].y);
+      split2(x1, i, v[t][i].x, v[t][i].y);
+    }
+#pragma unroll
+    for (int p = 2; p >= 0; --p) {
+      const pbf8 g = As[(2 * p + t) * 64 + lane];
+#pragma unroll
+      for (int x = 2 - p; x >= 0; --x) {
+        t0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(g, x0.p[x], t0, 0, 0, 0);
+        t1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(g, x1.p[x], t1, 0, 0, 0);
+      }
+    }
   }
   // C layout: lane l, register 4q + i -> component i%2 of amplitude 4q + 2(l/32) + i/2
   const uint32_t wr = lb ^ (half ? b.row[1] : 0u);
@@ -173,9 +230,12 @@ __device__ __forceinline__ void pass_block5(char *X, const double2 *As, const Pa
     }
 }
 
-__device__ __forceinline__ void pass_block4(char *X, const double (&a)[16], const PassBlock &b,
-                                            int lane, uint32_t lb, uint32_t tile2) {
+__device__ __forceinline__ void pass_block4(char *X, const double *As, const PassBlock &b, int lane,
+                                            uint32_t lb, uint32_t tile2) {
   const int q = lane >> 4;
+  double a[16];
+#pragma unroll
+  for (int s = 0; s < 16; ++s) a[s] = As[(4 * (s >> 1) + q) * 32 + 16 * (s & 1) + (lane & 15)];
   const uint32_t rd = (lb ^ ((q >> 1) ? b.row[0] : 0u)) | ((q & 1) ? 8u : 0u);
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -227,7 +287,7 @@ struct PassShape {
 };
 
 template <typename R, int CB>
-__global__ void __launch_bounds__((PassShape<R, CB>::NT), (PassShape<R, CB>::NW == 8 ? 4 : 2))
+__global__ void __launch_bounds__((PassShape<R, CB>::NT), (PassShape<R, CB>::NW == 8 ? 4 : PassShape<R, CB>::NW == 4 ? 3 : 2))
     k_pass(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t nchunks, PassGeom geom,
            const PassBlock *__restrict__ blocks, int nblocks, const char *__restrict__ image,
            uint64_t gstride) {
@@ -240,9 +300,9 @@ __global__ void __launch_bounds__((PassShape<R, CB>::NT), (PassShape<R, CB>::NW 
   constexpr int E0 = c64 ? 1 : 0;                     // chunk bit of thread bit 0 (16 B per access)
   constexpr int EK = E0 + TB;                         // chunk bit of access index bit 0
   constexpr int ITEM = c64 ? 8 : 16;
-  constexpr int NP = 1024 / NT;                       // 16-byte units of a block matrix per thread
+  constexpr int NP = (c64 ? 768 + NT - 1 : 1024) / NT;  // 16-byte units of a block matrix per thread
   __shared__ T Xs[1 << CB];
-  __shared__ float4 As[1024];
+  __shared__ float4 As[c64 ? 768 : 1024];
   char *X = reinterpret_cast<char *>(Xs);
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -311,18 +371,17 @@ __global__ void __launch_bounds__((PassShape<R, CB>::NT), (PassShape<R, CB>::NW 
       const PassBlock b = load_block(blocks + j);
 #pragma unroll
       for (int i = 0; i < NP; ++i)
-        if (i * NT < b.n16) reinterpret_cast<nt_f4 *>(As)[t + i * NT] = pre[i];
+        if (t + i * NT < b.n16) reinterpret_cast<nt_f4 *>(As)[t + i * NT] = pre[i];
       __syncthreads();
       if (j + 1 < nblocks) fetch(pre, blocks + j + 1);  // arrives during this block's products
       uint32_t lb = xor_lane<c64 ? 5 : 4>(b.col, lane);
       lb ^= xor_lane<WB>(b.wave, wave);
       if (b.k == 5) {
-        if constexpr (c64) pass_block5(X, As, b, lane, lb);
+        if constexpr (c64) pass_block5(X, reinterpret_cast<const pbf8 *>(As), b, lane, lb);
         else pass_block5(X, reinterpret_cast<const double2 *>(As), b, lane, lb);
       } else {
-        R a[16];
-        pass_a4(a, reinterpret_cast<const R *>(As), lane);
-        pass_block4(X, a, b, lane, lb, b.wave[WB]);
+        if constexpr (c64) pass_block4(X, reinterpret_cast<const pbf8 *>(As), b, lane, lb, b.wave[WB]);
+        else pass_block4(X, reinterpret_cast<const double *>(As), b, lane, lb, b.wave[WB]);
       }
       __syncthreads();
     }

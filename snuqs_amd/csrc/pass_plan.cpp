@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <cstring>
 
 namespace sq {
@@ -249,7 +250,7 @@ std::vector<PassBlock> pass_blocks(const PassPlan &p, sq_dtype_t dt, size_t *ima
       if (nc < ncol) d.col[nc++] = w; else d.wave[nw++] = w;
     }
     d.k = (uint16_t)b.k;
-    const size_t bytes = b.k == 5 ? 16384 : (c64 ? 4096 : 8192);
+    const size_t bytes = b.k == 5 ? (c64 ? 12288 : 16384) : (c64 ? 6144 : 8192);
     d.n16 = (uint16_t)(bytes / 16);
     d.goff = (uint32_t)(off / 16);
     off += bytes;
@@ -338,6 +339,26 @@ static void block_matrix(const PassBlockPlan &b, const PassGates &pg, BlockMatri
   }
 }
 
+// bf16 nearest to v, ties to even.  v is first cut to a float towards zero with a
+// sticky last bit, so that the second rounding sees which side of a tie v is on.
+static uint16_t to_bf16(double v) {
+  float f = (float)v;
+  uint32_t u;
+  std::memcpy(&u, &f, 4);
+  if ((double)f != v && f == f) {
+    if (std::fabs((double)f) > std::fabs(v)) --u;  // towards zero
+    u |= 1;
+  }
+  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);  // NaN
+  return (uint16_t)((u + 0x7fff + ((u >> 16) & 1)) >> 16);
+}
+static double from_bf16(uint16_t h) {
+  const uint32_t u = (uint32_t)h << 16;
+  float f;
+  std::memcpy(&f, &u, 4);
+  return f;
+}
+
 void pass_image(const PassPlan &p, const std::vector<PassBlock> &blocks, sq_dtype_t dt,
                 const PassGates &pg, char *img) {
   const bool c64 = dt == SQ_COMPLEX64;
@@ -347,38 +368,40 @@ void pass_image(const PassPlan &p, const std::vector<PassBlock> &blocks, sq_dtyp
     block_matrix(b, pg, &M);
     const int d = 1 << b.k;
     char *dst = img + (size_t)blocks[i].goff * 16;
-    if (b.k == 5) {
-      // entry (o, r): {Re, Im, Re + Im, 0} (complex64), {Re, Im} (complex128)
-      for (int o = 0; o < d; ++o)
-        for (int r = 0; r < d; ++r) {
-          const double re = M.re[r * d + o], im = M.im[r * d + o];
-          if (c64) {
-            float *e = (float *)dst + 4 * (o * d + r);
-            e[0] = (float)re;
-            e[1] = (float)im;
-            e[2] = (float)(re + im);
-            e[3] = 0.f;
-          } else {
-            double *e = (double *)dst + 2 * (o * d + r);
-            e[0] = re;
-            e[1] = im;
-          }
-        }
+    if (c64) {
+      // bf16 fragments (kernels_pass.hip): 5 targets the real and imaginary
+      // matrices, 4 targets the real 32x32 form, each in three parts of two
+      // fragments of 64 lanes x 8 columns
+      uint16_t *f = (uint16_t *)dst;
+      for (int m = 0; m < (b.k == 5 ? 2 : 1); ++m)
+        for (int t = 0; t < 2; ++t)
+          for (int lane = 0; lane < 64; ++lane)
+            for (int j = 0; j < 8; ++j) {
+              const int row = lane & 31, c = 16 * t + 8 * (lane >> 5) + j;
+              double v;
+              if (b.k == 5) {
+                v = (m ? M.im : M.re)[row * d + c];
+              } else {
+                const int e = (row >> 1) * d + (c >> 1);
+                v = (row & 1) == (c & 1) ? M.re[e] : (row & 1) ? M.im[e] : -M.im[e];
+              }
+              for (int part = 0; part < 3; ++part) {
+                const uint16_t h = to_bf16(v);
+                f[(((3 * m + part) * 2 + t) * 64 + lane) * 8 + j] = h;
+                v -= from_bf16(h);
+              }
+            }
       continue;
     }
-    // real form: row 2r + c, column 2o + c', column-major
+    double *f = (double *)dst;
     for (int o = 0; o < d; ++o)
       for (int r = 0; r < d; ++r) {
         const double re = M.re[r * d + o], im = M.im[r * d + o];
-        const int e0 = 2 * o * 32 + 2 * r, e1 = e0 + 32;
-        if (c64) {
-          float *f = (float *)dst;
-          f[e0] = (float)re;
-          f[e0 + 1] = (float)im;
-          f[e1] = (float)-im;
-          f[e1 + 1] = (float)re;
-        } else {
-          double *f = (double *)dst;
+        if (b.k == 5) {  // entry (o, r): {Re, Im}
+          f[2 * (o * d + r)] = re;
+          f[2 * (o * d + r) + 1] = im;
+        } else {  // real form: row 2r + c, column 2o + c', column-major
+          const int e0 = 2 * o * 32 + 2 * r, e1 = e0 + 32;
           f[e0] = re;
           f[e0 + 1] = im;
           f[e1] = -im;

@@ -411,11 +411,10 @@ int sq_qaoa_destroy(void *batch);
  * bit of a matrix's local index; 2^k x 2^k complex128 row-major).  Every
  * gate runs as a dense matrix on its targets.  The batch owns the states
  * (one device buffer).  sq_cbatch_run sets every state to |0...0> and
- * applies every circuit: step s applies gate s of every circuit that has
- * one, in one launch for the gates that run on the 5-target matrix-core
- * kernels and one for the others (at most 2 max(num_gates) + 2 launches,
- * captured into a hipGraph on the first use_graph call and replayed after).
- * Asynchronous on `stream`.
+ * applies every circuit: step s applies pass s (several gates, as in
+ * sq_program_run) of every circuit that has one, or gate s of the circuits too
+ * small for a pass (captured into a hipGraph on the first use_graph call and
+ * replayed after).  Asynchronous on `stream`.
  * Errors (SQ_ERR_INVALID): no circuits, a qubit count outside 1..30, a gate
  * with 0 or more than 5 targets or more targets than qubits, repeated or
  * out-of-range targets. */
@@ -428,7 +427,9 @@ int sq_cbatch_run(void *batch, int use_graph, void *stream);
  * 2^num_qubits[j] elements of the batch's dtype), ordered on `stream`. */
 int sq_cbatch_copy_state(void *batch, uint32_t circuit, void *dst,
                          uint64_t num_elems, void *stream);
-/* Kernel launches per run, bytes of all states, HBM bytes one run moves. */
+/* Launches per run and HBM bytes when each step is one gate of every circuit
+ * (upper bounds of what sq_cbatch_run takes with passes), bytes of all
+ * states. */
 int sq_cbatch_stats(void *batch, uint64_t *launches, double *state_bytes,
                     double *traffic_bytes);
 int sq_cbatch_destroy(void *batch);

@@ -317,7 +317,7 @@ static void plan_pass_set(int nq, sq_dtype_t dt, uint32_t nsets, const std::vect
   for (size_t g = 0; g < nt.size(); ++g)
     for (int t = 0; t < nt[g]; ++t) masks[g] |= 1ull << (nq - 1 - (int)targets[toff[g] + t]);
   *ps = PassSet{};
-  plan_passes(nq, dt, masks, touched, &ps->steps, &ps->plans);
+  plan_passes(nq, pass_chunk_bits(dt, nq), dt, masks, touched.data(), &ps->steps, &ps->plans);
   for (const PassPlan &p : ps->plans) {
     size_t bytes;
     ps->geoms.push_back(pass_geom(p));

@@ -5,28 +5,31 @@
 // has no batching; transpile.py:233-234 is where it would go).  Circuit j has
 // n_j qubits and its own list of gates (dense matrices on 1-5 targets, e.g.
 // the blocks of a fused circuit); its state lives at its own offset in one
-// device buffer.  Launch s applies gate s of every circuit that has one: a
-// table gives each gate its state, its workgroup range, its matrix and its
-// index map, and a workgroup looks up its gate (uniform) and sweeps its
-// share of the gate's groups.  So many small circuits, each of which alone
-// would leave most of the GPU idle, fill it together, and a batch of C
-// circuits of up to G gates takes at most 2G + 2 launches (captured in one
-// hipGraph) instead of the sum of the gate counts.
+// device buffer.
 //
-// Gates that run on the 5-target MFMA kernels in a one-circuit program (5
-// targets, or 4 widened to 5 on states of 15 qubits or more, with full
-// tiles) take the same kernels here through an entry table (one launch per
-// step for them); the others take k_cbatch_dense.  There a group is the 2^k
-// amplitudes a k-target gate mixes: one lane per group per grid pass,
-// consecutive lanes on consecutive groups (coalesced runs along the lowest
-// free bits); the matrix is staged in LDS, so every lane of a wave reads the
-// same entry (a broadcast).  Arithmetic in the state's precision.
+// Circuits large enough for a pass (kernels_pass.hip) are planned into passes
+// of several gates; launch s applies pass s of every such circuit, one
+// workgroup a chunk, a table giving each workgroup its circuit.  A circuit's
+// first pass starts from |0...0> without reading it.  Smaller circuits take
+// gate s of each in one launch of k_cbatch_dense.  So many small circuits,
+// each of which alone would leave most of the GPU idle, fill it together, and
+// a batch takes as many launches as its longest circuit has steps (captured in
+// one hipGraph).  48 circuits of 12-22 qubits, depth 10, complex64: 4.2 ms a
+// run with one gate a step, 1.7 ms with passes.
+//
+// k_cbatch_dense: a group is the 2^k amplitudes a k-target gate mixes; one lane
+// per group per grid pass, consecutive lanes on consecutive groups (coalesced
+// runs along the lowest free bits); the matrix is staged in LDS, so every lane
+// of a wave reads the same entry (a broadcast).  Arithmetic in the state's
+// precision.
 #include <algorithm>
+#include <cstring>
 #include <memory>
 #include <vector>
 
 #include "kernels.hpp"
 #include "kernels_cbatch.hpp"
+#include "pass_plan.hpp"
 
 namespace sq {
 
@@ -188,18 +191,20 @@ struct CBatch {
   std::vector<uint64_t> host_psi;
   uint64_t nelems = 0;
   void *states = nullptr;
-  void *mats = nullptr;
-  void *g3m = nullptr;      // matrices of the MFMA entries (4 reals per element)
+  void *mats = nullptr;       // matrices of k_cbatch_dense
   CBGate *tables = nullptr;
-  void *mtables = nullptr;  // MFMA entries (cbatch_mfma_entry)
+  void *pass = nullptr;       // entries, workgroup map, descriptors and matrices of the passes
+  size_t pass_map = 0, pass_desc = 0, pass_img = 0;  // byte offsets in `pass`
   uint64_t *psi = nullptr;
   struct Launch {
-    int mfma;  // 0: k_cbatch_dense over `tables`, 1: the MFMA kernels over `mtables`
-    size_t tab_off;
-    int count;
+    int cb;          // 0: k_cbatch_dense, otherwise a pass launch's chunk bits
+    size_t tab_off;  // first entry of `tables`, or first workgroup of the map
+    int count;       // entries (k_cbatch_dense)
     uint64_t blocks;
   };
   std::vector<Launch> launches;
+  bool zero_first = false;     // some circuit starts from a state in memory
+  uint64_t gate_launches = 0;  // launches when every step is one gate per circuit
   hipGraphExec_t exec = nullptr;
   hipGraph_t graph = nullptr;
   double state_bytes = 0, traffic_bytes = 0;
@@ -208,7 +213,7 @@ struct CBatch {
 static void free_cbatch(CBatch *b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
-  for (void *p : {b->states, b->mats, b->g3m, (void *)b->tables, b->mtables, (void *)b->psi})
+  for (void *p : {b->states, b->mats, (void *)b->tables, b->pass, (void *)b->psi})
     if (p) (void)hipFree(p);
 }
 
@@ -220,11 +225,12 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
   B->dt = dt;
   B->ncirc = ncirc;
   const size_t item = itemsize(dt);
-  // plans of every gate, circuit by circuit: as a program plans it with
-  // kPlanDense (a dense matrix on all its targets, 4-target blocks of large
-  // states widened to 5 for the MFMA kernels), and on exactly its own targets
-  // (kPlanExact) for k_cbatch_dense
-  std::vector<std::vector<GatePlan>> plans(ncirc), wplans(ncirc);
+  const bool c64 = dt == SQ_COMPLEX64;
+  // every gate as a dense matrix on exactly its targets
+  std::vector<std::vector<GatePlan>> plans(ncirc);
+  std::vector<std::vector<int>> cnt(ncirc);
+  std::vector<std::vector<size_t>> toff(ncirc), moff(ncirc);
+  std::vector<uint32_t> tg;
   size_t gi = 0, ti = 0, mi = 0;
   uint32_t maxg = 0;
   uint64_t amp = 0;
@@ -232,18 +238,18 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
     if (nq[j] < 1 || nq[j] > 30)
       return fail(SQ_ERR_INVALID, "circuit batch: qubit counts must be in [1, 30]");
     plans[j].resize(ng[j]);
-    wplans[j].resize(ng[j]);
     for (uint32_t g = 0; g < ng[j]; ++g, ++gi) {
       const int k = (int)nt[gi];
       if (k < 1 || k > kMaxK || k > (int)nq[j])
         return fail(SQ_ERR_INVALID, "circuit batch: circuit " + std::to_string(j) + ", gate " +
                                         std::to_string(g) + ": 1 to 5 targets, at most the qubit count");
-      SQ_TRY(make_plan(matrices + mi, targets + ti, k, (int)nq[j], (int)nq[j], &wplans[j][g],
-                       kPlanDense));
       SQ_TRY(make_plan(matrices + mi, targets + ti, k, (int)nq[j], (int)nq[j], &plans[j][g],
                        kPlanDense | kPlanExact));
       if (plans[j][g].kind != Kind::DENSE || plans[j][g].kk != k)
         return fail(SQ_ERR_INVALID, "circuit batch: internal: gate not planned dense");
+      cnt[j].push_back(k);
+      toff[j].push_back(ti);
+      moff[j].push_back(mi);
       ti += (size_t)k;
       mi += 2ull << (2 * k);
     }
@@ -253,33 +259,52 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
     amp += 1ull << nq[j];
     B->state_bytes += std::ldexp(1.0, (int)nq[j]) * (double)item;
   }
+  tg.assign(targets, targets + ti);
   B->nelems = amp;
-  // matrices in the state's precision, tables per launch
-  std::vector<double> hm;  // interleaved re/im, converted below
-  std::vector<double> g3;  // MFMA entries' matrices
-  std::vector<CBGate> tabs;
-  std::vector<uint8_t> mtabs;
-  const size_t mbytes = cbatch_mfma_entry_bytes();
-  const bool c64 = dt == SQ_COMPLEX64;
+  // Steps of the circuits that run in passes.  Chunks are chosen by the batch's
+  // amplitudes: together the circuits fill the chip as one state of that size
+  // would.
+  const int nbits = log2u(amp);
+  std::vector<std::vector<PassPlan>> passes(ncirc);
+  size_t steps = 0;
+  for (uint32_t j = 0; j < ncirc; ++j) {
+    const int cb = std::min<int>(pass_chunk_bits(dt, nbits), (int)nq[j]);
+    if (cb < pass_min_bits(dt) || ng[j] == 0) {
+      B->zero_first = true;
+      steps = std::max<size_t>(steps, ng[j]);
+      continue;
+    }
+    std::vector<uint64_t> masks(ng[j], 0);
+    for (uint32_t g = 0; g < ng[j]; ++g)
+      for (int b = 0; b < plans[j][g].kk; ++b) masks[g] |= 1ull << plans[j][g].tbit[b];
+    std::vector<Step> st;
+    plan_passes((int)nq[j], cb, dt, masks, nullptr, &st, &passes[j]);
+    steps = std::max(steps, passes[j].size());
+  }
+  // the gate-by-gate step count (stats): 5-target blocks (4 targets from 15
+  // qubits on) in one launch, the others in another
   for (uint32_t s = 0; s < maxg; ++s) {
-    CBatch::Launch L{0, tabs.size(), 0, 0};
-    CBatch::Launch M{1, mtabs.size() / mbytes, 0, 0};
-    uint64_t mtiles = 0;  // tiles of the step's MFMA entries (sets their grid)
-    for (uint32_t j = 0; j < ncirc; ++j)
-      if (s < ng[j]) mtiles += cbatch_mfma_tiles(wplans[j][s], c64, 1ull << nq[j]);
-    const uint64_t tpw = mfma_wave_tiles(mtiles);
+    bool big = false, small = false;
     for (uint32_t j = 0; j < ncirc; ++j) {
       if (s >= ng[j]) continue;
       B->traffic_bytes += 2.0 * std::ldexp(1.0, (int)nq[j]) * (double)item;
-      std::vector<uint8_t> ent(mbytes);
-      uint64_t nb = 0;
-      if (cbatch_mfma_entry(wplans[j][s], c64, 1ull << nq[j], B->host_psi[j], M.blocks, tpw, &g3,
-                            ent.data(), &nb)) {
-        mtabs.insert(mtabs.end(), ent.begin(), ent.end());
-        M.blocks += nb;
-        M.count++;
-        continue;
-      }
+      const int k = plans[j][s].kk;
+      const bool five = k == 5 ? (int)nq[j] >= pass_min_bits(dt) : k == 4 && nq[j] >= 15;
+      (five ? big : small) = true;
+    }
+    B->gate_launches += (uint64_t)big + (uint64_t)small;
+  }
+  // matrices in the state's precision, tables per launch
+  std::vector<double> hm;  // interleaved re/im, converted below
+  std::vector<CBGate> tabs;
+  std::vector<PassEntry> entries;
+  std::vector<uint32_t> wgs;
+  std::vector<PassBlock> descs;
+  std::vector<char> images;
+  for (size_t s = 0; s < steps; ++s) {
+    CBatch::Launch L{0, tabs.size(), 0, 0};
+    for (uint32_t j = 0; j < ncirc; ++j) {
+      if (!passes[j].empty() || s >= ng[j]) continue;
       const GatePlan &p = plans[j][s];
       CBGate e{};
       e.psi = B->host_psi[j];
@@ -302,12 +327,51 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
       L.count++;
       tabs.push_back(e);
     }
-    if (L.blocks > (uint64_t)INT32_MAX || M.blocks > (uint64_t)INT32_MAX)
+    if (L.blocks > (uint64_t)INT32_MAX)
       return fail(SQ_ERR_INVALID, "circuit batch: too many circuits for one launch per step");
     if (L.count) B->launches.push_back(L);
-    if (M.count) B->launches.push_back(M);
+    for (int cb = pass_min_bits(dt); cb <= kPassMaxBits; ++cb) {
+      CBatch::Launch P{cb, wgs.size(), 0, 0};
+      for (uint32_t j = 0; j < ncirc; ++j) {
+        if (s >= passes[j].size() || passes[j][s].cb != cb) continue;
+        const PassPlan &p = passes[j][s];
+        PassEntry e{};
+        size_t bytes;
+        const std::vector<PassBlock> pb = pass_blocks(p, dt, &bytes);
+        e.psi = B->host_psi[j];
+        e.first = P.blocks;
+        e.blocks = descs.size();
+        e.image = images.size();
+        e.nblocks = (int)pb.size();
+        e.initial = s == 0;
+        e.geom = pass_geom(p);
+        images.resize(images.size() + bytes);
+        pass_image(p, pb, dt,
+                   PassGates{matrices, &moff[j], &toff[j], &tg, &cnt[j], (int)nq[j]},
+                   images.data() + e.image);
+        descs.insert(descs.end(), pb.begin(), pb.end());
+        const uint64_t chunks = 1ull << (nq[j] - cb);
+        wgs.insert(wgs.end(), chunks, (uint32_t)entries.size());
+        P.blocks += chunks;
+        entries.push_back(e);
+      }
+      if (P.blocks > (1ull << 22))
+        return fail(SQ_ERR_INVALID, "circuit batch: too many circuits for one launch per step");
+      if (P.blocks) B->launches.push_back(P);
+    }
   }
   B->traffic_bytes += (double)amp * (double)item;  // the initial state
+  std::vector<char> pimg;
+  auto put = [&](const void *src, size_t bytes) {
+    const size_t off = (pimg.size() + 255) / 256 * 256;
+    pimg.resize(off + bytes);
+    if (bytes) std::memcpy(pimg.data() + off, src, bytes);
+    return off;
+  };
+  put(entries.data(), entries.size() * sizeof(PassEntry));
+  B->pass_map = put(wgs.data(), wgs.size() * sizeof(uint32_t));
+  B->pass_desc = put(descs.data(), descs.size() * sizeof(PassBlock));
+  B->pass_img = put(images.data(), images.size());
   auto dmalloc = [](void **ptr, size_t bytes) -> int {
     if (hipMalloc(ptr, std::max<size_t>(bytes, 16)) != hipSuccess) {
       (void)hipGetLastError();
@@ -320,9 +384,8 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
   const size_t nm = hm.size() / 2;
   int rc = dmalloc(&B->states, amp * item);
   if (!rc) rc = dmalloc(&B->mats, nm * item);
-  if (!rc) rc = dmalloc(&B->g3m, g3.size() * (c64 ? sizeof(float) : sizeof(double)));
   if (!rc) rc = dmalloc((void **)&B->tables, tabs.size() * sizeof(CBGate));
-  if (!rc) rc = dmalloc(&B->mtables, mtabs.size());
+  if (!rc) rc = dmalloc(&B->pass, pimg.size());
   if (!rc) rc = dmalloc((void **)&B->psi, ncirc * sizeof(uint64_t));
   if (rc) {
     free_cbatch(B.get());
@@ -337,18 +400,10 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
     ok = hipMemcpy(B->mats, hm.data(), hm.size() * sizeof(double), hipMemcpyHostToDevice) ==
          hipSuccess;
   }
-  if (c64) {
-    std::vector<float> gf(g3.begin(), g3.end());
-    ok = ok && (gf.empty() || hipMemcpy(B->g3m, gf.data(), gf.size() * sizeof(float),
-                                        hipMemcpyHostToDevice) == hipSuccess);
-  } else {
-    ok = ok && (g3.empty() || hipMemcpy(B->g3m, g3.data(), g3.size() * sizeof(double),
-                                        hipMemcpyHostToDevice) == hipSuccess);
-  }
   ok = ok && (tabs.empty() || hipMemcpy(B->tables, tabs.data(), tabs.size() * sizeof(CBGate),
                                         hipMemcpyHostToDevice) == hipSuccess);
-  ok = ok && (mtabs.empty() || hipMemcpy(B->mtables, mtabs.data(), mtabs.size(),
-                                         hipMemcpyHostToDevice) == hipSuccess);
+  ok = ok && (pimg.empty() || hipMemcpy(B->pass, pimg.data(), pimg.size(),
+                                        hipMemcpyHostToDevice) == hipSuccess);
   ok = ok && hipMemcpy(B->psi, B->host_psi.data(), ncirc * sizeof(uint64_t),
                        hipMemcpyHostToDevice) == hipSuccess;
   if (!ok) {
@@ -363,16 +418,19 @@ template <typename R>
 static int cb_enqueue_t(CBatch *B, hipStream_t st) {
   using T = typename CV<R>::T;
   T *s = (T *)B->states;
-  const uint64_t zb = std::min<uint64_t>((B->nelems + kBlock - 1) / kBlock, 1ull << 16);
-  hipLaunchKernelGGL(k_cbatch_zero<R>, dim3((unsigned)zb), dim3(kBlock), 0, st, s, B->nelems);
-  hipLaunchKernelGGL(k_cbatch_basis<R>, dim3((B->ncirc + kBlock - 1) / kBlock), dim3(kBlock), 0,
-                     st, s, B->psi, B->ncirc);
-  const size_t mbytes = cbatch_mfma_entry_bytes();
+  if (B->zero_first) {  // (a circuit's passes start from |0...0> by themselves)
+    const uint64_t zb = std::min<uint64_t>((B->nelems + kBlock - 1) / kBlock, 1ull << 16);
+    hipLaunchKernelGGL(k_cbatch_zero<R>, dim3((unsigned)zb), dim3(kBlock), 0, st, s, B->nelems);
+    hipLaunchKernelGGL(k_cbatch_basis<R>, dim3((B->ncirc + kBlock - 1) / kBlock), dim3(kBlock), 0,
+                       st, s, B->psi, B->ncirc);
+  }
+  const char *d = (const char *)B->pass;
   for (auto &L : B->launches) {
-    if (L.mfma)
-      SQ_TRY(launch_cbatch_mfma(B->dt, B->states, B->g3m,
-                                (const uint8_t *)B->mtables + L.tab_off * mbytes, L.count,
-                                L.blocks, st));
+    if (L.cb)
+      SQ_TRY(launch_pass_entries(L.cb, B->dt, B->states, (const PassEntry *)d,
+                                 (const uint32_t *)(d + B->pass_map) + L.tab_off,
+                                 (const PassBlock *)(d + B->pass_desc), d + B->pass_img, L.blocks,
+                                 st));
     else
       hipLaunchKernelGGL(k_cbatch_dense<R>, dim3((unsigned)L.blocks), dim3(kBlock), 0, st, s,
                          (const T *)B->mats, B->tables + L.tab_off, L.count);
@@ -426,7 +484,7 @@ int cbatch_copy_state(void *handle, uint32_t circuit, void *dst, uint64_t nelems
 
 int cbatch_stats(void *handle, uint64_t *launches, double *state_bytes, double *traffic_bytes) {
   CBatch *B = (CBatch *)handle;
-  if (launches) *launches = B->launches.size() + 2;  // + the two initial-state kernels
+  if (launches) *launches = B->gate_launches + 2;  // + the two initial-state kernels
   if (state_bytes) *state_bytes = B->state_bytes;
   if (traffic_bytes) *traffic_bytes = B->traffic_bytes;
   return SQ_OK;

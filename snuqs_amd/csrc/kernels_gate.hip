@@ -565,7 +565,7 @@ struct TileRange {
   uint64_t first, end, step;
   int rbits;  // ORD 2: log2(ntiles), else 0
 };
-// Workgroup wg of nwg (the launch's grid, or a circuit batch entry's share).
+// Workgroup wg of nwg.
 template <int ORD>
 __device__ __forceinline__ TileRange tile_range(uint64_t ntiles, int wave, uint64_t wg,
                                                 uint64_t nwg) {
@@ -616,12 +616,9 @@ __host__ __device__ constexpr uint32_t swz_c64(uint32_t x) {
 // complex128: element (c, r) at slot 16r + c, swizzled by XOR (r & 15).
 __host__ __device__ constexpr uint32_t swz_c128(uint32_t x) { return x ^ ((x >> 4) & 15u); }
 
-// IM / SA: IdxMap and StageArgs by value (kernel arguments), or const
-// references into a circuit batch's entry table (read in place: the index
-// map is indexed at run time).
-template <bool PIPE, int ORD, typename IM = IdxMap, typename SA = StageArgs>
+template <bool PIPE, int ORD>
 __device__ __forceinline__ void
-    k_mfma5_c64_body(float2 *__restrict__ sv, uint64_t ntiles, IM im, SA sa,
+    k_mfma5_c64_body(float2 *__restrict__ sv, uint64_t ntiles, IdxMap im, StageArgs sa,
                 const float4 *__restrict__ G, uint64_t wg, uint64_t nwg) {
   constexpr int D = 32, NS = 16;
   __shared__ float4 As[D * D];      // [o][r], 16 KB
@@ -851,9 +848,9 @@ __global__ void __launch_bounds__(kBlock)
 #undef SQ_KW
 }
 
-template <bool PIPE, int ORD, typename IM = IdxMap, typename SA = StageArgs>
+template <bool PIPE, int ORD>
 __device__ __forceinline__ void
-    k_mfma5_c128_body(double2 *__restrict__ sv, uint64_t ntiles, IM im, SA sa,
+    k_mfma5_c128_body(double2 *__restrict__ sv, uint64_t ntiles, IdxMap im, StageArgs sa,
                  const typename Q4<double>::T *__restrict__ G, uint64_t wg, uint64_t nwg) {
   using D4 = typename Q4<double>::T;
   constexpr int D = 32, NS = 8, NT = 2;
@@ -1583,45 +1580,8 @@ static int launch_plan_t(const GatePlan &p, typename CV<R>::T *sv,
   return SQ_OK;
 }
 
-// ---------------------------------------------------------------------------
-// Circuit batches (kernels_cbatch.hip): gates of several circuits in one
-// launch on the 5-target MFMA kernels, each entry its own state, tiles,
-// workgroup range and matrix.
-// ---------------------------------------------------------------------------
-struct CBMfma {
-  uint64_t psi;          // amplitude offset of the circuit's state
-  uint64_t ntiles;       // tiles of the gate
-  uint64_t first_block;  // first workgroup of the entry in its launch
-  uint64_t nblocks;      // its workgroups (the tile loop's grid)
-  uint64_t g;            // offset of its matrix (3m layout, 4-real elements)
-  IdxMap im;
-  StageArgs sa;
-};
-
-template <bool C64, bool PIPE>
-__global__ void __launch_bounds__(kBlock)
-    k_cbatch_mfma5(void *__restrict__ states, const void *__restrict__ g3m,
-                   const CBMfma *__restrict__ tab, int count) {
-  int lo = 0, hi = count - 1;  // the entry holding this workgroup (uniform)
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (tab[mid].first_block <= blockIdx.x) lo = mid; else hi = mid - 1;
-  }
-  const CBMfma &m = tab[__builtin_amdgcn_readfirstlane(lo)];
-  const uint64_t wg = blockIdx.x - m.first_block;
-  if constexpr (C64)
-    k_mfma5_c64_body<PIPE, 0, const IdxMap &, const StageArgs &>(
-        (float2 *)states + m.psi, m.ntiles, m.im, m.sa, (const float4 *)g3m + m.g, wg, m.nblocks);
-  else
-    k_mfma5_c128_body<PIPE, 0, const IdxMap &, const StageArgs &>(
-        (double2 *)states + m.psi, m.ntiles, m.im, m.sa,
-        (const typename Q4<double>::T *)g3m + m.g, wg, m.nblocks);
-}
-
-size_t cbatch_mfma_entry_bytes() { return sizeof(CBMfma); }
-
 // Tiles per wave of a launch of the 4-5 target MFMA kernels over
-// `total_tiles` tiles (untuned programs, parameter and circuit batches): up
+// `total_tiles` tiles (untuned programs and parameter batches): up
 // to the mfma_tiles_per_wave knob (a wave that walks several tiles overlaps
 // the next tile's loads with this one's products and stages the block matrix
 // once for all of them), but never so many that the launch drops below
@@ -1631,52 +1591,6 @@ uint64_t mfma_wave_tiles(uint64_t total_tiles) {
   uint64_t t = (uint64_t)tuning().mfma_tiles_per_wave;
   while (t > 1 && total_tiles < 4 * t * kMinWaveTileBlocks) t >>= 1;
   return t;
-}
-
-uint64_t cbatch_mfma_tiles(const GatePlan &p, bool c64, uint64_t nelems) {
-  if (p.kind != Kind::DENSE || p.kk != 5) return 0;
-  const uint64_t tile_groups = c64 ? 32 : 16;
-  const uint64_t nfree = nelems >> (__builtin_popcountll(p.fixed_mask) + p.kk);
-  StageArgs sa{};
-  if (nfree < tile_groups || nfree % tile_groups || !make_stage(p, c64, &sa)) return 0;
-  return nfree / tile_groups;
-}
-
-bool cbatch_mfma_entry(const GatePlan &p, bool c64, uint64_t nelems, uint64_t psi,
-                       uint64_t first_block, uint64_t tiles_per_wave,
-                       std::vector<double> *g3m, void *entry, uint64_t *nblocks) {
-  if (p.kind != Kind::DENSE || p.kk != 5) return false;
-  const uint64_t tile_groups = c64 ? 32 : 16;
-  const uint64_t nfree = nelems >> (__builtin_popcountll(p.fixed_mask) + p.kk);
-  CBMfma e{};
-  if (nfree < tile_groups || nfree % tile_groups || !make_stage(p, c64, &e.sa)) return false;
-  e.psi = psi;
-  e.ntiles = nfree / tile_groups;
-  e.first_block = first_block;
-  const uint64_t cap = 256ull * (uint64_t)tuning().mfma_blocks_per_cu[c64 ? 0 : 1];
-  const uint64_t per = 4 * std::max<uint64_t>(tiles_per_wave, 1);  // tiles per workgroup
-  e.nblocks = std::min<uint64_t>((e.ntiles + per - 1) / per, cap);
-  e.im = make_idxmap(p.fixed_mask | target_mask(p), p.fixed_val);
-  e.g = g3m->size() / 4;
-  const std::vector<double> b = fused_block_3m(p);
-  g3m->insert(g3m->end(), b.begin(), b.end());
-  std::memcpy(entry, &e, sizeof(e));
-  *nblocks = e.nblocks;
-  return true;
-}
-
-int launch_cbatch_mfma(sq_dtype_t dt, void *states, const void *g3m, const void *tab, int count,
-                       uint64_t blocks, hipStream_t st) {
-  const bool c64 = dt == SQ_COMPLEX64;
-  const bool pipe = tuning().mfma5_pipeline[c64 ? 0 : 1] != 0;
-  const CBMfma *t = (const CBMfma *)tab;
-  const dim3 g((unsigned)blocks), b(kBlock);
-  if (c64 && pipe) hipLaunchKernelGGL((k_cbatch_mfma5<true, true>), g, b, 0, st, states, g3m, t, count);
-  else if (c64) hipLaunchKernelGGL((k_cbatch_mfma5<true, false>), g, b, 0, st, states, g3m, t, count);
-  else if (pipe) hipLaunchKernelGGL((k_cbatch_mfma5<false, true>), g, b, 0, st, states, g3m, t, count);
-  else hipLaunchKernelGGL((k_cbatch_mfma5<false, false>), g, b, 0, st, states, g3m, t, count);
-  SQ_HIP(hipGetLastError());
-  return SQ_OK;
 }
 
 int launch_plan(const GatePlan &p, void *sv, sq_dtype_t dt, uint64_t nelems,

@@ -29,8 +29,8 @@
 
 namespace sq {
 
-// Workgroups of a pass: one chunk each (a dispatch holds fewer than 2^32
-// work-items).
+// Workgroups of a pass in x (one chunk each); the rest go to z (a dimension
+// holds fewer than 2^32 work-items).
 constexpr uint64_t kPassGrid = 1ull << 22;
 
 typedef float pfloatx16 __attribute__((ext_vector_type(16)));
@@ -287,27 +287,32 @@ struct PassShape {
 };
 
 template <typename R, int CB>
-__global__ void __launch_bounds__((PassShape<R, CB>::NT), (PassShape<R, CB>::NW == 8 ? 4 : PassShape<R, CB>::NW == 4 ? 3 : 2))
-    k_pass(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t nchunks, PassGeom geom,
-           const PassBlock *__restrict__ blocks, int nblocks, const char *__restrict__ image,
-           uint64_t gstride) {
-  using T = typename CV<R>::T;
+struct PassLds {
+  typename CV<R>::T x[1 << CB];
+  float4 a[sizeof(R) == 4 ? 768 : 1024];
+};
+
+// The pass on chunk c of a state: by every thread of the workgroup.  initial:
+// the state is |0...0> and is not read.
+template <typename R, int CB>
+__device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, uint64_t c,
+                                           const PassGeom &geom,
+                                           const PassBlock *__restrict__ blocks, int nblocks,
+                                           const nt_f4 *__restrict__ G, bool initial,
+                                           PassLds<R, CB> &lds) {
   using S = PassShape<R, CB>;
   constexpr bool c64 = sizeof(R) == 4;
   constexpr int NT = S::NT, NW = S::NW, NL = S::NL;
   constexpr int WB = CB - (c64 ? 10 : 9);             // wave index bits
-  constexpr int TB = 6 + (NW == 8 ? 3 : NW == 4 ? 2 : NW == 2 ? 1 : 0);  // thread index bits
+  constexpr int TB = 6 + WB;                          // thread index bits
   constexpr int E0 = c64 ? 1 : 0;                     // chunk bit of thread bit 0 (16 B per access)
   constexpr int EK = E0 + TB;                         // chunk bit of access index bit 0
   constexpr int ITEM = c64 ? 8 : 16;
   constexpr int NP = (c64 ? 768 + NT - 1 : 1024) / NT;  // 16-byte units of a block matrix per thread
-  __shared__ T Xs[1 << CB];
-  __shared__ float4 As[c64 ? 768 : 1024];
-  char *X = reinterpret_cast<char *>(Xs);
+  static_assert(NW == 1 << WB, "one wave a tile");
+  char *X = reinterpret_cast<char *>(lds.x);
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  sv += blockIdx.y * sstride;
-  const nt_f4 *G = reinterpret_cast<const nt_f4 *>(image + blockIdx.y * gstride);
   uint64_t la = 0;
   uint32_t tw = 0;
 #pragma unroll
@@ -341,63 +346,106 @@ __global__ void __launch_bounds__((PassShape<R, CB>::NT), (PassShape<R, CB>::NW 
         pre[i] = g[u < b.n16 ? u : b.n16 - 1];
       }
   };
-  auto chunk = [&](uint64_t c) {
-    uint64_t base = c;
-    for (int j = 0; j < geom.nins; ++j) {
-      const uint64_t lo = base & geom.lowmask[j];
-      base = ((base ^ lo) << 1) | lo;
+  uint64_t base = c;
+  for (int j = 0; j < geom.nins; ++j) {
+    const uint64_t lo = base & geom.lowmask[j];
+    base = ((base ^ lo) << 1) | lo;
+  }
+  typename CV<R>::T *p = sv + ((base << geom.shift) + la);
+  nt_f4 v[NL];
+  if (initial) {
+#pragma unroll
+    for (int k = 0; k < NL; ++k) v[k] = nt_f4{0.f, 0.f, 0.f, 0.f};
+    if (c != 0) {  // stays zero
+#pragma unroll
+      for (int k = 0; k < NL; ++k)
+        __builtin_nontemporal_store(v[k], reinterpret_cast<nt_f4 *>(p + ka(k)));
+      return;
     }
-    return sv + ((base << geom.shift) + la);
-  };
-  for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-    T *p = chunk(c);
-    nt_f4 v[NL];
+    if (t == 0) {
+      if constexpr (c64) {
+        v[0].x = 1.f;
+      } else {
+        const double2 one = make_double2(1.0, 0.0);
+        __builtin_memcpy(&v[0], &one, 16);
+      }
+    }
+  } else {
 #pragma unroll
     for (int k = 0; k < NL; ++k)
       v[k] = __builtin_nontemporal_load(reinterpret_cast<const nt_f4 *>(p + ka(k)));
-    nt_f4 pre[NP];
-    fetch(pre, blocks);
-    if (c != blockIdx.x) __syncthreads();  // the last chunk has been read out
+  }
+  nt_f4 pre[NP];
+  fetch(pre, blocks);
 #pragma unroll
-    for (int k = 0; k < NL; ++k) {
-      if constexpr (c64) {
-        *reinterpret_cast<float2 *>(X + (tw ^ kw(k))) = make_float2(v[k].x, v[k].y);
-        *reinterpret_cast<float2 *>(X + (tw ^ kw(k) ^ ITEM)) = make_float2(v[k].z, v[k].w);
-      } else {
-        *reinterpret_cast<nt_f4 *>(X + (tw ^ kw(k))) = v[k];
-      }
-    }
-    for (int j = 0; j < nblocks; ++j) {
-      const PassBlock b = load_block(blocks + j);
-#pragma unroll
-      for (int i = 0; i < NP; ++i)
-        if (t + i * NT < b.n16) reinterpret_cast<nt_f4 *>(As)[t + i * NT] = pre[i];
-      __syncthreads();
-      if (j + 1 < nblocks) fetch(pre, blocks + j + 1);  // arrives during this block's products
-      uint32_t lb = xor_lane<c64 ? 5 : 4>(b.col, lane);
-      lb ^= xor_lane<WB>(b.wave, wave);
-      if (b.k == 5) {
-        if constexpr (c64) pass_block5(X, reinterpret_cast<const pbf8 *>(As), b, lane, lb);
-        else pass_block5(X, reinterpret_cast<const double2 *>(As), b, lane, lb);
-      } else {
-        if constexpr (c64) pass_block4(X, reinterpret_cast<const pbf8 *>(As), b, lane, lb, b.wave[WB]);
-        else pass_block4(X, reinterpret_cast<const double *>(As), b, lane, lb, b.wave[WB]);
-      }
-      __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < NL; ++k) {
-      nt_f4 o;
-      if constexpr (c64) {
-        const float2 y0 = *reinterpret_cast<const float2 *>(X + (tw ^ kw(k)));
-        const float2 y1 = *reinterpret_cast<const float2 *>(X + (tw ^ kw(k) ^ ITEM));
-        o = nt_f4{y0.x, y0.y, y1.x, y1.y};
-      } else {
-        o = *reinterpret_cast<const nt_f4 *>(X + (tw ^ kw(k)));
-      }
-      __builtin_nontemporal_store(o, reinterpret_cast<nt_f4 *>(p + ka(k)));
+  for (int k = 0; k < NL; ++k) {
+    if constexpr (c64) {
+      *reinterpret_cast<float2 *>(X + (tw ^ kw(k))) = make_float2(v[k].x, v[k].y);
+      *reinterpret_cast<float2 *>(X + (tw ^ kw(k) ^ ITEM)) = make_float2(v[k].z, v[k].w);
+    } else {
+      *reinterpret_cast<nt_f4 *>(X + (tw ^ kw(k))) = v[k];
     }
   }
+  for (int j = 0; j < nblocks; ++j) {
+    const PassBlock b = load_block(blocks + j);
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (t + i * NT < b.n16) reinterpret_cast<nt_f4 *>(lds.a)[t + i * NT] = pre[i];
+    __syncthreads();
+    if (j + 1 < nblocks) fetch(pre, blocks + j + 1);  // arrives during this block's products
+    uint32_t lb = xor_lane<c64 ? 5 : 4>(b.col, lane);
+    lb ^= xor_lane<WB>(b.wave, wave);
+    if (b.k == 5) {
+      if constexpr (c64) pass_block5(X, reinterpret_cast<const pbf8 *>(lds.a), b, lane, lb);
+      else pass_block5(X, reinterpret_cast<const double2 *>(lds.a), b, lane, lb);
+    } else {
+      if constexpr (c64)
+        pass_block4(X, reinterpret_cast<const pbf8 *>(lds.a), b, lane, lb, b.wave[WB]);
+      else
+        pass_block4(X, reinterpret_cast<const double *>(lds.a), b, lane, lb, b.wave[WB]);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < NL; ++k) {
+    nt_f4 o;
+    if constexpr (c64) {
+      const float2 y0 = *reinterpret_cast<const float2 *>(X + (tw ^ kw(k)));
+      const float2 y1 = *reinterpret_cast<const float2 *>(X + (tw ^ kw(k) ^ ITEM));
+      o = nt_f4{y0.x, y0.y, y1.x, y1.y};
+    } else {
+      o = *reinterpret_cast<const nt_f4 *>(X + (tw ^ kw(k)));
+    }
+    __builtin_nontemporal_store(o, reinterpret_cast<nt_f4 *>(p + ka(k)));
+  }
+}
+
+#define SQ_PASS_BOUNDS \
+  __launch_bounds__((PassShape<R, CB>::NT), \
+                    (PassShape<R, CB>::NW == 8 ? 4 : PassShape<R, CB>::NW == 4 ? 3 : 2))
+
+template <typename R, int CB>
+__global__ void SQ_PASS_BOUNDS
+    k_pass(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t nchunks, PassGeom geom,
+           const PassBlock *__restrict__ blocks, int nblocks, const char *__restrict__ image,
+           uint64_t gstride) {
+  __shared__ PassLds<R, CB> lds;
+  const nt_f4 *G = reinterpret_cast<const nt_f4 *>(image + blockIdx.y * gstride);
+  const uint64_t c = (uint64_t)blockIdx.z * gridDim.x + blockIdx.x;
+  if (c < nchunks)
+    pass_chunk<R, CB>(sv + blockIdx.y * sstride, c, geom, blocks, nblocks, G, false, lds);
+}
+
+// Circuit batches: workgroup w takes chunk w - first of its entry.
+template <typename R, int CB>
+__global__ void SQ_PASS_BOUNDS
+    k_pass_entries(typename CV<R>::T *__restrict__ states, const PassEntry *__restrict__ entries,
+                   const uint32_t *__restrict__ entry, const PassBlock *__restrict__ blocks,
+                   const char *__restrict__ images) {
+  __shared__ PassLds<R, CB> lds;
+  const PassEntry &e = entries[__builtin_amdgcn_readfirstlane(entry[blockIdx.x])];
+  pass_chunk<R, CB>(states + e.psi, blockIdx.x - e.first, e.geom, blocks + e.blocks, e.nblocks,
+                    reinterpret_cast<const nt_f4 *>(images + e.image), e.initial != 0, lds);
 }
 
 template <typename R, int CB>
@@ -406,9 +454,36 @@ static void launch_pass_cb(const PassGeom &geom, void *sv, uint64_t nelems, uint
                            uint64_t gstride, hipStream_t st) {
   const uint64_t nchunks = nelems >> CB;
   const uint64_t g = std::min<uint64_t>(nchunks, kPassGrid);
-  hipLaunchKernelGGL((k_pass<R, CB>), dim3((unsigned)g, nsets), dim3(PassShape<R, CB>::NT), 0, st,
+  hipLaunchKernelGGL((k_pass<R, CB>), dim3((unsigned)g, nsets, (unsigned)((nchunks + g - 1) / g)), dim3(PassShape<R, CB>::NT), 0, st,
                      (typename CV<R>::T *)sv, nelems, nchunks, geom, blocks, nblocks,
                      (const char *)image, gstride);
+}
+
+// SQ_PASS(R, CB) for the dtype and chunk size.
+#define SQ_PASS_SWITCH(cb)                                                      \
+  switch ((dt == SQ_COMPLEX64 ? 0 : 100) + (cb)) {                              \
+    case 10: SQ_PASS(float, 10); break;                                         \
+    case 11: SQ_PASS(float, 11); break;                                         \
+    case 12: SQ_PASS(float, 12); break;                                         \
+    case 13: SQ_PASS(float, 13); break;                                         \
+    case 109: SQ_PASS(double, 9); break;                                        \
+    case 110: SQ_PASS(double, 10); break;                                       \
+    case 111: SQ_PASS(double, 11); break;                                       \
+    case 112: SQ_PASS(double, 12); break;                                       \
+    default: return fail(SQ_ERR_INVALID, "internal: pass chunk size");          \
+  }
+
+int launch_pass_entries(int cb, sq_dtype_t dt, void *states, const PassEntry *entries,
+                        const uint32_t *entry, const PassBlock *blocks, const void *images,
+                        uint64_t nwg, hipStream_t st) {
+#define SQ_PASS(R, CB)                                                                        \
+  hipLaunchKernelGGL((k_pass_entries<R, CB>), dim3((unsigned)nwg), dim3(PassShape<R, CB>::NT), \
+                     0, st, (typename CV<R>::T *)states, entries, entry, blocks,              \
+                     (const char *)images)
+  SQ_PASS_SWITCH(cb)
+#undef SQ_PASS
+  SQ_HIP(hipGetLastError());
+  return SQ_OK;
 }
 
 int launch_pass(const PassPlan &p, const PassGeom &geom, sq_dtype_t dt, void *sv,
@@ -418,23 +493,7 @@ int launch_pass(const PassPlan &p, const PassGeom &geom, sq_dtype_t dt, void *sv
     return fail(SQ_ERR_INVALID, "internal: pass does not fit the state");
 #define SQ_PASS(R, CB) \
   launch_pass_cb<R, CB>(geom, sv, nelems, nsets, blocks, nblocks, image, gstride, st)
-  if (dt == SQ_COMPLEX64) {
-    switch (p.cb) {
-      case 10: SQ_PASS(float, 10); break;
-      case 11: SQ_PASS(float, 11); break;
-      case 12: SQ_PASS(float, 12); break;
-      case 13: SQ_PASS(float, 13); break;
-      default: return fail(SQ_ERR_INVALID, "internal: pass chunk size");
-    }
-  } else {
-    switch (p.cb) {
-      case 9: SQ_PASS(double, 9); break;
-      case 10: SQ_PASS(double, 10); break;
-      case 11: SQ_PASS(double, 11); break;
-      case 12: SQ_PASS(double, 12); break;
-      default: return fail(SQ_ERR_INVALID, "internal: pass chunk size");
-    }
-  }
+  SQ_PASS_SWITCH(p.cb)
 #undef SQ_PASS
   SQ_HIP(hipGetLastError());
   return SQ_OK;

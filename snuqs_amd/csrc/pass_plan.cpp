@@ -108,21 +108,24 @@ static void make_blocks(const std::vector<int> &gates, const std::vector<uint64_
   }
 }
 
-void plan_passes(int nq, sq_dtype_t dt, const std::vector<uint64_t> &masks,
-                 const std::vector<double> &touched, std::vector<Step> *steps,
-                 std::vector<PassPlan> *passes) {
+int pass_min_bits(sq_dtype_t dt) { return dt == SQ_COMPLEX64 ? 10 : 9; }
+
+// Larger chunks hold more gates per pass; from 2^21 amplitudes on the chunks
+// still fill the chip (layered circuits of depth 10, fused, complex64: 22 qubits
+// 295 us with 2^13-amplitude chunks, 356 us with 2^12; 16 qubits 124 against
+// 91 us).
+int pass_chunk_bits(sq_dtype_t dt, int nbits) {
+  const int cmax = dt == SQ_COMPLEX64 ? 13 : 12;  // 64 KiB of LDS
+  return std::min(nbits, nbits >= 21 ? cmax : cmax - 1);
+}
+
+void plan_passes(int nq, int cb, sq_dtype_t dt, const std::vector<uint64_t> &masks,
+                 const double *touched, std::vector<Step> *steps, std::vector<PassPlan> *passes) {
   steps->clear();
   passes->clear();
   const int ng = (int)masks.size();
   const bool c64 = dt == SQ_COMPLEX64;
-  const int cmin = c64 ? 10 : 9;      // one 5-target tile
-  const int cmax = c64 ? 13 : 12;     // 64 KiB
-  // Larger chunks hold more gates per pass; from 21 qubits on the chunks
-  // still fill the chip (layered circuits of depth 10, fused: 22 qubits 295 us
-  // with the largest chunk, 356 us with the next smaller; 16 qubits 124 against
-  // 91 us).
-  const int cb = std::min(nq, nq >= 21 ? cmax : cmax - 1);
-  if (nq < cmin) {
+  if (cb < pass_min_bits(dt)) {
     for (int g = 0; g < ng; ++g) steps->push_back({g, -1});
     return;
   }
@@ -181,8 +184,9 @@ void plan_passes(int nq, sq_dtype_t dt, const std::vector<uint64_t> &masks,
       taken.insert(taken.end(), btaken.begin(), btaken.end());
     }
     double sweeps = 0.0;
-    for (int g : taken) sweeps += touched[g];
-    if (taken.size() >= 2 && sweeps > 1.0) {
+    if (touched)
+      for (int g : taken) sweeps += touched[g];
+    if (!touched || (taken.size() >= 2 && sweeps > 1.0)) {
       PassPlan p;
       for (int b = 0; b < nq && __builtin_popcountll(set) < cb; ++b) set |= 1ull << b;
       p.local = set;

@@ -37,12 +37,19 @@ struct Step {
   int pass = -1;
 };
 
-// Steps of a gate list on an nq-bit state.  masks[g]: the state bits gate g
-// acts on (0 for a global phase); touched[g]: the fraction of the amplitudes
-// it changes.  Gates are reordered only past gates they share no bit with.
-void plan_passes(int nq, sq_dtype_t dt, const std::vector<uint64_t> &masks,
-                 const std::vector<double> &touched, std::vector<Step> *steps,
-                 std::vector<PassPlan> *passes);
+// Smallest chunk (one 5-target tile) and the chunk for launches over 2^nbits
+// amplitudes.
+int pass_min_bits(sq_dtype_t dt);
+int pass_chunk_bits(sq_dtype_t dt, int nbits);
+
+// Steps of a gate list on an nq-bit state in chunks of 2^cb amplitudes (cb <=
+// nq; every step is one gate when cb < pass_min_bits).  masks[g]: the state
+// bits gate g acts on (0 for a global phase); touched[g]: the fraction of the
+// amplitudes it changes, or nullptr where gates have no kernels of their own
+// and every step is to be a pass.  Gates are reordered only past gates they
+// share no bit with.
+void plan_passes(int nq, int cb, sq_dtype_t dt, const std::vector<uint64_t> &masks,
+                 const double *touched, std::vector<Step> *steps, std::vector<PassPlan> *passes);
 
 // Device form of one block: byte offsets in the chunk's LDS image that the
 // block's column (group), wave and row (amplitude) index bits stand for; an
@@ -79,6 +86,22 @@ struct PassGates {
 };
 void pass_image(const PassPlan &p, const std::vector<PassBlock> &blocks, sq_dtype_t dt,
                 const PassGates &g, char *img);
+
+// One circuit's pass within a launch over many (kernels_cbatch.hip).
+struct PassEntry {
+  uint64_t psi;       // amplitude offset of the circuit's state
+  uint64_t first;     // first workgroup of the entry: one workgroup a chunk
+  uint64_t blocks;    // index of its first block descriptor
+  uint64_t image;     // byte offset of its matrix image
+  int nblocks;
+  int initial;        // the state is |0...0>, not read
+  PassGeom geom;
+};
+// Launch `nwg` workgroups over a table of entries of one chunk size; entry[w] is
+// workgroup w's entry.
+int launch_pass_entries(int cb, sq_dtype_t dt, void *states, const PassEntry *entries,
+                        const uint32_t *entry, const PassBlock *blocks, const void *images,
+                        uint64_t nwg, hipStream_t stream);
 
 // Launch a pass over nsets states of nelems amplitudes (state y at
 // sv + y * nelems, its matrices at image + y * gstride bytes).

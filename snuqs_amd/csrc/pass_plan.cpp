@@ -110,13 +110,14 @@ static void make_blocks(const std::vector<int> &gates, const std::vector<uint64_
 
 int pass_min_bits(sq_dtype_t dt) { return dt == SQ_COMPLEX64 ? 10 : 9; }
 
-// Larger chunks hold more gates per pass; from 2^21 amplitudes on the chunks
-// still fill the chip (layered circuits of depth 10, fused, complex64: 22 qubits
-// 295 us with 2^13-amplitude chunks, 356 us with 2^12; 16 qubits 124 against
-// 91 us).
+// Larger chunks hold more gates per pass; these sizes on they still fill the chip
+// (layered circuits of depth 10, fused: complex64 19 qubits 129 us with
+// 2^13-amplitude chunks and 113 us with 2^12, 20 qubits 122 and 124 us, 22 qubits
+// 295 and 356 us; complex128 20 qubits 188 us with 2^12 and 180 us with 2^11, 22
+// qubits 563 and 601 us; 64 sets of 20 qubits complex64 7.4 and 8.3 ms).
 int pass_chunk_bits(sq_dtype_t dt, int nbits) {
   const int cmax = dt == SQ_COMPLEX64 ? 13 : 12;  // 64 KiB of LDS
-  return std::min(nbits, nbits >= 21 ? cmax : cmax - 1);
+  return std::min(nbits, nbits >= (dt == SQ_COMPLEX64 ? 20 : 21) ? cmax : cmax - 1);
 }
 
 void plan_passes(int nq, int cb, sq_dtype_t dt, const std::vector<uint64_t> &masks,

@@ -35,33 +35,37 @@ from ._C.operation import GateOperation
 from ._C.operation import gate_operations as g
 
 
-def _gt(op1, i, op2, j) -> bool:
-    t1, t2 = op1.targets, op2.targets
-    if not t1 and not t2:
-        return i < j
-    if not t1:
-        return True
-    if not t2:
-        return False
-    if set(t1) & set(t2):
-        return i < j
-    s1, s2 = op1.sliceable(), op2.sliceable()
-    if s1 and s2:
-        return i < j
-    if s1 != s2:
-        return s1
-    return min(t1) > min(t2)
-
-
 def pseudo_sort_operations_descending(operations):
     ops = list(operations)
+    # what the comparison looks at: the targets as a bit mask (qubits numbered as
+    # they come), the smallest one and sliceable(), read from each gate once
+    keys, number = [], {}
+    for op in ops:
+        t, mask = op.targets, 0
+        for q in t:
+            mask |= 1 << number.setdefault(q, len(number))
+        keys.append((mask, min(t, default=0), op.sliceable()))
     for i in range(1, len(ops)):
-        cur = ops[i]
+        cur, key = ops[i], keys[i]
+        mask, low, sl = key
         j = i - 1
-        while j >= 0 and _gt(cur, i, ops[j], j):
-            ops[j + 1] = ops[j]
+        while j >= 0:
+            mask2, low2, sl2 = keys[j]
+            # whether `cur` goes before ops[j]: program order (no) where both
+            # have no targets, share a qubit or are sliceable
+            if not mask:
+                if not mask2:
+                    break
+            elif not mask2 or mask & mask2 or (sl and sl2):
+                break
+            elif sl != sl2:
+                if not sl:
+                    break
+            elif not low > low2:
+                break
+            ops[j + 1], keys[j + 1] = ops[j], keys[j]
             j -= 1
-        ops[j + 1] = cur
+        ops[j + 1], keys[j + 1] = cur, key
     return ops
 
 

@@ -1021,7 +1021,7 @@ static int expect_terms_locked(Workspace *w, const void *sv, sq_dtype_t dt, uint
   // at most 64 terms per launch (partials hold 64 x kRedBlocks values)
   for (uint32_t t0 = 0; t0 < nterms; t0 += 64) {
     const uint32_t c = std::min<uint32_t>(64, nterms - t0);
-    SQ_TRY(launch_pauli_terms(sv, dt, n, (int)c,
+    SQ_TRY(launch_pauli_terms(sv, dt, n, (int)c, x + t0,
                               (const char *)L.terms + t0 * pauli_term_bytes(),
                               L.alpha + t0, L.partial, L.vals + t0, st));
   }
@@ -1142,7 +1142,7 @@ int sq_expect_pauli_sum_noalloc(const void *sv, sq_dtype_t dt, uint64_t n, uint3
   SQ_HIP(hipMemcpyAsync(alpha, halpha, nterms * sizeof(double), hipMemcpyHostToDevice, st));
   for (uint32_t t0 = 0; t0 < nterms; t0 += 64) {
     const uint32_t c = std::min<uint32_t>(64, nterms - t0);
-    SQ_TRY(launch_pauli_terms(sv, dt, n, (int)c, terms + t0 * tb, alpha + t0, partial,
+    SQ_TRY(launch_pauli_terms(sv, dt, n, (int)c, x + t0, terms + t0 * tb, alpha + t0, partial,
                               vals + t0, st));
   }
   SQ_HIP(hipMemcpyAsync(hvals, vals, nterms * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -2455,7 +2455,7 @@ int sq_expect_pauli_sum_batch(const void *states, sq_dtype_t dt, uint64_t n, uin
     for (uint32_t t0 = 0; t0 < nterms; t0 += tc) {
       const uint32_t c = std::min(tc, nterms - t0);
       SQ_TRY(launch_pauli_terms_batch((const char *)states + s0 * n * itemsize(dt), dt, n, ns,
-                                      (int)c, terms + t0 * pauli_term_bytes(), alpha + t0,
+                                      (int)c, x + t0, terms + t0 * pauli_term_bytes(), alpha + t0,
                                       partial, vals + (size_t)s0 * nterms + t0, nterms, st));
     }
   }

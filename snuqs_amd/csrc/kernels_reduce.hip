@@ -10,6 +10,7 @@
 
 #include "kernels.hpp"
 #include "kernels_reduce.hpp"
+#include "pass_plan.hpp"
 
 namespace sq {
 
@@ -127,14 +128,22 @@ struct PauliTerm {
   int pad;
 };
 
+// The terms of a launch, of the nterms whose partial rows it fills.
+constexpr int kPauliLaunch = 64;
+struct PauliIds {
+  int count, nterms;
+  uint8_t id[kPauliLaunch];
+};
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    k_partial_pauli(const T *__restrict__ sv, uint64_t n,
-                    const PauliTerm *__restrict__ terms, double *partial) {
+    k_partial_pauli(const T *__restrict__ sv, uint64_t n, const PauliTerm *__restrict__ terms,
+                    PauliIds ids, double *partial) {
   // blockIdx.z: state z of a batch of consecutive n-amplitude states (0 for
-  // one state); partial row (z, term) at (z * gridDim.y + y) * gridDim.x
+  // one state); partial row (z, term) at (z * nterms + term) * gridDim.x
   sv += (uint64_t)blockIdx.z * n;
-  const PauliTerm pt = terms[blockIdx.y];
+  const int term = ids.id[blockIdx.y];
+  const PauliTerm pt = terms[term];
   double acc = 0.0, dummy = 0.0;
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
   if (pt.x == 0) {
@@ -160,7 +169,145 @@ __global__ void __launch_bounds__(kBlock)
   }
   block_sum2(acc, dummy);
   if (threadIdx.x == 0)
-    partial[((uint64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = acc;
+    partial[((uint64_t)blockIdx.z * ids.nterms + term) * gridDim.x + blockIdx.x] = acc;
+}
+
+// The terms of a group, whose x masks lie inside the local bits of one chunk
+// geometry (kernels_pass.hip): a workgroup reads a chunk into LDS once and forms
+// every term's sum over it from there, where k_partial_pauli reads the whole
+// state once per term.  FP64 products and sums as there; a term's sums of eight
+// are reduced over the wave together (ten shuffles instead of 48).
+// 64 strings of weight 4 on 64 states of 20 qubits, complex64 (34 GB of term
+// reads, 2.2 GB in chunks): 2.6 -> 2.0 ms; the sums are then bound by the
+// conversions to FP64.
+constexpr int kChunkThreads = 512;
+template <typename T>
+struct PauliChunkLds {
+  static constexpr int CB = sizeof(T) == 8 ? 13 : 12;
+  T x[1 << CB];
+  double acc[kChunkThreads / 64][kPauliLaunch];
+  uint32_t xl[kPauliLaunch], zl[kPauliLaunch];  // masks on chunk bits
+  uint64_t zh[kPauliLaunch];                    // z outside the chunk
+  int odd[kPauliLaunch];
+};
+
+// One term's sum over the chunk, this thread's share.
+template <typename T>
+__device__ __forceinline__ double pauli_chunk_term(const PauliChunkLds<T> &s, int k, uint64_t base) {
+  constexpr int CB = PauliChunkLds<T>::CB, NP = (1 << (CB - 1)) / kChunkThreads;
+  const uint32_t xl = __builtin_amdgcn_readfirstlane(s.xl[k]);
+  const uint32_t zl = __builtin_amdgcn_readfirstlane(s.zl[k]);
+  const int odd = __builtin_amdgcn_readfirstlane(s.odd[k]);
+  const uint32_t t = threadIdx.x;
+  const int neg = __popcll(base & s.zh[k]) & 1;
+  double acc = 0.0;
+  uint32_t dt;
+  if (xl == 0) {
+    dt = t;
+#pragma unroll
+    for (int q = 0; q < 2 * NP; ++q) {
+      const double2 v = ld2(s.x, dt + kChunkThreads * q);
+      const double sg = __popc((kChunkThreads * q) & zl) & 1 ? -1.0 : 1.0;
+      acc += sg * (v.x * v.x + v.y * v.y);
+    }
+  } else {
+    const uint32_t hm = (1u << (31 - __clz(xl))) - 1;  // pairs have the top bit of x clear
+    dt = ((t & ~hm) << 1) | (t & hm);
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+      const uint32_t f = kChunkThreads * q, dq = ((f & ~hm) << 1) | (f & hm);
+      const double2 a = ld2(s.x, dt | dq), b = ld2(s.x, (dt | dq) ^ xl);
+      const double sg = __popc(dq & zl) & 1 ? -1.0 : 1.0;
+      // conj(b) * a
+      const double v = odd ? b.x * a.y - b.y * a.x : b.x * a.x + b.y * a.y;
+      acc += sg * v;
+    }
+  }
+  return (neg ^ (__popc(dt & zl) & 1)) ? -acc : acc;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kChunkThreads, 4)
+    k_pauli_chunk(const T *__restrict__ sv, uint64_t n, uint64_t nchunks, PassGeom geom,
+                  const PauliTerm *__restrict__ terms, PauliIds ids, int nb,
+                  double *__restrict__ partial) {
+  using L = PauliChunkLds<T>;
+  constexpr int CB = L::CB, NL = (1 << CB) * (int)sizeof(T) / 16 / kChunkThreads;
+  constexpr int E0 = sizeof(T) == 8 ? 1 : 0;  // chunk bit of thread bit 0 (16 B per access)
+  constexpr int EK = E0 + 9;                  // chunk bit of access index bit 0
+  __shared__ L s;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  sv += (uint64_t)blockIdx.z * n;
+  if (t < ids.count) {
+    const PauliTerm pt = terms[ids.id[t]];
+    uint32_t xl = 0, zl = 0;
+    uint64_t local = 0;
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+      xl |= (pt.x & geom.addr[i]) ? 1u << i : 0u;
+      zl |= (pt.z & geom.addr[i]) ? 1u << i : 0u;
+      local |= geom.addr[i];
+    }
+    s.xl[t] = xl;
+    s.zl[t] = zl;
+    s.zh[t] = pt.z & ~local;
+    s.odd[t] = pt.ny & 1;
+  }
+  s.acc[wave][lane] = 0.0;  // 8 rows of 64
+  uint64_t la = 0;
+#pragma unroll
+  for (int i = 0; i < 9; ++i)
+    if ((t >> i) & 1) la += geom.addr[i + E0];
+  for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
+    uint64_t base = c;
+    for (int j = 0; j < geom.nins; ++j) {
+      const uint64_t lo = base & geom.lowmask[j];
+      base = ((base ^ lo) << 1) | lo;
+    }
+    base <<= geom.shift;
+    const T *p = sv + (base + la);
+    nt_f4 v[NL];
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      uint64_t a = 0;
+#pragma unroll
+      for (int i = 0; i < CB - EK; ++i) a += ((k >> i) & 1) ? geom.addr[EK + i] : 0;
+      v[k] = *reinterpret_cast<const nt_f4 *>(p + a);
+    }
+    if (c != blockIdx.x) __syncthreads();  // the last chunk's reads are done
+#pragma unroll
+    for (int k = 0; k < NL; ++k) reinterpret_cast<nt_f4 *>(s.x)[t + kChunkThreads * k] = v[k];
+    __syncthreads();
+    for (int k0 = 0; k0 < ids.count; k0 += 8) {
+      double a[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a[u] = k0 + u < ids.count ? pauli_chunk_term<T>(s, k0 + u, base) : 0.0;
+      // lanes 32-63 take over terms 4-7, then 16-31 of each half the upper two,
+      // then 8-15 the upper one; the last eight lanes sum one term
+#pragma unroll
+      for (int w = 4; w >= 1; w >>= 1) {
+        const bool up = lane & (8 * w);
+#pragma unroll
+        for (int u = 0; u < w; ++u) {
+          const double give = up ? a[u] : a[u + w], keep = up ? a[u + w] : a[u];
+          a[u] = keep + __shfl_xor(give, 8 * w);
+        }
+      }
+#pragma unroll
+      for (int w = 4; w >= 1; w >>= 1) a[0] += __shfl_xor(a[0], w);
+      const int u = ((lane >> 5) & 1) * 4 + ((lane >> 4) & 1) * 2 + ((lane >> 3) & 1);
+      if ((lane & 7) == 0 && k0 + u < ids.count) s.acc[wave][k0 + u] += a[0];
+    }
+  }
+  __syncthreads();
+  if (t < ids.count) {
+    double a = 0.0;
+#pragma unroll
+    for (int w = 0; w < kChunkThreads / 64; ++w) a += s.acc[w][t];
+    double *row = partial + ((uint64_t)blockIdx.z * ids.nterms + ids.id[t]) * nb;
+    row[blockIdx.x] = a;
+    for (int b = blockIdx.x + gridDim.x; b < nb; b += gridDim.x) row[b] = 0.0;
+  }
 }
 
 // out_j = sum_t c'_t (-1)^popcount((j^x_t) & z_t) in_{j^x_t},  c'_t = c_t i^ny_t
@@ -1053,19 +1200,103 @@ int launch_inner(const void *a, const void *b, sq_dtype_t dt, uint64_t n,
   return SQ_OK;
 }
 
-// terms_dev: PauliTerm[nterms] on the device; alpha_dev: per-term factors
-// (2*i^ny folded in); out_dev[t] = term value.
-int launch_pauli_terms(const void *sv, sq_dtype_t dt, uint64_t n, int nterms,
+// Groups of a launch's terms that one chunk geometry serves: the chunk's low
+// bits (128-byte runs) and the bits that the x masks still need most.
+struct PauliGroups {  // no heap: callers that cannot allocate use them too
+  int count = 0;
+  uint64_t local[kPauliLaunch / 3];
+  PauliIds ids[kPauliLaunch / 3];
+  PauliIds rest{};
+};
+static void pauli_groups(const uint64_t *x, int nterms, int nbits, int cb, int run,
+                         PauliGroups *out) {
+  out->rest.nterms = nterms;
+  int left[kPauliLaunch], nleft = nterms;
+  for (int t = 0; t < nterms; ++t) left[t] = t;
+  // a group reads the state once; below three terms the per-term kernel does no
+  // worse
+  while (nleft >= 3) {
+    uint64_t local = (1ull << run) - 1;
+    for (int room = cb - run; room > 0; --room) {
+      double score[64] = {0.0};
+      int best = -1;
+      for (int i = 0; i < nleft; ++i) {
+        const uint64_t need = x[left[i]] & ~local;
+        const int k = __builtin_popcountll(need);
+        if (k == 0 || k > room) continue;
+        for (uint64_t m = need; m; m &= m - 1) {
+          const int b = __builtin_ctzll(m);
+          score[b] += std::ldexp(1.0, -2 * k);
+          if (best < 0 || score[b] > score[best]) best = b;
+        }
+      }
+      if (best < 0) break;
+      local |= 1ull << best;
+    }
+    PauliIds &ids = out->ids[out->count];
+    ids.count = 0;
+    ids.nterms = nterms;
+    int keep = 0, kept[kPauliLaunch];
+    for (int i = 0; i < nleft; ++i) {
+      if (x[left[i]] & ~local) kept[keep++] = left[i];
+      else ids.id[ids.count++] = (uint8_t)left[i];
+    }
+    if (ids.count < 3) break;
+    for (int b = 0; b < nbits && __builtin_popcountll(local) < cb; ++b) local |= 1ull << b;
+    out->local[out->count++] = local;
+    nleft = keep;
+    std::copy(kept, kept + keep, left);
+  }
+  for (int i = 0; i < nleft; ++i) out->rest.id[out->rest.count++] = (uint8_t)left[i];
+}
+
+// Partial sums of up to kPauliLaunch terms over nsets states: rows (state, term)
+// of red_blocks(n / 2) values.  x: the terms' x masks on the host.
+template <typename T>
+static int launch_pauli_partials(const T *sv, uint64_t n, uint32_t nsets, int nterms,
+                                 const uint64_t *x, const PauliTerm *terms, double *partial,
+                                 hipStream_t st) {
+  if (nterms < 1 || nterms > kPauliLaunch)
+    return fail(SQ_ERR_INVALID, "internal: Pauli launch size");
+  constexpr int cb = PauliChunkLds<T>::CB;
+  const int nb = red_blocks(n / 2), nbits = log2u(n);
+  PauliGroups gr;
+  // Chunks from 2^20 complex64 amplitudes on (one state of 20 qubits, 64 terms:
+  // 128 workgroups take what the per-term kernel takes); the choice depends on n
+  // alone, so a batch gives the values of its states.
+  if (nbits >= (cb == 13 ? 20 : 19) && ((uintptr_t)sv & 15) == 0) {
+    const uint64_t nchunks = n >> cb;
+    const unsigned wg = (unsigned)std::min<uint64_t>(nchunks, nb);
+    pauli_groups(x, nterms, nbits, cb, cb == 13 ? 4 : 3, &gr);
+    for (int i = 0; i < gr.count; ++i) {
+      PassPlan p;
+      p.local = gr.local[i];
+      p.cb = cb;
+      hipLaunchKernelGGL(k_pauli_chunk<T>, dim3(wg, 1, nsets), dim3(kChunkThreads), 0, st, sv, n,
+                         nchunks, pass_geom(p), terms, gr.ids[i], nb, partial);
+    }
+  } else {
+    gr.rest.nterms = nterms;
+    for (int t = 0; t < nterms; ++t) gr.rest.id[gr.rest.count++] = (uint8_t)t;
+  }
+  if (gr.rest.count)
+    hipLaunchKernelGGL(k_partial_pauli<T>, dim3(nb, gr.rest.count, nsets), dim3(kBlock), 0, st, sv,
+                       n, terms, gr.rest, partial);
+  SQ_HIP(hipGetLastError());
+  return SQ_OK;
+}
+
+// terms_dev: PauliTerm[nterms] on the device, x their x masks on the host;
+// alpha_dev: per-term factors (2*i^ny folded in); out_dev[t] = term value.
+int launch_pauli_terms(const void *sv, sq_dtype_t dt, uint64_t n, int nterms, const uint64_t *x,
                        const void *terms_dev, const double *alpha_dev,
                        double *partial, double *out_dev, hipStream_t st) {
-  const int nb = red_blocks(n / 2);
+  const PauliTerm *terms = (const PauliTerm *)terms_dev;
   if (dt == SQ_COMPLEX64)
-    hipLaunchKernelGGL(k_partial_pauli<float2>, dim3(nb, nterms), dim3(kBlock), 0, st,
-                       (const float2 *)sv, n, (const PauliTerm *)terms_dev, partial);
+    SQ_TRY(launch_pauli_partials((const float2 *)sv, n, 1, nterms, x, terms, partial, st));
   else
-    hipLaunchKernelGGL(k_partial_pauli<double2>, dim3(nb, nterms), dim3(kBlock), 0, st,
-                       (const double2 *)sv, n, (const PauliTerm *)terms_dev, partial);
-  hipLaunchKernelGGL(k_finalize, dim3(nterms), dim3(kBlock), 0, st, partial, nb,
+    SQ_TRY(launch_pauli_partials((const double2 *)sv, n, 1, nterms, x, terms, partial, st));
+  hipLaunchKernelGGL(k_finalize, dim3(nterms), dim3(kBlock), 0, st, partial, red_blocks(n / 2),
                      alpha_dev, 0.0, out_dev);
   SQ_HIP(hipGetLastError());
   return SQ_OK;
@@ -1088,19 +1319,17 @@ size_t pauli_batch_partial_doubles(uint64_t n, uint32_t nsets, int nterms) {
 }
 
 int launch_pauli_terms_batch(const void *sv, sq_dtype_t dt, uint64_t n, uint32_t nsets,
-                             int nterms, const void *terms_dev, const double *alpha_dev,
-                             double *partial, double *out_dev, uint64_t out_stride,
-                             hipStream_t st) {
+                             int nterms, const uint64_t *x, const void *terms_dev,
+                             const double *alpha_dev, double *partial, double *out_dev,
+                             uint64_t out_stride, hipStream_t st) {
   if (nsets == 0 || nsets > 65535 || nterms < 1 || nterms > 65535)
     return fail(SQ_ERR_INVALID, "internal: batch expectation shape");
   const int nb = red_blocks(n / 2);
-  const dim3 grid(nb, nterms, nsets);
+  const PauliTerm *terms = (const PauliTerm *)terms_dev;
   if (dt == SQ_COMPLEX64)
-    hipLaunchKernelGGL(k_partial_pauli<float2>, grid, dim3(kBlock), 0, st,
-                       (const float2 *)sv, n, (const PauliTerm *)terms_dev, partial);
+    SQ_TRY(launch_pauli_partials((const float2 *)sv, n, nsets, nterms, x, terms, partial, st));
   else
-    hipLaunchKernelGGL(k_partial_pauli<double2>, grid, dim3(kBlock), 0, st,
-                       (const double2 *)sv, n, (const PauliTerm *)terms_dev, partial);
+    SQ_TRY(launch_pauli_partials((const double2 *)sv, n, nsets, nterms, x, terms, partial, st));
   hipLaunchKernelGGL(k_finalize_rows, dim3(nsets * nterms), dim3(kBlock), 0, st, partial, nb,
                      nterms, alpha_dev, out_dev, out_stride);
   SQ_HIP(hipGetLastError());

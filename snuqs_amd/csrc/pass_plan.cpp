@@ -3,7 +3,6 @@
 
 #include <algorithm>
 #include <array>
-#include <cmath>
 #include <cstring>
 
 namespace sq {
@@ -344,24 +343,26 @@ static void block_matrix(const PassBlockPlan &b, const PassGates &pg, BlockMatri
   }
 }
 
-// bf16 nearest to v, ties to even.  v is first cut to a float towards zero with a
-// sticky last bit, so that the second rounding sees which side of a tie v is on.
-static uint16_t to_bf16(double v) {
-  float f = (float)v;
-  uint32_t u;
-  std::memcpy(&u, &f, 4);
-  if ((double)f != v && f == f) {
-    if (std::fabs((double)f) > std::fabs(v)) --u;  // towards zero
-    u |= 1;
-  }
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);  // NaN
-  return (uint16_t)((u + 0x7fff + ((u >> 16) & 1)) >> 16);
-}
-static double from_bf16(uint16_t h) {
-  const uint32_t u = (uint32_t)h << 16;
-  float f;
-  std::memcpy(&f, &u, 4);
-  return f;
+// Three bf16 parts of each of the n values v, each part the nearest (ties to
+// even) to what the ones before leave: rounded in the double's own bits, which a
+// float then holds exactly.  v is used up.
+static void split_bf16(double *v, int n, uint16_t *p0, uint16_t *p1, uint16_t *p2) {
+  for (uint16_t *out : {p0, p1, p2})
+    for (int i = 0; i < n; ++i) {
+      uint64_t u;
+      std::memcpy(&u, v + i, 8);
+      u = (u + 0xfffffffffffull + ((u >> 45) & 1)) & ~0x1fffffffffffull;
+      double r;
+      std::memcpy(&r, &u, 8);
+      const float f = (float)(v[i] == v[i] ? r : v[i]);
+      uint32_t w;
+      std::memcpy(&w, &f, 4);
+      w &= 0xffff0000u;
+      float h;
+      std::memcpy(&h, &w, 4);
+      out[i] = (uint16_t)(w >> 16);
+      v[i] -= h;
+    }
 }
 
 void pass_image(const PassPlan &p, const std::vector<PassBlock> &blocks, sq_dtype_t dt,
@@ -378,24 +379,27 @@ void pass_image(const PassPlan &p, const std::vector<PassBlock> &blocks, sq_dtyp
       // matrices, 4 targets the real 32x32 form, each in three parts of two
       // fragments of 64 lanes x 8 columns
       uint16_t *f = (uint16_t *)dst;
-      for (int m = 0; m < (b.k == 5 ? 2 : 1); ++m)
-        for (int t = 0; t < 2; ++t)
-          for (int lane = 0; lane < 64; ++lane)
-            for (int j = 0; j < 8; ++j) {
-              const int row = lane & 31, c = 16 * t + 8 * (lane >> 5) + j;
-              double v;
-              if (b.k == 5) {
-                v = (m ? M.im : M.re)[row * d + c];
-              } else {
-                const int e = (row >> 1) * d + (c >> 1);
-                v = (row & 1) == (c & 1) ? M.re[e] : (row & 1) ? M.im[e] : -M.im[e];
-              }
-              for (int part = 0; part < 3; ++part) {
-                const uint16_t h = to_bf16(v);
-                f[(((3 * m + part) * 2 + t) * 64 + lane) * 8 + j] = h;
-                v -= from_bf16(h);
+      uint16_t re[3][1024], im[3][1024];
+      split_bf16(M.re, d * d, re[0], re[1], re[2]);
+      split_bf16(M.im, d * d, im[0], im[1], im[2]);
+      // column c = 16t + 8h + j of row r: fragment t, lane r + 32h, entry j
+      for (int p3 = 0; p3 < 3; ++p3)
+        for (int h8 = 0; h8 < 4; ++h8)
+          for (int row = 0; row < 32; ++row) {
+            const int at = (h8 >> 1) * 512 + (row + 32 * (h8 & 1)) * 8;
+            uint16_t *o = f + p3 * 1024 + at;
+            if (b.k == 5) {
+              std::memcpy(o, re[p3] + row * 32 + 8 * h8, 16);
+              std::memcpy(o + 3 * 1024, im[p3] + row * 32 + 8 * h8, 16);
+            } else {  // real form: row 2r + c', columns 2o, 2o + 1
+              const uint16_t *er = re[p3] + (row >> 1) * 16 + 4 * h8;
+              const uint16_t *ei = im[p3] + (row >> 1) * 16 + 4 * h8;
+              for (int q = 0; q < 4; ++q) {
+                o[2 * q] = (row & 1) ? ei[q] : er[q];
+                o[2 * q + 1] = (row & 1) ? er[q] : (uint16_t)(ei[q] ^ 0x8000u);
               }
             }
+          }
       continue;
     }
     double *f = (double *)dst;

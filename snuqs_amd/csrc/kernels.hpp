@@ -93,6 +93,22 @@ __device__ __forceinline__ void st_nt(uint4 *p, uint4 v) {
   __builtin_nontemporal_store(w, reinterpret_cast<nt_u4 *>(p));
 }
 
+// The same accesses, or ordinary ones (NT = false) for states that stay in the
+// caches between sweeps.
+template <bool NT>
+struct Mem {
+  template <typename T>
+  __device__ static __forceinline__ T ld(const T *p) {
+    if constexpr (NT) return ld_nt(p);
+    else return *p;
+  }
+  template <typename T>
+  __device__ static __forceinline__ void st(T *p, const T &v) {
+    if constexpr (NT) st_nt(p, v);
+    else *p = v;
+  }
+};
+
 // A 2x2 complex matrix in the state's precision, row-major; y = m x on the
 // amplitude pair (x0, x1) whose target bit is 0 / 1.
 template <typename R>

@@ -92,7 +92,7 @@ int launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream) {
 // ---------------------------------------------------------------------------
 // PHASE: multiply the amplitudes whose control bits match by one scalar.
 // ---------------------------------------------------------------------------
-template <typename R, int U>
+template <typename R, int U, bool NT>
 __device__ __forceinline__ void
     k_phase_body(typename CV<R>::T *__restrict__ sv, uint64_t nfree, IdxMap im,
             R pr, R pi) {
@@ -105,7 +105,7 @@ __device__ __forceinline__ void
     for (int u = 0; u < U; ++u) {
       uint64_t f = f0 + (uint64_t)u * kBlock;
       idx[u] = deposit(f, im);
-      if (f < nfree) v[u] = ld_nt(sv + idx[u]);
+      if (f < nfree) v[u] = Mem<NT>::ld(sv + idx[u]);
     }
   #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -113,16 +113,16 @@ __device__ __forceinline__ void
         T o;
         o.x = pr * v[u].x - pi * v[u].y;
         o.y = pr * v[u].y + pi * v[u].x;
-        st_nt(sv + idx[u], o);
+        Mem<NT>::st(sv + idx[u], o);
       }
     }
   }
 }
 
-template <typename R, int U>
+template <typename R, int U, bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_phase(typename CV<R>::T *__restrict__ sv, uint64_t nfree, IdxMap im, R pr, R pi) {
-  k_phase_body<R, U>(sv, nfree, im, pr, pi);
+  k_phase_body<R, U, NT>(sv, nfree, im, pr, pi);
 }
 // Batched forms (kb_*): one launch over a batch of states, blockIdx.y = the
 // state's index y in the batch; state y starts at sv + y * sstride and its
@@ -132,7 +132,7 @@ __global__ void __launch_bounds__(kBlock)
     kb_phase(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t nfree, IdxMap im,
              const typename CV<R>::T *__restrict__ tab) {
   const typename CV<R>::T ph = tab[blockIdx.y];
-  k_phase_body<R, U>(sv + blockIdx.y * sstride, nfree, im, ph.x, ph.y);
+  k_phase_body<R, U, true>(sv + blockIdx.y * sstride, nfree, im, ph.x, ph.y);
 }
 
 
@@ -149,7 +149,7 @@ struct DiagArgs {
 // A: DiagArgs by value (kernel argument) or a const reference into a batch's
 // per-state table (read in place: its entries are indexed at run time, and a
 // copy would sit in scratch).
-template <typename R, int U, typename A = DiagArgs<R>>
+template <typename R, int U, bool NT, typename A = DiagArgs<R>>
 __device__ __forceinline__ void
     k_diag_body(typename CV<R>::T *__restrict__ sv, uint64_t nfree, IdxMap im, A a) {
   using T = typename CV<R>::T;
@@ -167,7 +167,7 @@ __device__ __forceinline__ void
     for (int u = 0; u < U; ++u) {
       uint64_t f = f0 + (uint64_t)u * kBlock;
       idx[u] = deposit(f, im);
-      if (f < nfree) v[u] = ld_nt(sv + idx[u]);
+      if (f < nfree) v[u] = Mem<NT>::ld(sv + idx[u]);
     }
   #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -178,22 +178,22 @@ __device__ __forceinline__ void
         T o;
         o.x = pr * v[u].x - pi * v[u].y;
         o.y = pr * v[u].y + pi * v[u].x;
-        st_nt(sv + idx[u], o);
+        Mem<NT>::st(sv + idx[u], o);
       }
     }
   }
 }
 
-template <typename R, int U>
+template <typename R, int U, bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_diag(typename CV<R>::T *__restrict__ sv, uint64_t nfree, IdxMap im, DiagArgs<R> a) {
-  k_diag_body<R, U>(sv, nfree, im, a);
+  k_diag_body<R, U, NT>(sv, nfree, im, a);
 }
 template <typename R, int U>
 __global__ void __launch_bounds__(kBlock)
     kb_diag(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t nfree, IdxMap im,
             const DiagArgs<R> *__restrict__ tab) {
-  k_diag_body<R, U, const DiagArgs<R> &>(sv + blockIdx.y * sstride, nfree, im, tab[blockIdx.y]);
+  k_diag_body<R, U, true, const DiagArgs<R> &>(sv + blockIdx.y * sstride, nfree, im, tab[blockIdx.y]);
 }
 
 
@@ -208,7 +208,7 @@ struct PermArgs {
   int count;  // number of moved local indices (<= 8)
 };
 
-template <typename R, int U>
+template <typename R, int U, bool NT>
 __device__ __forceinline__ void
     k_perm_body(typename CV<R>::T *__restrict__ sv, uint64_t nfree, IdxMap im,
            PermArgs<R> a) {
@@ -224,7 +224,7 @@ __device__ __forceinline__ void
       if (f < nfree) {
   #pragma unroll
         for (int r = 0; r < 8; ++r)
-          if (r < a.count) v[u][r] = ld_nt(sv + base[u] + a.src[r]);
+          if (r < a.count) v[u][r] = Mem<NT>::ld(sv + base[u] + a.src[r]);
       }
     }
   #pragma unroll
@@ -236,7 +236,7 @@ __device__ __forceinline__ void
             T o;
             o.x = a.pr[r] * v[u][r].x - a.pi[r] * v[u][r].y;
             o.y = a.pr[r] * v[u][r].y + a.pi[r] * v[u][r].x;
-            st_nt(sv + base[u] + a.dst[r], o);
+            Mem<NT>::st(sv + base[u] + a.dst[r], o);
           }
         }
       }
@@ -244,16 +244,16 @@ __device__ __forceinline__ void
   }
 }
 
-template <typename R, int U>
+template <typename R, int U, bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_perm(typename CV<R>::T *__restrict__ sv, uint64_t nfree, IdxMap im, PermArgs<R> a) {
-  k_perm_body<R, U>(sv, nfree, im, a);
+  k_perm_body<R, U, NT>(sv, nfree, im, a);
 }
 template <typename R, int U>
 __global__ void __launch_bounds__(kBlock)
     kb_perm(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t nfree, IdxMap im,
             const PermArgs<R> *__restrict__ tab) {
-  k_perm_body<R, U>(sv + blockIdx.y * sstride, nfree, im, tab[blockIdx.y]);
+  k_perm_body<R, U, true>(sv + blockIdx.y * sstride, nfree, im, tab[blockIdx.y]);
 }
 
 
@@ -266,7 +266,7 @@ struct DenseArgs {
   uint64_t off[1 << K];
 };
 
-template <typename R, int K, int U>
+template <typename R, int K, int U, bool NT>
 __device__ __forceinline__ void
     k_dense_body(typename CV<R>::T *__restrict__ sv, uint64_t nfree, IdxMap im,
             DenseArgs<R, K> a) {
@@ -282,7 +282,7 @@ __device__ __forceinline__ void
       base[u] = deposit(f, im);
       if (f < nfree) {
   #pragma unroll
-        for (int c = 0; c < D; ++c) x[u][c] = ld_nt(sv + base[u] + a.off[c]);
+        for (int c = 0; c < D; ++c) x[u][c] = Mem<NT>::ld(sv + base[u] + a.off[c]);
       }
     }
   #pragma unroll
@@ -300,23 +300,23 @@ __device__ __forceinline__ void
           T o;
           o.x = yr;
           o.y = yi;
-          st_nt(sv + base[u] + a.off[r], o);
+          Mem<NT>::st(sv + base[u] + a.off[r], o);
         }
       }
     }
   }
 }
 
-template <typename R, int K, int U>
+template <typename R, int K, int U, bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_dense(typename CV<R>::T *__restrict__ sv, uint64_t nfree, IdxMap im, DenseArgs<R, K> a) {
-  k_dense_body<R, K, U>(sv, nfree, im, a);
+  k_dense_body<R, K, U, NT>(sv, nfree, im, a);
 }
 template <typename R, int K, int U>
 __global__ void __launch_bounds__(kBlock)
     kb_dense(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t nfree, IdxMap im,
              const DenseArgs<R, K> *__restrict__ tab) {
-  k_dense_body<R, K, U>(sv + blockIdx.y * sstride, nfree, im, tab[blockIdx.y]);
+  k_dense_body<R, K, U, true>(sv + blockIdx.y * sstride, nfree, im, tab[blockIdx.y]);
 }
 
 
@@ -1000,7 +1000,7 @@ __device__ __forceinline__ uint64_t small_tile_base(uint64_t t, const IdxMap &im
   return (deposit(t, im) << st.shift) | st.fval;
 }
 
-template <typename R, int TB>
+template <typename R, int TB, bool NT>
 __device__ __forceinline__ void small_tile_load(const typename CV<R>::T *sv, uint64_t base,
                                                 typename CV<R>::T *X, int lane,
                                                 const SmallTile &st) {
@@ -1017,7 +1017,7 @@ __device__ __forceinline__ void small_tile_load(const typename CV<R>::T *sv, uin
 #pragma unroll
       for (int b = 0; b < TB - 7; ++b)
         if ((k >> b) & 1) ka += st.a[7 + b];
-      const float4 v = ld_nt(reinterpret_cast<const float4 *>(sv + base + la + ka));
+      const float4 v = Mem<NT>::ld(reinterpret_cast<const float4 *>(sv + base + la + ka));
       *reinterpret_cast<float4 *>(X + 2 * (lane + 64 * k)) = v;
     }
   } else {
@@ -1032,13 +1032,13 @@ __device__ __forceinline__ void small_tile_load(const typename CV<R>::T *sv, uin
 #pragma unroll
       for (int b = 0; b < TB - 6; ++b)
         if ((k >> b) & 1) ka += st.a[6 + b];
-      const double2 v = ld_nt(sv + base + la + ka);
+      const double2 v = Mem<NT>::ld(sv + base + la + ka);
       X[lane + 64 * k] = make_double2(v.x, v.y);
     }
   }
 }
 
-template <typename R, int TB>
+template <typename R, int TB, bool NT>
 __device__ __forceinline__ void small_tile_store(typename CV<R>::T *sv, uint64_t base,
                                                  const typename CV<R>::T *X, int lane,
                                                  const SmallTile &st) {
@@ -1055,7 +1055,7 @@ __device__ __forceinline__ void small_tile_store(typename CV<R>::T *sv, uint64_t
       for (int b = 0; b < TB - 7; ++b)
         if ((k >> b) & 1) ka += st.a[7 + b];
       const float4 v = *reinterpret_cast<const float4 *>(X + 2 * (lane + 64 * k));
-      st_nt(reinterpret_cast<float4 *>(sv + base + la + ka), v);
+      Mem<NT>::st(reinterpret_cast<float4 *>(sv + base + la + ka), v);
     }
   } else {
     constexpr int CH = 1 << (TB - 6);
@@ -1070,7 +1070,7 @@ __device__ __forceinline__ void small_tile_store(typename CV<R>::T *sv, uint64_t
       for (int b = 0; b < TB - 6; ++b)
         if ((k >> b) & 1) ka += st.a[6 + b];
       const double2 v = X[lane + 64 * k];
-      st_nt(sv + base + la + ka, make_double2(v.x, v.y));
+      Mem<NT>::st(sv + base + la + ka, make_double2(v.x, v.y));
     }
   }
 }
@@ -1084,7 +1084,7 @@ __device__ __forceinline__ uint32_t small_group(int lane, const SmallTile &st) {
   return c;
 }
 
-template <typename R, int K>
+template <typename R, int K, bool NT>
 __device__ __forceinline__ void
     k_small_dense_body(typename CV<R>::T *__restrict__ sv, uint64_t ntiles, IdxMap im,
                   SmallTile st, DenseArgs<R, K> a) {
@@ -1097,7 +1097,7 @@ __device__ __forceinline__ void
   const uint32_t cb = small_group(lane, st);
   for (uint64_t t = tr.first; t < tr.end; t += tr.step) {
     const uint64_t base = small_tile_base(t, im, st);
-    small_tile_load<R, TB>(sv, base, X, lane, st);
+    small_tile_load<R, TB, NT>(sv, base, X, lane, st);
     wave_lds_sync();
     if (lane < st.nact) {
       T x[D];
@@ -1119,22 +1119,22 @@ __device__ __forceinline__ void
       }
     }
     wave_lds_sync();
-    small_tile_store<R, TB>(sv, base, X, lane, st);
+    small_tile_store<R, TB, NT>(sv, base, X, lane, st);
     wave_lds_sync();
   }
 }
 
-template <typename R, int K>
+template <typename R, int K, bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_small_dense(typename CV<R>::T *__restrict__ sv, uint64_t ntiles, IdxMap im, SmallTile st,
                   DenseArgs<R, K> a) {
-  k_small_dense_body<R, K>(sv, ntiles, im, st, a);
+  k_small_dense_body<R, K, NT>(sv, ntiles, im, st, a);
 }
 template <typename R, int K>
 __global__ void __launch_bounds__(kBlock)
     kb_small_dense(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t ntiles,
                    IdxMap im, SmallTile st, const DenseArgs<R, K> *__restrict__ tab) {
-  k_small_dense_body<R, K>(sv + blockIdx.y * sstride, ntiles, im, st, tab[blockIdx.y]);
+  k_small_dense_body<R, K, true>(sv + blockIdx.y * sstride, ntiles, im, st, tab[blockIdx.y]);
 }
 
 
@@ -1147,7 +1147,7 @@ struct SmallPermArgs {
   int count;
 };
 
-template <typename R, int K>
+template <typename R, int K, bool NT>
 __device__ __forceinline__ void
     k_small_perm_body(typename CV<R>::T *__restrict__ sv, uint64_t ntiles, IdxMap im,
                  SmallTile st, SmallPermArgs<R> a) {
@@ -1160,7 +1160,7 @@ __device__ __forceinline__ void
   const uint32_t cb = small_group(lane, st);
   for (uint64_t t = tr.first; t < tr.end; t += tr.step) {
     const uint64_t base = small_tile_base(t, im, st);
-    small_tile_load<R, TB>(sv, base, X, lane, st);
+    small_tile_load<R, TB, NT>(sv, base, X, lane, st);
     wave_lds_sync();
     if (lane < st.nact) {
       T v[D];
@@ -1178,22 +1178,22 @@ __device__ __forceinline__ void
       }
     }
     wave_lds_sync();
-    small_tile_store<R, TB>(sv, base, X, lane, st);
+    small_tile_store<R, TB, NT>(sv, base, X, lane, st);
     wave_lds_sync();
   }
 }
 
-template <typename R, int K>
+template <typename R, int K, bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_small_perm(typename CV<R>::T *__restrict__ sv, uint64_t ntiles, IdxMap im, SmallTile st,
                  SmallPermArgs<R> a) {
-  k_small_perm_body<R, K>(sv, ntiles, im, st, a);
+  k_small_perm_body<R, K, NT>(sv, ntiles, im, st, a);
 }
 template <typename R, int K>
 __global__ void __launch_bounds__(kBlock)
     kb_small_perm(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t ntiles,
                   IdxMap im, SmallTile st, const SmallPermArgs<R> *__restrict__ tab) {
-  k_small_perm_body<R, K>(sv + blockIdx.y * sstride, ntiles, im, st, tab[blockIdx.y]);
+  k_small_perm_body<R, K, true>(sv + blockIdx.y * sstride, ntiles, im, st, tab[blockIdx.y]);
 }
 
 
@@ -1418,7 +1418,7 @@ static DenseArgs<R, K> dense_args(const GatePlan &p) {
   return a;
 }
 
-template <typename R>
+template <typename R, bool NT>
 static int launch_plan_t(const GatePlan &p, typename CV<R>::T *sv,
                          uint64_t nelems, hipStream_t st, const R *gdev) {
   const int nfixed = __builtin_popcountll(p.fixed_mask);
@@ -1429,7 +1429,7 @@ static int launch_plan_t(const GatePlan &p, typename CV<R>::T *sv,
       constexpr int U = 4;
       const uint64_t nfree = nelems >> nfixed;
       IdxMap im = make_idxmap(p.fixed_mask, p.fixed_val);
-      hipLaunchKernelGGL((k_phase<R, U>), grid_for(nfree, kBlock * U),
+      hipLaunchKernelGGL((k_phase<R, U, NT>), grid_for(nfree, kBlock * U),
                          dim3(kBlock), 0, st, sv, nfree, im, (R)p.m[0].real(),
                          (R)p.m[0].imag());
       break;
@@ -1439,7 +1439,7 @@ static int launch_plan_t(const GatePlan &p, typename CV<R>::T *sv,
       const uint64_t nfree = nelems >> nfixed;
       IdxMap im = make_idxmap(p.fixed_mask, p.fixed_val);
       const DiagArgs<R> a = diag_args<R>(p);
-      hipLaunchKernelGGL((k_diag<R, U>), grid_for(nfree, kBlock * U),
+      hipLaunchKernelGGL((k_diag<R, U, NT>), grid_for(nfree, kBlock * U),
                          dim3(kBlock), 0, st, sv, nfree, im, a);
       break;
     }
@@ -1452,18 +1452,18 @@ static int launch_plan_t(const GatePlan &p, typename CV<R>::T *sv,
         const SmallPermArgs<R> a = small_perm_args<R>(p, stile);
         const dim3 grid = sweep_grid(ntiles, 4);
         if (p.kk == 1)
-          hipLaunchKernelGGL((k_small_perm<R, 1>), grid, dim3(kBlock), 0, st, sv, ntiles, sim, stile, a);
+          hipLaunchKernelGGL((k_small_perm<R, 1, NT>), grid, dim3(kBlock), 0, st, sv, ntiles, sim, stile, a);
         else if (p.kk == 2)
-          hipLaunchKernelGGL((k_small_perm<R, 2>), grid, dim3(kBlock), 0, st, sv, ntiles, sim, stile, a);
+          hipLaunchKernelGGL((k_small_perm<R, 2, NT>), grid, dim3(kBlock), 0, st, sv, ntiles, sim, stile, a);
         else
-          hipLaunchKernelGGL((k_small_perm<R, 3>), grid, dim3(kBlock), 0, st, sv, ntiles, sim, stile, a);
+          hipLaunchKernelGGL((k_small_perm<R, 3, NT>), grid, dim3(kBlock), 0, st, sv, ntiles, sim, stile, a);
         break;
       }
       constexpr int U = 2;
       const uint64_t nfree = nelems >> (nfixed + p.kk);
       IdxMap im = make_idxmap(p.fixed_mask | target_mask(p), p.fixed_val);
       const PermArgs<R> a = perm_args<R>(p);
-      hipLaunchKernelGGL((k_perm<R, U>), grid_for(nfree, kBlock * U),
+      hipLaunchKernelGGL((k_perm<R, U, NT>), grid_for(nfree, kBlock * U),
                          dim3(kBlock), 0, st, sv, nfree, im, a);
       break;
     }
@@ -1480,10 +1480,10 @@ static int launch_plan_t(const GatePlan &p, typename CV<R>::T *sv,
   case KV: {                                                                    \
     const DenseArgs<R, KV> a = dense_args<R, KV>(p);                            \
     if (small)                                                                  \
-      hipLaunchKernelGGL((k_small_dense<R, KV>), sweep_grid(ntiles, 4),         \
+      hipLaunchKernelGGL((k_small_dense<R, KV, NT>), sweep_grid(ntiles, 4),         \
                          dim3(kBlock), 0, st, sv, ntiles, sim, stile, a);       \
     else                                                                        \
-      hipLaunchKernelGGL((k_dense<R, KV, UV>), grid_sweep1(nfree),              \
+      hipLaunchKernelGGL((k_dense<R, KV, UV, NT>), grid_sweep1(nfree),              \
                          dim3(kBlock), 0, st, sv, nfree, im, a);                \
     break;                                                                      \
   }
@@ -1593,13 +1593,22 @@ uint64_t mfma_wave_tiles(uint64_t total_tiles) {
   return t;
 }
 
+// Ordinary instead of non-temporal accesses where the state stays in the 256 MiB
+// Infinity Cache from one gate to the next (28 and more one-gate calls on one
+// state, us): 16 MiB complex128 207 against 200 non-temporal, 32 MiB complex64
+// 328 / 354, 64 MiB 519 / 650, 128 MiB 1044 / 1260, 256 MiB complex128 1863 /
+// 2351, 512 MiB complex64 4330 / 4652, 1 GiB complex128 11878 / 11569.
+static bool sweep_cached(uint64_t bytes) { return bytes >= 32ull << 20 && bytes <= 512ull << 20; }
+
 int launch_plan(const GatePlan &p, void *sv, sq_dtype_t dt, uint64_t nelems,
                 hipStream_t stream, const void *dev_matrix) {
-  if (dt == SQ_COMPLEX64)
-    return launch_plan_t<float>(p, (float2 *)sv, nelems, stream,
-                                (const float *)dev_matrix);
-  return launch_plan_t<double>(p, (double2 *)sv, nelems, stream,
-                               (const double *)dev_matrix);
+  const bool cached = sweep_cached(nelems * itemsize(dt));
+  if (dt == SQ_COMPLEX64) {
+    const auto launch = cached ? launch_plan_t<float, false> : launch_plan_t<float, true>;
+    return launch(p, (float2 *)sv, nelems, stream, (const float *)dev_matrix);
+  }
+  const auto launch = cached ? launch_plan_t<double, false> : launch_plan_t<double, true>;
+  return launch(p, (double2 *)sv, nelems, stream, (const double *)dev_matrix);
 }
 
 // ---------------------------------------------------------------------------

@@ -299,7 +299,7 @@ __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, u
                                            const PassGeom &geom,
                                            const PassBlock *__restrict__ blocks, int nblocks,
                                            const nt_f4 *__restrict__ G, bool initial,
-                                           PassLds<R, CB> &lds) {
+                                           bool cached, PassLds<R, CB> &lds) {
   using S = PassShape<R, CB>;
   constexpr bool c64 = sizeof(R) == 4;
   constexpr int NT = S::NT, NW = S::NW, NL = S::NL;
@@ -370,6 +370,9 @@ __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, u
         __builtin_memcpy(&v[0], &one, 16);
       }
     }
+  } else if (cached) {
+#pragma unroll
+    for (int k = 0; k < NL; ++k) v[k] = *reinterpret_cast<const nt_f4 *>(p + ka(k));
   } else {
 #pragma unroll
     for (int k = 0; k < NL; ++k)
@@ -416,7 +419,8 @@ __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, u
     } else {
       o = *reinterpret_cast<const nt_f4 *>(X + (tw ^ kw(k)));
     }
-    __builtin_nontemporal_store(o, reinterpret_cast<nt_f4 *>(p + ka(k)));
+    if (cached) *reinterpret_cast<nt_f4 *>(p + ka(k)) = o;
+    else __builtin_nontemporal_store(o, reinterpret_cast<nt_f4 *>(p + ka(k)));
   }
 }
 
@@ -428,12 +432,13 @@ template <typename R, int CB>
 __global__ void SQ_PASS_BOUNDS
     k_pass(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t nchunks, PassGeom geom,
            const PassBlock *__restrict__ blocks, int nblocks, const char *__restrict__ image,
-           uint64_t gstride) {
+           uint64_t gstride, int cached) {
   __shared__ PassLds<R, CB> lds;
   const nt_f4 *G = reinterpret_cast<const nt_f4 *>(image + blockIdx.y * gstride);
   const uint64_t c = (uint64_t)blockIdx.z * gridDim.x + blockIdx.x;
   if (c < nchunks)
-    pass_chunk<R, CB>(sv + blockIdx.y * sstride, c, geom, blocks, nblocks, G, false, lds);
+    pass_chunk<R, CB>(sv + blockIdx.y * sstride, c, geom, blocks, nblocks, G, false,
+                      cached != 0, lds);
 }
 
 // Circuit batches: workgroup w takes chunk w - first of its entry.
@@ -441,11 +446,21 @@ template <typename R, int CB>
 __global__ void SQ_PASS_BOUNDS
     k_pass_entries(typename CV<R>::T *__restrict__ states, const PassEntry *__restrict__ entries,
                    const uint32_t *__restrict__ entry, const PassBlock *__restrict__ blocks,
-                   const char *__restrict__ images) {
+                   const char *__restrict__ images, int cached) {
   __shared__ PassLds<R, CB> lds;
   const PassEntry &e = entries[__builtin_amdgcn_readfirstlane(entry[blockIdx.x])];
   pass_chunk<R, CB>(states + e.psi, blockIdx.x - e.first, e.geom, blocks + e.blocks, e.nblocks,
-                    reinterpret_cast<const nt_f4 *>(images + e.image), e.initial != 0, lds);
+                    reinterpret_cast<const nt_f4 *>(images + e.image), e.initial != 0, cached != 0,
+                    lds);
+}
+
+// Ordinary instead of non-temporal accesses: states of up to 1 MiB (the L2s:
+// 16 qubits complex64 70.7 against 74.5 us a circuit) and of 64-256 MiB (the
+// Infinity Cache: 23, 24 and 25 qubits complex64 452 / 460, 839 / 880 and 1590 /
+// 1712 us); between them and above they are slower (8 MiB 122 / 120, 16 MiB
+// complex128 235 / 184, 32 MiB 268 / 262, 512 MiB 4925 / 4880).
+static bool pass_cached(uint64_t bytes) {
+  return bytes <= 1ull << 20 || (bytes >= 64ull << 20 && bytes <= 256ull << 20);
 }
 
 template <typename R, int CB>
@@ -456,7 +471,7 @@ static void launch_pass_cb(const PassGeom &geom, void *sv, uint64_t nelems, uint
   const uint64_t g = std::min<uint64_t>(nchunks, kPassGrid);
   hipLaunchKernelGGL((k_pass<R, CB>), dim3((unsigned)g, nsets, (unsigned)((nchunks + g - 1) / g)), dim3(PassShape<R, CB>::NT), 0, st,
                      (typename CV<R>::T *)sv, nelems, nchunks, geom, blocks, nblocks,
-                     (const char *)image, gstride);
+                     (const char *)image, gstride, (int)pass_cached(nelems * nsets * sizeof(typename CV<R>::T)));
 }
 
 // SQ_PASS(R, CB) for the dtype and chunk size.
@@ -479,7 +494,7 @@ int launch_pass_entries(int cb, sq_dtype_t dt, void *states, const PassEntry *en
 #define SQ_PASS(R, CB)                                                                        \
   hipLaunchKernelGGL((k_pass_entries<R, CB>), dim3((unsigned)nwg), dim3(PassShape<R, CB>::NT), \
                      0, st, (typename CV<R>::T *)states, entries, entry, blocks,              \
-                     (const char *)images)
+                     (const char *)images, (int)pass_cached((nwg << cb) * itemsize(dt)))
   SQ_PASS_SWITCH(cb)
 #undef SQ_PASS
   SQ_HIP(hipGetLastError());

@@ -293,13 +293,13 @@ struct PassLds {
 };
 
 // The pass on chunk c of a state: by every thread of the workgroup.  initial:
-// the state is |0...0> and is not read.
-template <typename R, int CB>
+// the state is |0...0> and is not read.  STREAM: non-temporal accesses.
+template <typename R, int CB, bool STREAM>
 __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, uint64_t c,
                                            const PassGeom &geom,
                                            const PassBlock *__restrict__ blocks, int nblocks,
                                            const nt_f4 *__restrict__ G, bool initial,
-                                           bool cached, PassLds<R, CB> &lds) {
+                                           PassLds<R, CB> &lds) {
   using S = PassShape<R, CB>;
   constexpr bool c64 = sizeof(R) == 4;
   constexpr int NT = S::NT, NW = S::NW, NL = S::NL;
@@ -370,13 +370,13 @@ __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, u
         __builtin_memcpy(&v[0], &one, 16);
       }
     }
-  } else if (cached) {
-#pragma unroll
-    for (int k = 0; k < NL; ++k) v[k] = *reinterpret_cast<const nt_f4 *>(p + ka(k));
   } else {
 #pragma unroll
-    for (int k = 0; k < NL; ++k)
-      v[k] = __builtin_nontemporal_load(reinterpret_cast<const nt_f4 *>(p + ka(k)));
+    for (int k = 0; k < NL; ++k) {
+      const nt_f4 *q = reinterpret_cast<const nt_f4 *>(p + ka(k));
+      if constexpr (STREAM) v[k] = __builtin_nontemporal_load(q);
+      else v[k] = *q;
+    }
   }
   nt_f4 pre[NP];
   fetch(pre, blocks);
@@ -419,8 +419,9 @@ __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, u
     } else {
       o = *reinterpret_cast<const nt_f4 *>(X + (tw ^ kw(k)));
     }
-    if (cached) *reinterpret_cast<nt_f4 *>(p + ka(k)) = o;
-    else __builtin_nontemporal_store(o, reinterpret_cast<nt_f4 *>(p + ka(k)));
+    nt_f4 *q = reinterpret_cast<nt_f4 *>(p + ka(k));
+    if constexpr (STREAM) __builtin_nontemporal_store(o, q);
+    else *q = o;
   }
 }
 
@@ -428,37 +429,37 @@ __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, u
   __launch_bounds__((PassShape<R, CB>::NT), \
                     (PassShape<R, CB>::NW == 8 ? 4 : PassShape<R, CB>::NW == 4 ? 3 : 2))
 
-template <typename R, int CB>
+template <typename R, int CB, bool STREAM>
 __global__ void SQ_PASS_BOUNDS
     k_pass(typename CV<R>::T *__restrict__ sv, uint64_t sstride, uint64_t nchunks, PassGeom geom,
            const PassBlock *__restrict__ blocks, int nblocks, const char *__restrict__ image,
-           uint64_t gstride, int cached) {
+           uint64_t gstride) {
   __shared__ PassLds<R, CB> lds;
   const nt_f4 *G = reinterpret_cast<const nt_f4 *>(image + blockIdx.y * gstride);
   const uint64_t c = (uint64_t)blockIdx.z * gridDim.x + blockIdx.x;
   if (c < nchunks)
-    pass_chunk<R, CB>(sv + blockIdx.y * sstride, c, geom, blocks, nblocks, G, false,
-                      cached != 0, lds);
+    pass_chunk<R, CB, STREAM>(sv + blockIdx.y * sstride, c, geom, blocks, nblocks, G, false, lds);
 }
 
 // Circuit batches: workgroup w takes chunk w - first of its entry.
-template <typename R, int CB>
+template <typename R, int CB, bool STREAM>
 __global__ void SQ_PASS_BOUNDS
     k_pass_entries(typename CV<R>::T *__restrict__ states, const PassEntry *__restrict__ entries,
                    const uint32_t *__restrict__ entry, const PassBlock *__restrict__ blocks,
-                   const char *__restrict__ images, int cached) {
+                   const char *__restrict__ images) {
   __shared__ PassLds<R, CB> lds;
   const PassEntry &e = entries[__builtin_amdgcn_readfirstlane(entry[blockIdx.x])];
-  pass_chunk<R, CB>(states + e.psi, blockIdx.x - e.first, e.geom, blocks + e.blocks, e.nblocks,
-                    reinterpret_cast<const nt_f4 *>(images + e.image), e.initial != 0, cached != 0,
-                    lds);
+  pass_chunk<R, CB, STREAM>(states + e.psi, blockIdx.x - e.first, e.geom, blocks + e.blocks, e.nblocks,
+                        reinterpret_cast<const nt_f4 *>(images + e.image), e.initial != 0, lds);
 }
 
 // Ordinary instead of non-temporal accesses: states of up to 1 MiB (the L2s:
-// 16 qubits complex64 70.7 against 74.5 us a circuit) and of 64-256 MiB (the
-// Infinity Cache: 23, 24 and 25 qubits complex64 452 / 460, 839 / 880 and 1590 /
-// 1712 us); between them and above they are slower (8 MiB 122 / 120, 16 MiB
-// complex128 235 / 184, 32 MiB 268 / 262, 512 MiB 4925 / 4880).
+// 16 qubits complex64 70.8 against 74.3 us a circuit) and of 64-256 MiB (the
+// Infinity Cache: 23, 24 and 25 qubits complex64 426 / 427, 809 / 850 and 1597 /
+// 1695 us); between them and above they are slower (8 MiB 122 / 120, 16 MiB
+// 174 / 158 and complex128 235 / 184, 32 MiB 268 / 262, 512 MiB 4925 / 4880).
+// The choice is a template argument: the compiler merges accesses that differ
+// in this hint alone.
 static bool pass_cached(uint64_t bytes) {
   return bytes <= 1ull << 20 || (bytes >= 64ull << 20 && bytes <= 256ull << 20);
 }
@@ -469,9 +470,11 @@ static void launch_pass_cb(const PassGeom &geom, void *sv, uint64_t nelems, uint
                            uint64_t gstride, hipStream_t st) {
   const uint64_t nchunks = nelems >> CB;
   const uint64_t g = std::min<uint64_t>(nchunks, kPassGrid);
-  hipLaunchKernelGGL((k_pass<R, CB>), dim3((unsigned)g, nsets, (unsigned)((nchunks + g - 1) / g)), dim3(PassShape<R, CB>::NT), 0, st,
+  const auto k = pass_cached(nelems * nsets * sizeof(typename CV<R>::T)) ? k_pass<R, CB, false>
+                                                                         : k_pass<R, CB, true>;
+  hipLaunchKernelGGL(k, dim3((unsigned)g, nsets, (unsigned)((nchunks + g - 1) / g)), dim3(PassShape<R, CB>::NT), 0, st,
                      (typename CV<R>::T *)sv, nelems, nchunks, geom, blocks, nblocks,
-                     (const char *)image, gstride, (int)pass_cached(nelems * nsets * sizeof(typename CV<R>::T)));
+                     (const char *)image, gstride);
 }
 
 // SQ_PASS(R, CB) for the dtype and chunk size.
@@ -491,10 +494,11 @@ static void launch_pass_cb(const PassGeom &geom, void *sv, uint64_t nelems, uint
 int launch_pass_entries(int cb, sq_dtype_t dt, void *states, const PassEntry *entries,
                         const uint32_t *entry, const PassBlock *blocks, const void *images,
                         uint64_t nwg, hipStream_t st) {
-#define SQ_PASS(R, CB)                                                                        \
-  hipLaunchKernelGGL((k_pass_entries<R, CB>), dim3((unsigned)nwg), dim3(PassShape<R, CB>::NT), \
-                     0, st, (typename CV<R>::T *)states, entries, entry, blocks,              \
-                     (const char *)images, (int)pass_cached((nwg << cb) * itemsize(dt)))
+  const bool cached = pass_cached((nwg << cb) * itemsize(dt));
+#define SQ_PASS(R, CB)                                                                          \
+  hipLaunchKernelGGL((cached ? k_pass_entries<R, CB, false> : k_pass_entries<R, CB, true>),     \
+                     dim3((unsigned)nwg), dim3(PassShape<R, CB>::NT), 0, st,                    \
+                     (typename CV<R>::T *)states, entries, entry, blocks, (const char *)images)
   SQ_PASS_SWITCH(cb)
 #undef SQ_PASS
   SQ_HIP(hipGetLastError());

@@ -93,3 +93,34 @@ def test_unaligned_complex64_state(C):
     got = out[1:1 + (1 << n)].astype(np.complex128)
     assert np.abs(got - run_oracle(n, ops, init.astype(np.complex128))).max() <= TOL["complex64"]
     assert out[0] == 0 and not out[1 + (1 << n):].any()  # nothing beside the state
+
+
+# 64 MiB: the smallest state above 1 MiB that passes read with ordinary accesses
+@pytest.mark.parametrize("dtype,n", [("complex128", 22), ("complex64", 23)])
+def test_passes_with_ordinary_accesses(C, dtype, n):
+    rng = np.random.default_rng(n)
+    ops = _circuit(n, rng, 12)
+    init = random_state(n, rng, np.complex64 if dtype == "complex64" else np.complex128)
+    sv = device_state(C, n, dtype, init)
+    C.functionals.Program(n, ops, dtype=dtype).run(sv)
+    assert np.abs(to_np(C, sv) - run_oracle(n, ops, init.astype(np.complex128))).max() <= TOL[dtype]
+
+
+# 32 MiB: the smallest state that single gates read with ordinary accesses; a
+# diagonal, a swap, dense gates of 1 to 5 targets, low, high and mixed bits
+@pytest.mark.parametrize("dtype,n", [("complex128", 21), ("complex64", 22)])
+def test_gates_with_ordinary_accesses(C, dtype, n):
+    from snuqs_amd.circuits import haar_unitary
+    from snuqs_amd._C.operation import gate_operations as g
+
+    rng = np.random.default_rng(n)
+    ops = [g.Hadamard([0]), g.Hadamard([n - 1]), g.RotZ([3], 0.4), g.CX([1, n - 2]),
+           g.Swap([0, n - 1]), g.CCNot([2, n // 2, n - 1])]
+    for k in (2, 3, 4, 5):
+        for t in (list(range(k)), list(range(n - k, n)), [int(q) for q in rng.permutation(n)[:k]]):
+            ops.append(g.Unitary(t, haar_unitary(1 << k, rng)))
+    init = random_state(n, rng, np.complex64 if dtype == "complex64" else np.complex128)
+    sv = device_state(C, n, dtype, init)
+    for op in ops:
+        C.functionals.apply(sv, op, n, op.targets)
+    assert np.abs(to_np(C, sv) - run_oracle(n, ops, init.astype(np.complex128))).max() <= TOL[dtype]

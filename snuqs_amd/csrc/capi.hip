@@ -1185,7 +1185,6 @@ static int sample_from(const double *probs, const void *sv, sq_dtype_t dt, int n
   int dev;
   SQ_TRY(current_device(&dev));
   std::lock_guard<std::mutex> lk(g_ws_mutex[dev]);
-  const size_t cdf_b = n * sizeof(double) + 256;
   const size_t io_b = shots * 16 + 512;
   const size_t red_b = (kRedBlocks + 64) * sizeof(double) + 256;
   hipStream_t st = (hipStream_t)stream;
@@ -1195,6 +1194,7 @@ static int sample_from(const double *probs, const void *sv, sq_dtype_t dt, int n
   for (int route = exact ? 0 : 1; route < 2; ++route) {
     const size_t scr_b =
         (route ? sample_scratch_bytes(n, exact != 0) : sample_exact_scratch_bytes(n)) + 256;
+    const size_t cdf_b = route ? n * sizeof(double) + 256 : 0;
     const size_t prob_b = route && sv ? n * sizeof(double) + 256 : 0;
     SQ_TRY(ws_reserve(dev, cdf_b + scr_b + red_b + prob_b + io_b + 1024, io_b, &w));
     char *d = (char *)w->dev;
@@ -1211,10 +1211,10 @@ static int sample_from(const double *probs, const void *sv, sq_dtype_t dt, int n
     if (route == 0) {
       const int *bad_dev;
       if (sv)
-        SQ_TRY(sample_exact_state(sv, dt, normalize ? red : nullptr, n, cdf, du, shots, dout, scr,
+        SQ_TRY(sample_exact_state(sv, dt, normalize ? red : nullptr, n, du, shots, dout, scr,
                                   &bad_dev, st));
       else
-        SQ_TRY(sample_exact(probs, n, cdf, du, shots, dout, scr, &bad_dev, st));
+        SQ_TRY(sample_exact(probs, n, du, shots, dout, scr, &bad_dev, st));
       SQ_HIP(hipMemcpyAsync(&bad, bad_dev, sizeof(int), hipMemcpyDeviceToHost, st));
     } else {
       if (sv && normalize) SQ_TRY(launch_probabilities_div(sv, dt, n, pr, red, st));

@@ -153,15 +153,15 @@ void fill_pauli_apply_terms(int nterms, const uint64_t *x, const uint64_t *z,
 int sample_cdf(const double *p, uint64_t n, double *cdf, bool exact,
                void *scratch, size_t scratch_bytes, hipStream_t st);
 // Exact samples: out_dev[s] = the first index whose cdf is above u_dev[s]
-// (numpy's choice), the cdf being written where it is needed.  *bad_dev (device)
+// (numpy's choice); scratch: sample_exact_scratch_bytes(n).  *bad_dev (device)
 // is nonzero when p holds negative or non-finite entries; nothing else is
 // written then.
-int sample_exact(const double *p, uint64_t n, double *cdf, const double *u_dev, uint64_t shots,
+int sample_exact(const double *p, uint64_t n, const double *u_dev, uint64_t shots,
                  int64_t *out_dev, void *scratch, const int **bad_dev, hipStream_t st);
 // The same from a state: the probabilities are |a|^2 (/ *norm2_dev unless it is
 // null), formed in FP64 where they are used.
 int sample_exact_state(const void *sv, sq_dtype_t dt, const double *norm2_dev, uint64_t n,
-                       double *cdf, const double *u_dev, uint64_t shots, int64_t *out_dev,
+                       const double *u_dev, uint64_t shots, int64_t *out_dev,
                        void *scratch, const int **bad_dev, hipStream_t st);
 size_t sample_exact_scratch_bytes(uint64_t n);
 size_t sample_scratch_bytes(uint64_t n, bool exact);

@@ -22,10 +22,12 @@
 // tile, that tile's elements are gone through (the crossing element is added
 // with one ordinary double add).  That gives the exact c at every tile's
 // start; a last pass writes the cdf inside the tiles that some uniform falls
-// into.  Nothing waits for the host.  The state is read four times (norm, sums,
-// maps, cdf) and the cdf written once: 2.7 GB at 2^26 complex64 amplitudes,
-// 0.4 ms at copy rate; measured 1.1 ms (norm 0.12, sums 0.09, maps 0.13, chain
-// 0.28, a serial chain of some 70 scans, cdf 0.24, search 0.03), 20 ms with an
+// into, the last entry of every 16, and a sample adds up the elements of its
+// 16.  Nothing waits for the host.  The state is read four times (norm, sums,
+// maps, cdf): 2.1 GB at 2^26 complex64 amplitudes, 0.34 ms at copy rate;
+// measured 0.98 ms (norm 0.1, sums 0.09, maps 0.13, chain 0.28, a serial chain of
+// some 70 scans, cdf 0.16 + 0.06, search 0.02; with the whole cdf written 1.10 ms,
+// cdf 0.24 of it), 20 ms with an
 // epoch of launches and host reads per binade.  Inputs that are not finite and
 // non-negative take the older route, an epoch of launches per binade driven by
 // the host.
@@ -273,6 +275,13 @@ int launch_search(const double *cdf, uint64_t n, const double *u_dev, uint64_t s
 constexpr int kTileThreads = 1024;
 constexpr int kTileItems = 4;
 constexpr int kTile = kTileThreads * kTileItems;
+// Of a tile's cdf the last entry of every kGroup elements is kept.
+constexpr int kGroup = 16;
+constexpr int kTileGroups = kTile / kGroup;
+constexpr int kGroupThreads = kGroup / kTileItems;
+__device__ __forceinline__ bool group_end(int i, int cnt) {
+  return (i & (kGroup - 1)) == kGroup - 1 || i == cnt - 1;
+}
 constexpr double kTop = 9007199254740992.0;  // 2^53: C has left the binade
 
 // What a tile does to C (integers held as doubles: exact below 2^53, and sums
@@ -399,7 +408,7 @@ __device__ __forceinline__ int block_min(int v) {
 }
 
 // The recurrence over one tile's elements (thread t holds items 4t .. 4t + 3,
-// cnt in all) from c; writes the cdf to out unless it is null and returns c
+// cnt in all) from c; writes the groups' last cdf entries to out and returns c
 // after the tile.  Every round of the loop ends the tile or passes one
 // element that starts a binade.
 __device__ __forceinline__ double walk_tile(const double (&x)[kTileItems], int cnt, double c,
@@ -454,11 +463,10 @@ __device__ __forceinline__ double walk_tile(const double (&x)[kTileItems], int c
         first = block_min(f);
       }
     }
-    if (out) {
 #pragma unroll
-      for (int j = 0; j < kTileItems; ++j)
-        if (i0 + j >= s && i0 + j < cnt && i0 + j < first) out[i0 + j] = down(v[j]);
-    }
+    for (int j = 0; j < kTileItems; ++j)
+      if (i0 + j >= s && i0 + j < first && group_end(i0 + j, cnt) && i0 + j < cnt)
+        out[(i0 + j) / kGroup] = down(v[j]);
     const bool last = first >= cnt;  // stays in the binade to the tile's end
     if (last ? (int)threadIdx.x == (cnt - 1) / kTileItems : f == first) {
       double l = start, px = 0.0;  // C before (after, at the end) the element
@@ -472,7 +480,7 @@ __device__ __forceinline__ double walk_tile(const double (&x)[kTileItems], int c
         }
       }
       sc = down(l) + px;
-      if (out && !last) out[first] = sc;
+      if (!last && group_end(first, cnt)) out[first / kGroup] = sc;
     }
     __syncthreads();
     c = sc;
@@ -652,11 +660,11 @@ __global__ void __launch_bounds__(kTileThreads)
 }
 
 // One workgroup: the exact c before every tile, tile_in[t], and after the
-// last, tile_in[nt]; the cdf of the tiles it goes through.
+// last, tile_in[nt]; the group ends of the tiles it goes through.
 template <typename S>
 __global__ void __launch_bounds__(kTileThreads)
     k_tile_chain(S src, uint64_t n, uint64_t nt, const TileMap *__restrict__ maps,
-                 double *__restrict__ tile_in, double *__restrict__ cdf, int *bad) {
+                 double *__restrict__ tile_in, double *__restrict__ ends, int *bad) {
   if (*bad) return;
   __shared__ double sc;
   const int tid = threadIdx.x;
@@ -701,7 +709,7 @@ __global__ void __launch_bounds__(kTileThreads)
       c = sc;
       double x[kTileItems];
       const int cnt = load_tile(src, n, t0 + f, x);
-      c = walk_tile(x, cnt, c, cdf + (t0 + f) * kTile);
+      c = walk_tile(x, cnt, c, ends + (t0 + f) * kTileGroups);
       s = f + 1;
     }
   }
@@ -732,7 +740,7 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// How a needed tile gets its cdf: by one plain scan, by a scan with ties, or not
+// How a needed tile gets its group ends: by one plain scan, by a scan with ties, or not
 // here (c leaves its binade there: k_tile_chain has written it).
 enum class TileCdf { kDone, kPlain, kTied };
 __device__ __forceinline__ TileCdf tile_cdf(const double *tile_in, const TileMap *maps, uint64_t t) {
@@ -742,20 +750,21 @@ __device__ __forceinline__ TileCdf tile_cdf(const double *tile_in, const TileMap
   return maps[t].flags & kTies ? TileCdf::kTied : TileCdf::kPlain;
 }
 
-// The cdf of the needed tiles, written where k_tile_search looks: the plain
-// ones (few registers, so two workgroups share a CU) and the others.
+// The group ends of the needed tiles: the plain ones (few registers, so two
+// workgroups share a CU) and the others.  Bound by the read of the state; the
+// whole cdf, 8 bytes an element, was as much to write as complex64 is to read.
 template <typename S>
 __global__ void __launch_bounds__(kTileThreads, 8)
     k_tile_cdf(S src, uint64_t n, const double *__restrict__ tile_in,
                const TileMap *__restrict__ maps, const int *__restrict__ need,
-               double *__restrict__ cdf, const int *__restrict__ bad) {
+               double *__restrict__ ends, const int *__restrict__ bad) {
   constexpr int W = kTileThreads / 64;
   __shared__ double w[W];
   if (*bad || !need[blockIdx.x] || tile_cdf(tile_in, maps, blockIdx.x) != TileCdf::kPlain)
     return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double x[kTileItems];
-  const int cnt = load_tile(src, n, blockIdx.x, x);
+  load_tile(src, n, blockIdx.x, x);
   const double c = tile_in[blockIdx.x];
   const int e = binade(c);
   const Scale up(52 - e), down(e - 52);
@@ -777,52 +786,72 @@ __global__ void __launch_bounds__(kTileThreads, 8)
 #pragma unroll
   for (int v = 0; v < W; ++v)
     if (v < wave) start += w[v];
-  double *out = cdf + (uint64_t)blockIdx.x * kTile + threadIdx.x * kTileItems;
-#pragma unroll
-  for (int j = 0; j < kTileItems; ++j) x[j] = down(start + x[j]);
-  if (cnt == kTile) {
-    *reinterpret_cast<double2 *>(out) = make_double2(x[0], x[1]);
-    *reinterpret_cast<double2 *>(out + 2) = make_double2(x[2], x[3]);
-  } else {
-#pragma unroll
-    for (int j = 0; j < kTileItems; ++j)
-      if ((int)threadIdx.x * kTileItems + j < cnt) out[j] = x[j];
-  }
+  // (elements past the state's end add nothing)
+  if (threadIdx.x % kGroupThreads == kGroupThreads - 1)
+    ends[(uint64_t)blockIdx.x * kTileGroups + threadIdx.x / kGroupThreads] =
+        down(start + x[kTileItems - 1]);
 }
 
 template <typename S>
 __global__ void __launch_bounds__(kTileThreads)
     k_tile_cdf_walk(S src, uint64_t n, uint64_t nt, const double *__restrict__ tile_in,
                     const TileMap *__restrict__ maps, const int *__restrict__ need,
-                    double *__restrict__ cdf, const int *__restrict__ bad) {
+                    double *__restrict__ ends, const int *__restrict__ bad) {
   if (*bad) return;
   for (uint64_t t = blockIdx.x; t < nt; t += gridDim.x) {
     if (!need[t] || tile_cdf(tile_in, maps, t) != TileCdf::kTied) continue;
     double x[kTileItems];
     const int cnt = load_tile(src, n, t, x);
-    walk_tile(x, cnt, tile_in[t], cdf + t * kTile);
+    walk_tile(x, cnt, tile_in[t], ends + t * kTileGroups);
   }
 }
 
-// out[s]: the uniform's tile on entry, its element on return.
+// out[s]: the uniform's tile on entry, its element on return: the first group
+// whose end is above the uniform, then the recurrence itself over its elements.
+template <typename S>
 __global__ void __launch_bounds__(kBlock)
-    k_tile_search(const double *__restrict__ cdf, uint64_t n, const double *__restrict__ tile_in,
-                  uint64_t nt, const double *__restrict__ u, uint64_t shots,
-                  int64_t *__restrict__ out, const int *__restrict__ bad) {
+    k_tile_search(S src, const double *__restrict__ ends, uint64_t n,
+                  const double *__restrict__ tile_in, uint64_t nt, const double *__restrict__ u,
+                  uint64_t shots, int64_t *__restrict__ out, const int *__restrict__ bad) {
   if (*bad) return;
   const double total = tile_in[nt];
   for (uint64_t s = (uint64_t)blockIdx.x * kBlock + threadIdx.x; s < shots;
        s += (uint64_t)gridDim.x * kBlock) {
     const uint64_t tile = (uint64_t)out[s];
-    uint64_t lo = tile * kTile, hi = lo + kTile;
-    if (tile >= nt) lo = n;
-    if (hi > n) hi = n;
-    const double v = u[s];
-    while (lo < hi) {
-      const uint64_t mid = lo + ((hi - lo) >> 1);
-      if (cdf[mid] / total <= v) lo = mid + 1; else hi = mid;
+    uint64_t i = n;
+    if (tile < nt) {
+      const double v = u[s];
+      const uint64_t left = n - tile * kTile;
+      const int ngroups = left < kTile ? ((int)left + kGroup - 1) / kGroup : kTileGroups;
+      const double *end = ends + tile * kTileGroups;
+      int lo = 0, hi = ngroups - 1;  // the tile's end is above v
+      while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (end[mid] / total <= v) lo = mid + 1; else hi = mid;
+      }
+      double c = lo ? end[lo - 1] : tile_in[tile];
+      i = tile * kTile + (uint64_t)lo * kGroup;
+      const int cnt = (int)(n - i < (uint64_t)kGroup ? n - i : (uint64_t)kGroup);
+      double x[kGroupThreads][kTileItems];
+#pragma unroll
+      for (int q = 0; q < kGroupThreads; ++q) {
+        if (cnt == kGroup) {
+          src.four(i + q * kTileItems, x[q]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < kTileItems; ++j)
+            x[q][j] = q * kTileItems + j < cnt ? src.one(i + q * kTileItems + j) : 0.0;
+        }
+      }
+      int below = 0;  // elements whose cdf is not above v (the cdf never falls)
+#pragma unroll
+      for (int j = 0; j < kGroup; ++j) {
+        c += x[j / kTileItems][j % kTileItems];
+        below += j < cnt - 1 && c / total <= v;
+      }
+      i += below;
     }
-    out[s] = (int64_t)lo;
+    out[s] = (int64_t)i;
   }
 }
 
@@ -830,8 +859,8 @@ static uint64_t tile_count(uint64_t n) { return (n + kTile - 1) / kTile; }
 
 size_t sample_exact_scratch_bytes(uint64_t n) {
   const uint64_t nt = tile_count(n);
-  return nt * (sizeof(double) + sizeof(TileMap) + sizeof(int)) + (nt + 1) * sizeof(double) +
-         scan_scratch<double>(nt) + 8 * 256;
+  return nt * ((1 + kTileGroups) * sizeof(double) + sizeof(TileMap) + sizeof(int)) +
+         (nt + 1) * sizeof(double) + scan_scratch<double>(nt) + 8 * 256;
 }
 
 // ---- host driver -----------------------------------------------------------
@@ -851,7 +880,7 @@ static inline char *align_up(char *p) {
 }
 
 template <typename S>
-static int sample_exact_t(const S &src, uint64_t n, double *cdf, const double *u_dev,
+static int sample_exact_t(const S &src, uint64_t n, const double *u_dev,
                           uint64_t shots, int64_t *out_dev, void *scratch, const int **bad_dev,
                           hipStream_t st) {
   const uint64_t nt = tile_count(n);
@@ -864,6 +893,8 @@ static int sample_exact_t(const S &src, uint64_t n, double *cdf, const double *u
   w = align_up(w + (nt + 1) * sizeof(double));
   TileMap *maps = (TileMap *)w;
   w = align_up(w + nt * sizeof(TileMap));
+  double *ends = (double *)w;
+  w = align_up(w + nt * kTileGroups * sizeof(double));
   int *bad = need + nt;
   SQ_HIP(hipMemsetAsync(need, 0, (nt + 1) * sizeof(int), st));
   const dim3 g((unsigned)nt), b(kTileThreads);
@@ -873,34 +904,34 @@ static int sample_exact_t(const S &src, uint64_t n, double *cdf, const double *u
   hipLaunchKernelGGL(k_tile_maps<S>, g, b, 0, st, src, n, (const double *)sums, maps);
   hipLaunchKernelGGL(k_tile_tie_maps<S>, g, b, 0, st, src, n, maps);
   hipLaunchKernelGGL(k_tile_chain<S>, dim3(1), b, 0, st, src, n, nt, (const TileMap *)maps,
-                     tile_in, cdf, bad);
+                     tile_in, ends, bad);
   hipLaunchKernelGGL(k_tile_find, sweep_grid(shots, kBlock), dim3(kBlock), 0, st,
                      (const double *)tile_in, nt, u_dev, shots, out_dev, need, (const int *)bad);
   hipLaunchKernelGGL(k_tile_cdf<S>, g, b, 0, st, src, n, (const double *)tile_in,
-                     (const TileMap *)maps, (const int *)need, cdf, (const int *)bad);
+                     (const TileMap *)maps, (const int *)need, ends, (const int *)bad);
   hipLaunchKernelGGL(k_tile_cdf_walk<S>, dim3((unsigned)std::min<uint64_t>(nt, 1024)), b, 0, st,
                      src, n, nt, (const double *)tile_in, (const TileMap *)maps,
-                     (const int *)need, cdf, (const int *)bad);
-  hipLaunchKernelGGL(k_tile_search, sweep_grid(shots, kBlock), dim3(kBlock), 0, st,
-                     (const double *)cdf, n, (const double *)tile_in, nt, u_dev, shots, out_dev,
+                     (const int *)need, ends, (const int *)bad);
+  hipLaunchKernelGGL(k_tile_search<S>, sweep_grid(shots, kBlock), dim3(kBlock), 0, st, src,
+                     (const double *)ends, n, (const double *)tile_in, nt, u_dev, shots, out_dev,
                      (const int *)bad);
   SQ_HIP(hipGetLastError());
   *bad_dev = bad;
   return SQ_OK;
 }
 
-int sample_exact(const double *p, uint64_t n, double *cdf, const double *u_dev, uint64_t shots,
+int sample_exact(const double *p, uint64_t n, const double *u_dev, uint64_t shots,
                  int64_t *out_dev, void *scratch, const int **bad_dev, hipStream_t st) {
-  return sample_exact_t(FromArray{p}, n, cdf, u_dev, shots, out_dev, scratch, bad_dev, st);
+  return sample_exact_t(FromArray{p}, n, u_dev, shots, out_dev, scratch, bad_dev, st);
 }
 
 int sample_exact_state(const void *sv, sq_dtype_t dt, const double *norm2_dev, uint64_t n,
-                       double *cdf, const double *u_dev, uint64_t shots, int64_t *out_dev,
+                       const double *u_dev, uint64_t shots, int64_t *out_dev,
                        void *scratch, const int **bad_dev, hipStream_t st) {
   if (dt == SQ_COMPLEX64)
-    return sample_exact_t(FromState<float2>{(const float2 *)sv, norm2_dev}, n, cdf, u_dev, shots,
+    return sample_exact_t(FromState<float2>{(const float2 *)sv, norm2_dev}, n, u_dev, shots,
                           out_dev, scratch, bad_dev, st);
-  return sample_exact_t(FromState<double2>{(const double2 *)sv, norm2_dev}, n, cdf, u_dev, shots,
+  return sample_exact_t(FromState<double2>{(const double2 *)sv, norm2_dev}, n, u_dev, shots,
                         out_dev, scratch, bad_dev, st);
 }
 

@@ -35,7 +35,7 @@ def _amplitudes(kind, n, rng):
 
 @pytest.mark.parametrize("dtype", ["complex128", "complex64"])
 @pytest.mark.parametrize("kind", ["random", "uniform", "ties", "zeros", "tiny", "steps"])
-@pytest.mark.parametrize("n", [1, 3, 11, 12, 13, 16])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 11, 12, 13, 16])
 def test_exact_samples_by_tiles(C, n, kind, dtype):
     if kind == "tiny" and dtype == "complex64":
         pytest.skip("below complex64's range")

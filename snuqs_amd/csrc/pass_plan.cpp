@@ -320,6 +320,34 @@ static void block_matrix(const PassBlockPlan &b, const PassGates &pg, BlockMatri
       }
       continue;
     }
+    if (k == 1) {  // row pairs in place
+      const double a0 = m[0], b0 = m[1], a1 = m[2], b1 = m[3];
+      const double a2 = m[4], b2 = m[5], a3 = m[6], b3 = m[7];
+      const bool real = b0 == 0.0 && b1 == 0.0 && b2 == 0.0 && b3 == 0.0;
+      for (int base = 0; base < d; ++base) {
+        if (base & mask) continue;
+        double *__restrict__ r0 = M->re + base * d, *__restrict__ i0 = M->im + base * d;
+        double *__restrict__ r1 = M->re + (base | mask) * d, *__restrict__ i1 = M->im + (base | mask) * d;
+        if (real) {
+          for (int c = 0; c < d; ++c) {
+            const double x0 = r0[c], y0 = i0[c], x1 = r1[c], y1 = i1[c];
+            r0[c] = a0 * x0 + a1 * x1;
+            i0[c] = a0 * y0 + a1 * y1;
+            r1[c] = a2 * x0 + a3 * x1;
+            i1[c] = a2 * y0 + a3 * y1;
+          }
+          continue;
+        }
+        for (int c = 0; c < d; ++c) {
+          const double x0 = r0[c], y0 = i0[c], x1 = r1[c], y1 = i1[c];
+          r0[c] = (a0 * x0 - b0 * y0) + (a1 * x1 - b1 * y1);
+          i0[c] = (a0 * y0 + b0 * x0) + (a1 * y1 + b1 * x1);
+          r1[c] = (a2 * x0 - b2 * y0) + (a3 * x1 - b3 * y1);
+          i1[c] = (a2 * y0 + b2 * x0) + (a3 * y1 + b3 * x1);
+        }
+      }
+      continue;
+    }
     for (int base = 0; base < d; ++base) {
       if (base & mask) continue;
       for (int s = 0; s < dk; ++s) {
@@ -343,26 +371,24 @@ static void block_matrix(const PassBlockPlan &b, const PassGates &pg, BlockMatri
   }
 }
 
-// Three bf16 parts of each of the n values v, each part the nearest (ties to
-// even) to what the ones before leave: rounded in the double's own bits, which a
-// float then holds exactly.  v is used up.
-static void split_bf16(double *v, int n, uint16_t *p0, uint16_t *p1, uint16_t *p2) {
-  for (uint16_t *out : {p0, p1, p2})
+// Three bf16 parts of each of the n (at most 1024) values v, each part a nearest
+// 8-bit value to what the ones before leave: t - (t - v) with t = (2^45 + 1) v
+// keeps a double's 8 leading bits (Veltkamp), which a float then holds exactly.
+// v is used up.
+static void split_bf16(double *__restrict__ v, int n, uint16_t *p0, uint16_t *p1, uint16_t *p2) {
+  float f[1024];
+  for (uint16_t *out : {p0, p1, p2}) {
     for (int i = 0; i < n; ++i) {
-      uint64_t u;
-      std::memcpy(&u, v + i, 8);
-      u = (u + 0xfffffffffffull + ((u >> 45) & 1)) & ~0x1fffffffffffull;
-      double r;
-      std::memcpy(&r, &u, 8);
-      const float f = (float)(v[i] == v[i] ? r : v[i]);
-      uint32_t w;
-      std::memcpy(&w, &f, 4);
-      w &= 0xffff0000u;
-      float h;
-      std::memcpy(&h, &w, 4);
-      out[i] = (uint16_t)(w >> 16);
-      v[i] -= h;
+      const double t = v[i] * (0x1p45 + 1.0);
+      f[i] = (float)(t - (t - v[i]));
+      v[i] -= f[i];
     }
+    for (int i = 0; i < n; ++i) {
+      uint32_t w;
+      std::memcpy(&w, f + i, 4);
+      out[i] = (uint16_t)(w >> 16);
+    }
+  }
 }
 
 void pass_image(const PassPlan &p, const std::vector<PassBlock> &blocks, sq_dtype_t dt,

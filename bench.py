@@ -12,7 +12,9 @@ cores; the unfused per-gate sweep is measured too.
 value = algorithmic HBM bytes of the launched kernels / wall time of the timed
 steps (2 x touched amplitudes x 8 B per kernel).  Per-kernel durations come
 from HIP events recorded on the launch stream around every kernel of every
-timed step.
+timed step.  The timed steps launch one kernel per fused block (gate sweeps);
+``passes`` reports the same circuit as Program.run launches it, several blocks
+to a pass over the state.
 
 Also reported: the dominant kernel's roofline, a plain copy kernel's
 bandwidth, the 24-qubit hardware-efficient ansatz gradient by adjoint vs
@@ -531,6 +533,15 @@ def main():
     flops_exec = 0.75 * flops
     norm = C.functionals.norm2(sv)
     log(f"fused: {wall / args.steps * 1e3:.1f} ms/step, {value:.0f} GB/s, norm^2 {norm:.12f}")
+    prog.run(sv)
+    C.core.cuda.device_synchronize()
+    t0 = time.perf_counter()
+    for _ in range(args.steps):
+        prog.run(sv)
+    C.core.cuda.device_synchronize()
+    wall_p = time.perf_counter() - t0
+    passes = {"ms_per_step": wall_p / args.steps * 1e3, "speedup": wall / wall_p}
+    log(f"in passes: {passes['ms_per_step']:.1f} ms/step")
     if args.gate_times:
         rows = []
         for g, (op, (cls, kk, b)) in enumerate(zip(fused, info)):
@@ -618,6 +629,7 @@ def main():
             "mfma_frac_fp32_executed": (flops_exec / (avg_ms * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS
                                         if flops else None),
         },
+        "passes": passes,
         "kernel_ms_per_step": kernel_ms / args.steps,
         # the same bytes over the summed kernel times (HIP events), without launch gaps
         "GBps_kernel_only": step_bytes * args.steps / (kernel_ms * 1e-3) / 1e9,

@@ -90,8 +90,8 @@ int sq_copy(void *dst, const void *src, size_t bytes, void *stream);
  * 128 B runs; default 1) and "adjoint_fuse_runs" (0-3, diagonal runs folded
  * into the low pass of the layer next to them: bit 0 forward, bit 1 reverse;
  * default 3) and "mfma_tiles_per_wave" (1-64, tiles per wave of the 4-5 target
- * MFMA kernels in programs without a tuned shape and in parameter and circuit
- * batches (which size their grids by it when built), lowered where a launch
+ * MFMA kernels in programs without a tuned shape and in parameter batches
+ * (which size their grids by it when built), lowered where a launch
  * would drop below 2048 workgroups; the grid cap above still applies;
  * default 4).  A gate tuned by
  * sq_program_tune uses its own shape instead.  No reference counterpart. */
@@ -171,8 +171,8 @@ int sq_program_run(void *program, void *sv, uint64_t num_elems, void *stream);
  * Asynchronous on `stream` like sq_program_run. */
 int sq_program_run_graph(void *program, void *sv, uint64_t num_elems, void *stream);
 /* Measurement variant of sq_program_run: every gate as a launch of its own
- * kernel, with a HIP event recorded before each and one after the last on `stream`, waits for completion and writes
- * each gate's elapsed time to ms_per_gate[num_gates] (0 for gates that
+ * kernel, with a HIP event recorded before each and one after the last on
+ * `stream`, waits for completion and writes each gate's elapsed time to ms_per_gate[num_gates] (0 for gates that
  * launch nothing). */
 int sq_program_run_timed(void *program, void *sv, uint64_t num_elems,
                          void *stream, float *ms_per_gate);
@@ -182,7 +182,8 @@ int sq_program_run_timed(void *program, void *sv, uint64_t num_elems,
  * gate's fastest for the gate and its inverse.  Choices are cached process-wide by dtype, state
  * size and target/control bits, so later programs with the same gates reuse
  * them without timing.  Results do not depend on the shape (the same
- * arithmetic runs in every shape).  sv is overwritten: the gates are applied
+ * arithmetic runs in every shape).  The shapes apply to gates run alone, not to
+ * the passes of sq_program_run.  sv is overwritten: the gates are applied
  * to it many times.  *num_tuned (may be NULL) = gates given a shape. */
 int sq_program_tune(void *program, void *sv, uint64_t num_elems, int reps,
                     void *stream, uint32_t *num_tuned);

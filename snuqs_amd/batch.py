@@ -3,9 +3,9 @@
 The reference runs one circuit per call and has no batching (its
 optimize_operations stub, src/braket/snuqs/transpile.py:233-234, is where
 one would go).  Here K parameter sets of a parametrised circuit run together:
-the K states sit in one device buffer (``StateBatch``), every gate is one
-launch over all K states with each state's own matrix (``BatchProgram``,
-sq_batch_*), and the energies of all K states come from one batched Pauli
+the K states sit in one device buffer (``StateBatch``), every pass over the
+states (several gates, or one) is one launch over all K of them with each
+state's own matrices (``BatchProgram``, sq_batch_*), and the energies of all K states come from one batched Pauli
 reduction (``expectation_batch``).  Fusion groups gates by their targets
 only, so every set fuses into the same blocks (``fuse_operations_batch``).
 """

@@ -5,9 +5,10 @@ no batching (``transpile.py:233-234`` is where it would go).  For workloads of
 many circuits, each too small to fill the GPU alone (ensembles, sweeps,
 training batches of different circuits), ``circuit_batch`` compiles every
 circuit (by default fused into blocks of at most 5 qubits) and the engine
-(``_C.functionals.CircuitBatch``, ``sq_cbatch_*``) runs them together: launch
-s applies block s of every circuit that has one, so the batch takes as many
-launches as its longest circuit has blocks, captured in one hipGraph.
+(``_C.functionals.CircuitBatch``, ``sq_cbatch_*``) runs them together: step s
+applies pass s (several blocks on chunks of the state held on chip) of every
+circuit that has one, one launch per chunk size, so the batch takes about as
+many launches as its longest circuit has passes, captured in one hipGraph.
 
     batch = circuit_batch([(14, ops_a), (20, ops_b), ...], dtype="complex64")
     batch.run()

@@ -154,8 +154,8 @@ int sample_cdf(const double *p, uint64_t n, double *cdf, bool exact,
                void *scratch, size_t scratch_bytes, hipStream_t st);
 // Exact samples: out_dev[s] = the first index whose cdf is above u_dev[s]
 // (numpy's choice); scratch: sample_exact_scratch_bytes(n).  *bad_dev (device)
-// is nonzero when p holds negative or non-finite entries; nothing else is
-// written then.
+// is nonzero when p holds negative or non-finite entries or its sum overflows;
+// out_dev is not written then.
 int sample_exact(const double *p, uint64_t n, const double *u_dev, uint64_t shots,
                  int64_t *out_dev, void *scratch, const int **bad_dev, hipStream_t st);
 // The same from a state: the probabilities are |a|^2 (/ *norm2_dev unless it is

@@ -702,7 +702,7 @@ __global__ void __launch_bounds__(kTileThreads)
         break;
       }
       const double end = start + (odd(start) ? d1 : d0);
-      const int f = block_min(end >= kTop ? tid : kTileThreads);
+      const int f = block_min(tid >= s && end >= kTop ? tid : kTileThreads);
       if (t < nt && tid >= s && tid <= f) tile_in[t] = down(start);
       if (tid == f) sc = down(start);
       __syncthreads();
@@ -710,13 +710,14 @@ __global__ void __launch_bounds__(kTileThreads)
       double x[kTileItems];
       const int cnt = load_tile(src, n, t0 + f, x);
       c = walk_tile(x, cnt, c, ends + (t0 + f) * kTileGroups);
-      s = f + 1;
+      if (!(c < __builtin_inf())) {  // the sum overflows (c is uniform): no binade to go on in
+        if (tid == 0) *bad = 1;
+        return;
+      }
+      s = f + 1;  // s <= f: every round passes a tile
     }
   }
-  if (tid == 0) {
-    tile_in[nt] = c;
-    if (!(c < __builtin_inf())) *bad = 1;  // the sum overflows
-  }
+  if (tid == 0) tile_in[nt] = c;
 }
 
 // The tile of each uniform: the first whose end is above it (the entries

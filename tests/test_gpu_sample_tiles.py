@@ -68,9 +68,7 @@ def test_more_tiles_than_one_scan(C):
         assert np.array_equal(C.functionals.sample(sv, u, exact=True, normalize=True), want)
 
 
-def test_negative_entries_through_the_c_abi(C):
-    """An array with a negative entry still takes the older route (numpy
-    refuses it; here it gives the cumsum's answer as before)."""
+def _library(C):
     import ctypes
     import os
 
@@ -78,6 +76,42 @@ def test_negative_entries_through_the_c_abi(C):
     P, Q = ctypes.c_void_p, ctypes.c_uint64
     L.sq_sample.argtypes = [P, Q, P, Q, ctypes.c_int, P, P]
     L.sq_memcpy_h2d.argtypes = [P, P, ctypes.c_size_t, P]
+    return L
+
+
+# finite entries whose sum passes the largest double: at the last entry numpy's
+# cdf ends in inf and every index is the last; before it the call is refused
+@pytest.mark.parametrize("n,at", [(1, (0, 1)), (2, (0, 1)), (2, (1, 3)), (13, (10, 20)),
+                                  (13, (10, 8000)), (23, (1 << 22, (1 << 22) + 5)),
+                                  (23, (7, (1 << 23) - 1))])
+def test_sums_past_the_range_of_doubles(C, n, at):
+    L = _library(C)
+    p = np.zeros(1 << n)
+    p[list(at)] = 1.2e308
+    buf = C.result_types.StateVector(C.DeviceType.CUDA, n, dtype="complex64")  # 8 bytes an entry
+    u = np.array([0.0, 0.3, 0.9])
+    out = np.full(3, -1, np.int64)
+    assert L.sq_memcpy_h2d(buf.data_ptr, p.ctypes.data, p.nbytes, None) == 0
+    rc = L.sq_sample(buf.data_ptr, 1 << n, u.ctypes.data, 3, 1, out.ctypes.data, None)
+    if at[1] == (1 << n) - 1:
+        assert rc == 0 and (out == (1 << n) - 1).all()
+    else:
+        assert rc == 1  # SQ_ERR_INVALID
+    # the same from a state
+    a = np.zeros(1 << n, np.complex128)
+    a[list(at)] = 1.1e154  # squares to 1.21e308
+    sv = device_state(C, n, "complex128", a)
+    if at[1] == (1 << n) - 1:
+        assert (C.functionals.sample(sv, u, exact=True) == (1 << n) - 1).all()
+    else:
+        with pytest.raises(ValueError):
+            C.functionals.sample(sv, u, exact=True)
+
+
+def test_negative_entries_through_the_c_abi(C):
+    """An array with a negative entry still takes the older route (numpy
+    refuses it; here it gives the cumsum's answer as before)."""
+    L = _library(C)
     n = 13
     p = np.random.default_rng(1).random(1 << n) / (1 << n)
     p[5000] = -p[5000]

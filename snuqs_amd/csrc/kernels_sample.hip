@@ -552,14 +552,27 @@ __device__ __forceinline__ int load_tile(const S &src, uint64_t n, uint64_t tile
   return cnt;
 }
 
+// The tile of this workgroup: a launch over nt tiles (a power of two) is
+// tile_grid(nt), in two dimensions where one would hold 2^32 work-items (2^34
+// elements).
+constexpr uint64_t kTileGridX = 1ull << 20;
+static dim3 tile_grid(uint64_t nt) {
+  const uint64_t x = std::min(nt, kTileGridX);
+  return dim3((unsigned)x, (unsigned)((nt + x - 1) / x));
+}
+__device__ __forceinline__ uint64_t tile_index() {
+  return (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
+}
+
 // Sum of each tile (any order: it only bounds c); *bad is set by an element
 // that is negative or not finite.
 template <typename S>
 __global__ void __launch_bounds__(kTileThreads)
     k_tile_sums(S src, uint64_t n, double *__restrict__ sums, int *__restrict__ bad) {
   __shared__ double w[kTileThreads / 64];
+  const uint64_t tile = tile_index();
   double x[kTileItems];
-  load_tile(src, n, blockIdx.x, x);
+  load_tile(src, n, tile, x);
   double s = 0.0;
   bool b = false;
 #pragma unroll
@@ -574,7 +587,7 @@ __global__ void __launch_bounds__(kTileThreads)
   if (threadIdx.x == 0) {
     s = 0.0;
     for (int v = 0; v < kTileThreads / 64; ++v) s += w[v];
-    sums[blockIdx.x] = s;
+    sums[tile] = s;
   }
 }
 
@@ -587,9 +600,10 @@ __global__ void __launch_bounds__(kTileThreads, 8)
   __shared__ double w[2][W];
   __shared__ int wf[W];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t tile = tile_index();
   double x[kTileItems];
-  load_tile(src, n, blockIdx.x, x);
-  const double a = blockIdx.x ? scanned[blockIdx.x - 1] : 0.0;
+  load_tile(src, n, tile, x);
+  const double a = tile ? scanned[tile - 1] : 0.0;
   const double slack = (double)(n + 16) * 0x1p-51;
   TileMap m{};
   m.e = binade(a * (1.0 - slack));
@@ -632,17 +646,18 @@ __global__ void __launch_bounds__(kTileThreads, 8)
   m.d[2] = m.d[3] = t1;
   if (!(f & 1)) m.flags |= kAllZero;
   if (f & 2) m.flags |= kTies;
-  if (threadIdx.x == 0) maps[blockIdx.x] = m;
+  if (threadIdx.x == 0) maps[tile] = m;
 }
 
 // The maps of the tiles that hold ties, which depend on the parity of C.
 template <typename S>
 __global__ void __launch_bounds__(kTileThreads)
     k_tile_tie_maps(S src, uint64_t n, TileMap *__restrict__ maps) {
-  const int flags = maps[blockIdx.x].flags, e = maps[blockIdx.x].e;
+  const uint64_t tile = tile_index();
+  const int flags = maps[tile].flags, e = maps[tile].e;
   if (!(flags & kTies)) return;
   double x[kTileItems];
-  load_tile(src, n, blockIdx.x, x);
+  load_tile(src, n, tile, x);
   for (int k = 0; k < ((flags & kHasNext) ? 2 : 1); ++k) {
     const Scale up(52 - e - k);
     double d0, d1, s0 = 0.0, s1 = 0.0;
@@ -653,8 +668,8 @@ __global__ void __launch_bounds__(kTileThreads)
     }
     scan_maps(s0, s1, d0, d1);
     if (threadIdx.x == 0) {
-      maps[blockIdx.x].d[2 * k] = d0;
-      maps[blockIdx.x].d[2 * k + 1] = d1;
+      maps[tile].d[2 * k] = d0;
+      maps[tile].d[2 * k + 1] = d1;
     }
   }
 }
@@ -761,12 +776,12 @@ __global__ void __launch_bounds__(kTileThreads, 8)
                double *__restrict__ ends, const int *__restrict__ bad) {
   constexpr int W = kTileThreads / 64;
   __shared__ double w[W];
-  if (*bad || !need[blockIdx.x] || tile_cdf(tile_in, maps, blockIdx.x) != TileCdf::kPlain)
-    return;
+  const uint64_t tile = tile_index();
+  if (*bad || !need[tile] || tile_cdf(tile_in, maps, tile) != TileCdf::kPlain) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double x[kTileItems];
-  load_tile(src, n, blockIdx.x, x);
-  const double c = tile_in[blockIdx.x];
+  load_tile(src, n, tile, x);
+  const double c = tile_in[tile];
   const int e = binade(c);
   const Scale up(52 - e), down(e - 52);
   double d1;
@@ -789,7 +804,7 @@ __global__ void __launch_bounds__(kTileThreads, 8)
     if (v < wave) start += w[v];
   // (elements past the state's end add nothing)
   if (threadIdx.x % kGroupThreads == kGroupThreads - 1)
-    ends[(uint64_t)blockIdx.x * kTileGroups + threadIdx.x / kGroupThreads] =
+    ends[tile * kTileGroups + threadIdx.x / kGroupThreads] =
         down(start + x[kTileItems - 1]);
 }
 
@@ -898,7 +913,7 @@ static int sample_exact_t(const S &src, uint64_t n, const double *u_dev,
   w = align_up(w + nt * kTileGroups * sizeof(double));
   int *bad = need + nt;
   SQ_HIP(hipMemsetAsync(need, 0, (nt + 1) * sizeof(int), st));
-  const dim3 g((unsigned)nt), b(kTileThreads);
+  const dim3 g = tile_grid(nt), b(kTileThreads);
   hipLaunchKernelGGL(k_tile_sums<S>, g, b, 0, st, src, n, sums, bad);
   SQ_HIP(hipGetLastError());
   SQ_TRY(scan_inplace<double>(sums, nt, (double *)w, st));

@@ -68,6 +68,26 @@ def test_more_tiles_than_one_scan(C):
         assert np.array_equal(C.functionals.sample(sv, u, exact=True, normalize=True), want)
 
 
+def test_largest_state(C):
+    """34 qubits complex64 (128 GiB): 2^22 tiles, whose threads one launch
+    dimension does not hold.  H on the first, a middle and the last qubit gives
+    eight equal entries."""
+    n, item = 34, 8
+    if C.core.cuda.mem_info()[0] < (item << n) + (1 << (n - 1)) + (4 << 30):
+        pytest.skip("needs 140 GiB of free device memory")
+    g = C.operation.gate_operations
+    sv = device_state(C, n, "complex64")
+    where = np.zeros(1, np.int64)
+    for q in (0, 16, n - 1):
+        C.functionals.apply(sv, g.Hadamard([q]), n, [q])
+        where = np.concatenate([where, where | 1 << (n - 1 - q)])
+    u = np.random.default_rng(5).random(500)
+    # the entries differ in the last bits only: no uniform is that close to k / 8
+    assert np.abs(8 * u - np.round(8 * u)).min() > 1e-5
+    got = C.functionals.sample(sv, u, exact=True, normalize=True)
+    assert np.array_equal(got, np.sort(where)[(8 * u).astype(int)])
+
+
 def _library(C):
     import ctypes
     import os

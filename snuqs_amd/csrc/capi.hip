@@ -499,14 +499,8 @@ static int upload_passes(Program *p, hipStream_t st) {
   return SQ_OK;
 }
 
-// The program's forward launches: its steps, or every gate on its own kernel
-// where the state is not on the 16-byte boundary that the passes need.
+// The program's forward launches: its steps.
 static int program_launches(Program *p, void *sv, uint64_t n, hipStream_t st) {
-  if ((uintptr_t)sv & 15) {
-    for (size_t g = 0; g < p->fwd.size(); ++g)
-      SQ_TRY(launch_plan(p->fwd[g], sv, p->dt, n, st, p->fwd_dev[g]));
-    return SQ_OK;
-  }
   for (const Step &s : p->passes.steps) {
     if (s.pass >= 0)
       SQ_TRY(launch_pass_step(p->passes, s.pass, p->dt, sv, n, 1, p->dev_pass, st));

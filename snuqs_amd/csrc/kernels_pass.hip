@@ -33,6 +33,9 @@ namespace sq {
 // holds fewer than 2^32 work-items).
 constexpr uint64_t kPassGrid = 1ull << 22;
 
+// 16 bytes of a state, which starts at any of its elements' boundaries (the
+// accesses are global_load / store_dwordx4, which ask for no more than dwords).
+typedef float state_f4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float pfloatx16 __attribute__((ext_vector_type(16)));
 typedef double pdoublex4 __attribute__((ext_vector_type(4)));
 
@@ -359,7 +362,7 @@ __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, u
     if (c != 0) {  // stays zero
 #pragma unroll
       for (int k = 0; k < NL; ++k)
-        __builtin_nontemporal_store(v[k], reinterpret_cast<nt_f4 *>(p + ka(k)));
+        __builtin_nontemporal_store((state_f4)v[k], reinterpret_cast<state_f4 *>(p + ka(k)));
       return;
     }
     if (t == 0) {
@@ -373,7 +376,7 @@ __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, u
   } else {
 #pragma unroll
     for (int k = 0; k < NL; ++k) {
-      const nt_f4 *q = reinterpret_cast<const nt_f4 *>(p + ka(k));
+      const state_f4 *q = reinterpret_cast<const state_f4 *>(p + ka(k));
       if constexpr (STREAM) v[k] = __builtin_nontemporal_load(q);
       else v[k] = *q;
     }
@@ -419,8 +422,8 @@ __device__ __forceinline__ void pass_chunk(typename CV<R>::T *__restrict__ sv, u
     } else {
       o = *reinterpret_cast<const nt_f4 *>(X + (tw ^ kw(k)));
     }
-    nt_f4 *q = reinterpret_cast<nt_f4 *>(p + ka(k));
-    if constexpr (STREAM) __builtin_nontemporal_store(o, q);
+    state_f4 *q = reinterpret_cast<state_f4 *>(p + ka(k));
+    if constexpr (STREAM) __builtin_nontemporal_store((state_f4)o, q);
     else *q = o;
   }
 }

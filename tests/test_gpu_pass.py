@@ -62,10 +62,33 @@ def test_set_gates_from_identities(C, dtype):
     assert np.abs(to_np(C, sv) - run_oracle(n, ops)).max() <= TOL[dtype]
 
 
+P = ctypes.c_void_p
+
+
+def _library(C):
+    L = ctypes.CDLL(os.path.join(os.path.dirname(C.__file__), "libsnuqs_hip.so"))
+    U32 = ctypes.c_uint32
+    L.sq_memcpy_h2d.argtypes = [P, P, ctypes.c_size_t, P]
+    L.sq_program_create.argtypes = [ctypes.POINTER(P), ctypes.c_int, U32, U32, P, P, P]
+    L.sq_program_run.argtypes = [P, P, ctypes.c_uint64, P]
+    L.sq_program_destroy.argtypes = [P]
+    L.sq_batch_create.argtypes = [ctypes.POINTER(P), ctypes.c_int, U32, U32, U32, P, P, P]
+    L.sq_batch_run.argtypes = [P, P, ctypes.c_uint64, P]
+    L.sq_batch_run_graph.argtypes = [P, P, ctypes.c_uint64, P]
+    L.sq_batch_destroy.argtypes = [P]
+    return L
+
+
+def _gate_arrays(ops):
+    return (np.array([len(op.targets) for op in ops], np.uint32),
+            np.array([q for op in ops for q in op.targets], np.uint32),
+            np.concatenate([np.asarray(op.matrix(), np.complex128).ravel() for op in ops]))
+
+
 def test_unaligned_complex64_state(C):
     """A complex64 state at an odd amplitude (8 bytes past a 16-byte
     boundary), as a C caller may hold it, gets the same result."""
-    L = ctypes.CDLL(os.path.join(os.path.dirname(C.__file__), "libsnuqs_hip.so"))
+    L = _library(C)
     n = 14
     rng = np.random.default_rng(6)
     ops = _circuit(n, rng, 30)
@@ -73,16 +96,8 @@ def test_unaligned_complex64_state(C):
     buf = C.result_types.StateVector(C.DeviceType.CUDA, n + 1, dtype="complex64")
     host = np.zeros(2 << n, np.complex64)
     host[1:1 + (1 << n)] = init
-    P = ctypes.c_void_p
-    nt = np.array([len(op.targets) for op in ops], np.uint32)
-    tg = np.array([q for op in ops for q in op.targets], np.uint32)
-    ms = np.concatenate([np.asarray(op.matrix(), np.complex128).ravel() for op in ops])
+    nt, tg, ms = _gate_arrays(ops)
     prog = P()
-    L.sq_memcpy_h2d.argtypes = [P, P, ctypes.c_size_t, P]
-    L.sq_program_create.argtypes = [ctypes.POINTER(P), ctypes.c_int, ctypes.c_uint32,
-                                    ctypes.c_uint32, P, P, P]
-    L.sq_program_run.argtypes = [P, P, ctypes.c_uint64, P]
-    L.sq_program_destroy.argtypes = [P]
     assert L.sq_memcpy_h2d(buf.data_ptr, host.ctypes.data, host.nbytes, None) == 0
     assert L.sq_program_create(ctypes.byref(prog), 0, n, len(ops), nt.ctypes.data, tg.ctypes.data,
                                ms.ctypes.data) == 0
@@ -93,6 +108,35 @@ def test_unaligned_complex64_state(C):
     got = out[1:1 + (1 << n)].astype(np.complex128)
     assert np.abs(got - run_oracle(n, ops, init.astype(np.complex128))).max() <= TOL["complex64"]
     assert out[0] == 0 and not out[1 + (1 << n):].any()  # nothing beside the state
+
+
+@pytest.mark.parametrize("dtype,at", [("complex64", 8), ("complex128", 16)])
+def test_unaligned_batch_states(C, dtype, at):
+    """The states of a parameter batch one element past the buffer's start."""
+    L = _library(C)
+    n, sets = 12, 3
+    rng = np.random.default_rng(7)
+    circuits = [_circuit(n, np.random.default_rng(8), 30) for _ in range(sets)]
+    nt, tg, _ = _gate_arrays(circuits[0])
+    ms = np.concatenate([_gate_arrays(ops)[2] for ops in circuits])
+    init = [random_state(n, rng, np.dtype(dtype)) for _ in range(sets)]
+    batch = P()
+    assert L.sq_batch_create(ctypes.byref(batch), dtype == "complex128", n, sets, len(nt),
+                             nt.ctypes.data, tg.ctypes.data, ms.ctypes.data) == 0
+    buf = C.result_types.StateVector(C.DeviceType.CUDA, n + 2, dtype=dtype)
+    for run in (L.sq_batch_run, L.sq_batch_run_graph):
+        host = np.zeros(4 << n, dtype)
+        host[1:1 + (sets << n)] = np.concatenate(init)
+        assert L.sq_memcpy_h2d(buf.data_ptr, host.ctypes.data, host.nbytes, None) == 0
+        assert run(batch, buf.data_ptr + at, 1 << n, None) == 0
+        C.core.cuda.device_synchronize()
+        out = np.array(buf.cpu(), copy=True)
+        for y in range(sets):
+            got = out[1 + (y << n):1 + ((y + 1) << n)].astype(np.complex128)
+            ref = run_oracle(n, circuits[y], init[y].astype(np.complex128))
+            assert np.abs(got - ref).max() <= TOL[dtype], y
+        assert out[0] == 0 and not out[1 + (sets << n):].any()
+    L.sq_batch_destroy(batch)
 
 
 # 64 MiB: the smallest state above 1 MiB that passes read with ordinary accesses

@@ -13,6 +13,7 @@
 #include <array>
 #include <map>
 #include <mutex>
+#include <new>
 #include <tuple>
 #include <vector>
 
@@ -330,18 +331,50 @@ static void plan_pass_set(int nq, sq_dtype_t dt, uint32_t nsets, const std::vect
   }
 }
 
-// Host image of a pass set: `gates.matrices` is set 0's matrices, set y's lie
-// set_doubles further on.
-static void pass_set_image(const PassSet &ps, sq_dtype_t dt, uint32_t nsets, PassGates gates,
-                           size_t set_doubles, char *img) {
+// Every gate on its own kernel.
+static void without_passes(size_t ngates, PassSet *ps) {
+  *ps = PassSet{};
+  for (size_t g = 0; g < ngates; ++g) ps->steps.push_back({(int)g, -1});
+}
+
+// Write the descriptors and matrices of a pass set to `dev` (ps.total bytes):
+// `gates.matrices` is set 0's matrices, set y's lie set_doubles further on.  The
+// image goes through a host buffer of a bounded size, in order; returns when the
+// last copy is done.  SQ_ERR_OOM: no room for the buffer.
+static int upload_pass_set(const PassSet &ps, sq_dtype_t dt, uint32_t nsets, PassGates gates,
+                           size_t set_doubles, void *dev, hipStream_t st) {
+  constexpr size_t kStage = (size_t)64 << 20;
+  size_t largest = 0;
+  for (size_t i = 0; i < ps.plans.size(); ++i)
+    largest = std::max({largest, ps.image[i] - ps.desc[i], ps.stride[i]});
+  std::vector<char> buf;
+  try {
+    buf.resize(std::min(ps.total, std::max(kStage, largest)));
+  } catch (const std::bad_alloc &) {
+    return fail(SQ_ERR_OOM, "passes: no host memory for their matrices");
+  }
+  size_t used = 0, done = 0;
+  auto flush = [&]() -> int {
+    SQ_HIP(hipMemcpyAsync((char *)dev + done, buf.data(), used, hipMemcpyHostToDevice, st));
+    SQ_HIP(hipStreamSynchronize(st));
+    done += used;
+    used = 0;
+    return SQ_OK;
+  };
   const double *m0 = gates.matrices;
   for (size_t i = 0; i < ps.plans.size(); ++i) {
-    std::memcpy(img + ps.desc[i], ps.blocks[i].data(), ps.blocks[i].size() * sizeof(PassBlock));
+    const size_t desc = ps.image[i] - ps.desc[i];
+    if (used + desc > buf.size()) SQ_TRY(flush());
+    std::memcpy(buf.data() + used, ps.blocks[i].data(), ps.blocks[i].size() * sizeof(PassBlock));
+    used += desc;
     for (uint32_t y = 0; y < nsets; ++y) {
+      if (used + ps.stride[i] > buf.size()) SQ_TRY(flush());
       gates.matrices = m0 + y * set_doubles;
-      pass_image(ps.plans[i], ps.blocks[i], dt, gates, img + ps.image[i] + y * ps.stride[i]);
+      pass_image(ps.plans[i], ps.blocks[i], dt, gates, buf.data() + used);
+      used += ps.stride[i];
     }
   }
+  return used ? flush() : SQ_OK;
 }
 
 static int launch_pass_step(const PassSet &ps, int i, sq_dtype_t dt, void *sv, uint64_t nelems,
@@ -489,14 +522,10 @@ static std::vector<char> program_image(Program *p) {
 
 // The passes' descriptors and matrices, from the program's matrices.
 static int upload_passes(Program *p, hipStream_t st) {
-  if (!p->passes.total) return SQ_OK;
-  std::vector<char> img(p->passes.total);
-  pass_set_image(p->passes, p->dt, 1,
-                 PassGates{p->mats.data(), &p->moffs, &p->toff, &p->targets, &p->nt, p->nq}, 0,
-                 img.data());
-  SQ_HIP(hipMemcpyAsync(p->dev_pass, img.data(), img.size(), hipMemcpyHostToDevice, st));
-  SQ_HIP(hipStreamSynchronize(st));
-  return SQ_OK;
+  if (!p->dev_pass) return SQ_OK;
+  return upload_pass_set(p->passes, p->dt, 1,
+                         PassGates{p->mats.data(), &p->moffs, &p->toff, &p->targets, &p->nt, p->nq},
+                         0, p->dev_pass, st);
 }
 
 // The program's forward launches: its steps.
@@ -557,17 +586,21 @@ int sq_program_create(void **program, sq_dtype_t dt, uint32_t nq, uint32_t ng,
   for (const GatePlan &g : prog->fwd) touched.push_back(g.touched);
   plan_pass_set(prog->nq, dt, 1, prog->nt, prog->toff, prog->targets, touched, &prog->passes);
   if (prog->passes.total) {
-    if (hipMalloc(&prog->dev_pass, prog->passes.total) != hipSuccess) {
-      (void)hipGetLastError();  // no room for the passes' matrices: gate by gate
+    int rc = SQ_ERR_OOM;
+    if (hipMalloc(&prog->dev_pass, prog->passes.total) == hipSuccess) {
+      rc = upload_passes(prog.get(), nullptr);
+    } else {
+      (void)hipGetLastError();
       prog->dev_pass = nullptr;
-      prog->passes = PassSet{};
-      for (uint32_t g = 0; g < ng; ++g) prog->passes.steps.push_back({(int)g, -1});
     }
-    const int rc = upload_passes(prog.get(), nullptr);
     if (rc != SQ_OK) {
       if (prog->dev_pass) (void)hipFree(prog->dev_pass);
-      if (prog->dev_mats) (void)hipFree(prog->dev_mats);
-      return rc;
+      prog->dev_pass = nullptr;
+      if (rc != SQ_ERR_OOM) {
+        if (prog->dev_mats) (void)hipFree(prog->dev_mats);
+        return rc;
+      }
+      without_passes(ng, &prog->passes);  // no room for the passes' matrices: gate by gate
     }
   }
   *program = prog.release();
@@ -2131,9 +2164,9 @@ struct Batch {
   };
   std::vector<Gate> gates;
   PassSet passes;             // planned once, at creation
-  size_t pass_off = 0;        // their device data in `dev`
+  void *dev_pass = nullptr;   // their descriptors and matrices
   std::vector<char> in_pass;  // gates that run inside a pass: no tables of their own
-  void *dev = nullptr;
+  void *dev = nullptr;        // tables and block matrices of the other gates
   size_t dev_cap = 0;
   uint64_t launches = 0;
   double bytes = 0.0;
@@ -2166,17 +2199,13 @@ static bool same_structure(const GatePlan &a, const GatePlan &b) {
   return true;
 }
 
-// Plans of every gate and set, the host image of the argument tables and
-// block matrices, and its size.  A gate whose sets' matrices fall into
+// Plans of every gate and set.  A gate whose sets' matrices fall into
 // different classes (e.g. RotY(0) = identity next to RotY(0.3)) is planned as
 // a dense gate on all its targets in every set.
-static int plan_batch(Batch *b, const double *matrices, bool create, std::vector<char> *img) {
+static int plan_batch(Batch *b, const double *matrices) {
   const uint64_t n = 1ull << b->nq;
   const size_t ng = b->nt.size();
   std::vector<Batch::Gate> gates(ng);
-  std::vector<char> tab;
-  std::vector<std::pair<size_t, const GatePlan *>> blocks;  // (offset, plan)
-  size_t blk_total = 0;
   uint64_t launches = 0;
   double bytes = 0.0;
   for (size_t g = 0; g < ng; ++g) {
@@ -2204,38 +2233,40 @@ static int plan_batch(Batch *b, const double *matrices, bool create, std::vector
       bytes += 2.0 * P[y].touched * (double)n * itemsize(b->dt);
     ++launches;
   }
-  if (create) {
-    std::vector<double> touched(ng, 0.0);
-    for (size_t g = 0; g < ng; ++g)
-      if (!gates[g].plans.empty()) touched[g] = gates[g].plans[0].touched;
-    plan_pass_set(b->nq, b->dt, b->nsets, b->nt, b->toff, b->targets, touched, &b->passes);
-    b->in_pass.assign(ng, 1);
-    for (const Step &s : b->passes.steps)
-      if (s.gate >= 0) b->in_pass[s.gate] = 0;
-  }
-  for (size_t g = 0; g < ng; ++g) {
-    const std::vector<GatePlan> &P = gates[g].plans;
+  b->gates.swap(gates);
+  b->launches = launches;
+  b->bytes = bytes;
+  return SQ_OK;
+}
+
+// Host image of the argument tables and block matrices of the gates that run on
+// their own.
+static int batch_tables(Batch *b, std::vector<char> *img) {
+  const uint64_t n = 1ull << b->nq;
+  std::vector<char> tab;
+  std::vector<std::pair<size_t, const GatePlan *>> blocks;  // (offset, plan)
+  size_t blk_total = 0;
+  for (size_t g = 0; g < b->gates.size(); ++g) {
+    Batch::Gate &gt = b->gates[g];
+    const std::vector<GatePlan> &P = gt.plans;
+    gt.blk_off = (size_t)-1;
     if (P.empty() || b->in_pass[g]) continue;
     std::vector<const GatePlan *> pp(b->nsets);
     for (uint32_t y = 0; y < b->nsets; ++y) pp[y] = &P[y];
     tab.resize((tab.size() + 255) / 256 * 256);
-    gates[g].tab_off = tab.size();
+    gt.tab_off = tab.size();
     SQ_TRY(batch_gate_table(pp.data(), b->nsets, b->dt, n, &tab));
     if (has_block(P[0])) {
       const size_t bb = block_bytes(P[0].kk, b->dt);
-      gates[g].blk_off = blk_total;
-      gates[g].gstride = bb / (4 * (b->dt == SQ_COMPLEX64 ? 4 : 8));
+      gt.blk_off = blk_total;
+      gt.gstride = bb / (4 * (b->dt == SQ_COMPLEX64 ? 4 : 8));
       for (uint32_t y = 0; y < b->nsets; ++y) blocks.push_back({blk_total + y * bb, &P[y]});
       blk_total += b->nsets * bb;
     }
   }
-  // image: tables, blocks, passes (256-byte aligned)
+  // image: tables, then blocks (256-byte aligned)
   const size_t tab_bytes = (tab.size() + 255) / 256 * 256;
-  b->pass_off = tab_bytes + blk_total;
-  img->assign(b->pass_off + b->passes.total, 0);
-  pass_set_image(b->passes, b->dt, b->nsets,
-                 PassGates{matrices, &b->moffs, &b->toff, &b->targets, &b->nt, b->nq},
-                 b->set_doubles, img->data() + b->pass_off);
+  img->assign(tab_bytes + blk_total, 0);
   std::memcpy(img->data(), tab.data(), tab.size());
   std::vector<const GatePlan *> bp;
   std::vector<size_t> bo;
@@ -2244,11 +2275,8 @@ static int plan_batch(Batch *b, const double *matrices, bool create, std::vector
     bo.push_back(tab_bytes + e.first);
   }
   block_image(bp, b->dt, bo, img->data());
-  for (auto &gt : gates)
+  for (auto &gt : b->gates)
     if (gt.blk_off != (size_t)-1) gt.blk_off += tab_bytes;
-  b->gates.swap(gates);
-  b->launches = launches;
-  b->bytes = bytes;
   return SQ_OK;
 }
 
@@ -2271,12 +2299,53 @@ static int upload_batch(Batch *b, const std::vector<char> &img, hipStream_t st) 
   return SQ_OK;
 }
 
+// The gates that passes hold.
+static void batch_in_pass(Batch *b) {
+  b->in_pass.assign(b->nt.size(), 1);
+  for (const Step &s : b->passes.steps)
+    if (s.gate >= 0) b->in_pass[s.gate] = 0;
+}
+
+// Plan the batch's passes and take the memory for them, if it is to be had.
+static void plan_batch_passes(Batch *b) {
+  std::vector<double> touched(b->nt.size(), 0.0);
+  for (size_t g = 0; g < touched.size(); ++g)
+    if (!b->gates[g].plans.empty()) touched[g] = b->gates[g].plans[0].touched;
+  plan_pass_set(b->nq, b->dt, b->nsets, b->nt, b->toff, b->targets, touched, &b->passes);
+  if (b->passes.total && hipMalloc(&b->dev_pass, b->passes.total) != hipSuccess) {
+    (void)hipGetLastError();
+    b->dev_pass = nullptr;
+    without_passes(b->nt.size(), &b->passes);
+  }
+  batch_in_pass(b);
+}
+
+// The device data of a batch's steps; gate by gate where there is no room for
+// the passes' matrices (6 KiB or more a block and set) beside the rest.
+static int upload_batch_steps(Batch *b, const double *matrices, hipStream_t st) {
+  while (true) {
+    int rc = SQ_OK;
+    if (b->dev_pass)
+      rc = upload_pass_set(b->passes, b->dt, b->nsets,
+                           PassGates{matrices, &b->moffs, &b->toff, &b->targets, &b->nt, b->nq},
+                           b->set_doubles, b->dev_pass, st);
+    std::vector<char> img;
+    if (rc == SQ_OK) rc = batch_tables(b, &img);
+    if (rc == SQ_OK) rc = upload_batch(b, img, st);
+    if (rc != SQ_ERR_OOM || !b->dev_pass) return rc;
+    SQ_HIP(hipFree(b->dev_pass));
+    b->dev_pass = nullptr;
+    without_passes(b->nt.size(), &b->passes);
+    batch_in_pass(b);
+  }
+}
+
 static int batch_launches(Batch *b, void *states, hipStream_t st) {
   const uint64_t n = 1ull << b->nq;
   const char *d = (const char *)b->dev;
   for (const Step &s : b->passes.steps) {
     if (s.pass >= 0) {
-      SQ_TRY(launch_pass_step(b->passes, s.pass, b->dt, states, n, b->nsets, d + b->pass_off, st));
+      SQ_TRY(launch_pass_step(b->passes, s.pass, b->dt, states, n, b->nsets, b->dev_pass, st));
       continue;
     }
     const Batch::Gate &gt = b->gates[s.gate];
@@ -2327,9 +2396,14 @@ int sq_batch_create(void **batch, sq_dtype_t dt, uint32_t nq, uint32_t nsets, ui
     moff += 2ull << (2 * k);
   }
   b->set_doubles = moff;
-  std::vector<char> img;
-  SQ_TRY(plan_batch(b.get(), matrices, true, &img));
-  SQ_TRY(upload_batch(b.get(), img, nullptr));
+  SQ_TRY(plan_batch(b.get(), matrices));
+  plan_batch_passes(b.get());
+  const int rc = upload_batch_steps(b.get(), matrices, nullptr);
+  if (rc != SQ_OK) {
+    if (b->dev_pass) (void)hipFree(b->dev_pass);
+    if (b->dev) (void)hipFree(b->dev);
+    return rc;
+  }
   *batch = b.release();
   return SQ_OK;
 }
@@ -2338,12 +2412,11 @@ int sq_batch_set_matrices(void *batch, const double *matrices, void *stream) {
   Batch *b = (Batch *)batch;
   if (!b) return fail(SQ_ERR_INVALID, "null batch");
   if (!matrices && !b->nt.empty()) return fail(SQ_ERR_INVALID, "null matrices");
-  std::vector<char> img;
-  SQ_TRY(plan_batch(b, matrices, false, &img));
+  SQ_TRY(plan_batch(b, matrices));
   drop_batch_graph(b);
   // work already queued on `stream` may still read the old tables: the new
-  // image is copied behind it
-  return upload_batch(b, img, (hipStream_t)stream);
+  // ones are copied behind it
+  return upload_batch_steps(b, matrices, (hipStream_t)stream);
 }
 
 int sq_batch_run(void *batch, void *states, uint64_t n, void *stream) {
@@ -2395,6 +2468,7 @@ int sq_batch_destroy(void *batch) {
   Batch *b = (Batch *)batch;
   if (!b) return SQ_OK;
   drop_batch_graph(b);
+  if (b->dev_pass) SQ_HIP(hipFree(b->dev_pass));
   if (b->dev) SQ_HIP(hipFree(b->dev));
   delete b;
   return SQ_OK;

@@ -168,3 +168,71 @@ def test_gates_with_ordinary_accesses(C, dtype, n):
     for op in ops:
         C.functionals.apply(sv, op, n, op.targets)
     assert np.abs(to_np(C, sv) - run_oracle(n, ops, init.astype(np.complex128))).max() <= TOL[dtype]
+
+
+@pytest.fixture
+def little_memory(C):
+    """Device memory taken until 64 MiB or less are left."""
+    L = _library(C)
+    L.sq_malloc.argtypes = [ctypes.POINTER(P), ctypes.c_size_t]
+    L.sq_free.argtypes = [P]
+    left, held = 64 << 20, []
+
+    def take():
+        size = C.core.cuda.mem_info()[0] - left
+        while size >= 1 << 20:
+            p = P()
+            if L.sq_malloc(ctypes.byref(p), size) == 0:
+                held.append(p)
+                size = min(size, C.core.cuda.mem_info()[0] - left)
+            else:
+                size //= 2
+        assert C.core.cuda.mem_info()[0] <= left + (4 << 20)
+
+    yield take
+    for p in held:
+        L.sq_free(p)
+
+
+def _small_gates(n, gates, seed):
+    from snuqs_amd.circuits import haar_unitary
+    from snuqs_amd._C.operation import gate_operations as g
+
+    where, rng = np.random.default_rng(n), np.random.default_rng(seed)
+    return [g.Unitary([int(q) for q in where.permutation(n)[:k]], haar_unitary(1 << k, rng))
+            for k in where.integers(1, 3, gates)]
+
+
+def test_program_without_room_for_passes(C, little_memory):
+    """60,000 gates on 10 qubits: some 100 MB of pass matrices."""
+    n = 10
+    ops = _small_gates(n, 60000, 1)
+    sv = device_state(C, n, "complex128")
+    little_memory()
+    prog = C.functionals.Program(n, ops, dtype="complex128")
+    prog.run(sv)
+    # 60,000 roundings of 2^-53 on a unit vector, in the same order as the oracle
+    assert np.abs(to_np(C, sv) - run_oracle(n, ops)).max() <= 1e-11
+
+
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+def test_batch_without_room_for_passes(C, little_memory, dtype):
+    """2,048 sets of 120 gates on 10 qubits: 6 KiB or more a block and set,
+    some 250 MB, where the gates' own tables are 20; new matrices too."""
+    from snuqs_amd.batch import BatchProgram, StateBatch
+
+    n, sets, gates = 10, 2048, 120
+    different = [_small_gates(n, gates, seed) for seed in range(3)]
+    states = StateBatch(sets, n, dtype=dtype)
+    little_memory()
+    b = BatchProgram(n, [different[y % 3] for y in range(sets)], dtype=dtype)
+    for first in (0, 1):
+        if first:
+            b.set_gates([different[(y + 1) % 3] for y in range(sets)])
+        for use_graph in (False, True):
+            states.initialize_basis_z()
+            b.run(states, use_graph=use_graph)
+            for y in (0, 1, 2, sets - 1):
+                got = np.array(states.state(y).cpu(), copy=True).astype(np.complex128)
+                ref = run_oracle(n, different[(y + first) % 3])
+                assert np.abs(got - ref).max() <= TOL[dtype], (y, use_graph)

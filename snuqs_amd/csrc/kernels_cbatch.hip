@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <cstring>
 #include <memory>
+#include <new>
 #include <vector>
 
 #include "kernels.hpp"
@@ -215,84 +216,62 @@ static void free_cbatch(CBatch *b) {
   if (b->graph) (void)hipGraphDestroy(b->graph);
   for (void *p : {b->states, b->mats, (void *)b->tables, b->pass, (void *)b->psi})
     if (p) (void)hipFree(p);
+  b->states = b->mats = b->pass = nullptr;
+  b->tables = nullptr;
+  b->psi = nullptr;
 }
 
-int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *nq,
-                  const uint32_t *ng, const uint32_t *nt, const uint32_t *targets,
-                  const double *matrices) {
-  if (ncirc == 0) return fail(SQ_ERR_INVALID, "circuit batch: no circuits");
-  auto B = std::make_unique<CBatch>();
-  B->dt = dt;
-  B->ncirc = ncirc;
-  const size_t item = itemsize(dt);
-  const bool c64 = dt == SQ_COMPLEX64;
-  // every gate as a dense matrix on exactly its targets
-  std::vector<std::vector<GatePlan>> plans(ncirc);
-  std::vector<std::vector<int>> cnt(ncirc);
-  std::vector<std::vector<size_t>> toff(ncirc), moff(ncirc);
-  std::vector<uint32_t> tg;
-  size_t gi = 0, ti = 0, mi = 0;
-  uint32_t maxg = 0;
-  uint64_t amp = 0;
-  for (uint32_t j = 0; j < ncirc; ++j) {
-    if (nq[j] < 1 || nq[j] > 30)
-      return fail(SQ_ERR_INVALID, "circuit batch: qubit counts must be in [1, 30]");
-    plans[j].resize(ng[j]);
-    for (uint32_t g = 0; g < ng[j]; ++g, ++gi) {
-      const int k = (int)nt[gi];
-      if (k < 1 || k > kMaxK || k > (int)nq[j])
-        return fail(SQ_ERR_INVALID, "circuit batch: circuit " + std::to_string(j) + ", gate " +
-                                        std::to_string(g) + ": 1 to 5 targets, at most the qubit count");
-      SQ_TRY(make_plan(matrices + mi, targets + ti, k, (int)nq[j], (int)nq[j], &plans[j][g],
-                       kPlanDense | kPlanExact));
-      if (plans[j][g].kind != Kind::DENSE || plans[j][g].kk != k)
-        return fail(SQ_ERR_INVALID, "circuit batch: internal: gate not planned dense");
-      cnt[j].push_back(k);
-      toff[j].push_back(ti);
-      moff[j].push_back(mi);
-      ti += (size_t)k;
-      mi += 2ull << (2 * k);
-    }
-    maxg = std::max(maxg, ng[j]);
-    B->nq.push_back(nq[j]);
-    B->host_psi.push_back(amp);
-    amp += 1ull << nq[j];
-    B->state_bytes += std::ldexp(1.0, (int)nq[j]) * (double)item;
+// Gates of a batch's circuits as dense matrices on exactly their targets.
+struct CBInput {
+  const double *matrices;
+  std::vector<std::vector<GatePlan>> plans;        // [circuit][gate]
+  std::vector<std::vector<int>> nt;
+  std::vector<std::vector<size_t>> toff, moff;     // in `targets`, in `matrices`
+  std::vector<uint32_t> targets;
+};
+
+static int cb_malloc(void **ptr, size_t bytes) {
+  if (hipMalloc(ptr, std::max<size_t>(bytes, 16)) != hipSuccess) {
+    (void)hipGetLastError();
+    *ptr = nullptr;
+    return fail(SQ_ERR_OOM, "circuit batch: device allocation of " + std::to_string(bytes) +
+                                " failed");
   }
-  tg.assign(targets, targets + ti);
-  B->nelems = amp;
+  return SQ_OK;
+}
+
+// Steps, launches and device data of a batch: circuits large enough run in
+// passes if `with_passes`, every circuit gate by gate otherwise.  SQ_ERR_OOM: no
+// room on the device or the host; `B` then holds no device data.
+static int cbatch_build(CBatch *B, const CBInput &in, bool with_passes) try {
+  const sq_dtype_t dt = B->dt;
+  const bool c64 = dt == SQ_COMPLEX64;
+  const size_t item = itemsize(dt);
+  const uint32_t ncirc = B->ncirc;
+  const std::vector<uint32_t> &nq = B->nq;
+  const auto &plans = in.plans;
+  B->launches.clear();
+  B->zero_first = false;
   // Steps of the circuits that run in passes.  Chunks are chosen by the batch's
   // amplitudes: together the circuits fill the chip as one state of that size
   // would.
-  const int nbits = log2u(amp);
+  const int nbits = log2u(B->nelems);
   std::vector<std::vector<PassPlan>> passes(ncirc);
   size_t steps = 0;
   for (uint32_t j = 0; j < ncirc; ++j) {
     const int cb = std::min<int>(pass_chunk_bits(dt, nbits), (int)nq[j]);
-    if (cb < pass_min_bits(dt) || ng[j] == 0) {
+    const size_t ng = plans[j].size();
+    if (!with_passes || cb < pass_min_bits(dt) || ng == 0) {
       B->zero_first = true;
-      steps = std::max<size_t>(steps, ng[j]);
+      steps = std::max(steps, ng);
       continue;
     }
-    std::vector<uint64_t> masks(ng[j], 0);
-    for (uint32_t g = 0; g < ng[j]; ++g)
+    std::vector<uint64_t> masks(ng, 0);
+    for (size_t g = 0; g < ng; ++g)
       for (int b = 0; b < plans[j][g].kk; ++b) masks[g] |= 1ull << plans[j][g].tbit[b];
     std::vector<Step> st;
     plan_passes((int)nq[j], cb, dt, masks, nullptr, &st, &passes[j]);
     steps = std::max(steps, passes[j].size());
-  }
-  // the gate-by-gate step count (stats): 5-target blocks (4 targets from 15
-  // qubits on) in one launch, the others in another
-  for (uint32_t s = 0; s < maxg; ++s) {
-    bool big = false, small = false;
-    for (uint32_t j = 0; j < ncirc; ++j) {
-      if (s >= ng[j]) continue;
-      B->traffic_bytes += 2.0 * std::ldexp(1.0, (int)nq[j]) * (double)item;
-      const int k = plans[j][s].kk;
-      const bool five = k == 5 ? (int)nq[j] >= pass_min_bits(dt) : k == 4 && nq[j] >= 15;
-      (five ? big : small) = true;
-    }
-    B->gate_launches += (uint64_t)big + (uint64_t)small;
   }
   // matrices in the state's precision, tables per launch
   std::vector<double> hm;  // interleaved re/im, converted below
@@ -304,7 +283,7 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
   for (size_t s = 0; s < steps; ++s) {
     CBatch::Launch L{0, tabs.size(), 0, 0};
     for (uint32_t j = 0; j < ncirc; ++j) {
-      if (!passes[j].empty() || s >= ng[j]) continue;
+      if (!passes[j].empty() || s >= plans[j].size()) continue;
       const GatePlan &p = plans[j][s];
       CBGate e{};
       e.psi = B->host_psi[j];
@@ -347,7 +326,7 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
         e.geom = pass_geom(p);
         images.resize(images.size() + bytes);
         pass_image(p, pb, dt,
-                   PassGates{matrices, &moff[j], &toff[j], &tg, &cnt[j], (int)nq[j]},
+                   PassGates{in.matrices, &in.moff[j], &in.toff[j], &in.targets, &in.nt[j], (int)nq[j]},
                    images.data() + e.image);
         descs.insert(descs.end(), pb.begin(), pb.end());
         const uint64_t chunks = 1ull << (nq[j] - cb);
@@ -360,7 +339,6 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
       if (P.blocks) B->launches.push_back(P);
     }
   }
-  B->traffic_bytes += (double)amp * (double)item;  // the initial state
   std::vector<char> pimg;
   auto put = [&](const void *src, size_t bytes) {
     const size_t off = (pimg.size() + 255) / 256 * 256;
@@ -372,27 +350,18 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
   B->pass_map = put(wgs.data(), wgs.size() * sizeof(uint32_t));
   B->pass_desc = put(descs.data(), descs.size() * sizeof(PassBlock));
   B->pass_img = put(images.data(), images.size());
-  auto dmalloc = [](void **ptr, size_t bytes) -> int {
-    if (hipMalloc(ptr, std::max<size_t>(bytes, 16)) != hipSuccess) {
-      (void)hipGetLastError();
-      *ptr = nullptr;
-      return fail(SQ_ERR_OOM, "circuit batch: device allocation of " + std::to_string(bytes) +
-                                  " failed");
-    }
-    return SQ_OK;
-  };
   const size_t nm = hm.size() / 2;
-  int rc = dmalloc(&B->states, amp * item);
-  if (!rc) rc = dmalloc(&B->mats, nm * item);
-  if (!rc) rc = dmalloc((void **)&B->tables, tabs.size() * sizeof(CBGate));
-  if (!rc) rc = dmalloc(&B->pass, pimg.size());
-  if (!rc) rc = dmalloc((void **)&B->psi, ncirc * sizeof(uint64_t));
+  int rc = cb_malloc(&B->states, B->nelems * item);
+  if (!rc) rc = cb_malloc(&B->mats, nm * item);
+  if (!rc) rc = cb_malloc((void **)&B->tables, tabs.size() * sizeof(CBGate));
+  if (!rc) rc = cb_malloc(&B->pass, pimg.size());
+  if (!rc) rc = cb_malloc((void **)&B->psi, ncirc * sizeof(uint64_t));
   if (rc) {
-    free_cbatch(B.get());
+    free_cbatch(B);
     return rc;
   }
   bool ok = true;
-  if (dt == SQ_COMPLEX64) {
+  if (c64) {
     std::vector<float> hf(hm.begin(), hm.end());
     ok = hipMemcpy(B->mats, hf.data(), hf.size() * sizeof(float), hipMemcpyHostToDevice) ==
          hipSuccess;
@@ -407,9 +376,77 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
   ok = ok && hipMemcpy(B->psi, B->host_psi.data(), ncirc * sizeof(uint64_t),
                        hipMemcpyHostToDevice) == hipSuccess;
   if (!ok) {
-    free_cbatch(B.get());
+    free_cbatch(B);
     return fail(SQ_ERR_HIP, "circuit batch: upload failed");
   }
+  return SQ_OK;
+} catch (const std::bad_alloc &) {
+  free_cbatch(B);
+  return fail(SQ_ERR_OOM, "circuit batch: no host memory for its tables");
+}
+
+int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *nq,
+                  const uint32_t *ng, const uint32_t *nt, const uint32_t *targets,
+                  const double *matrices) {
+  if (ncirc == 0) return fail(SQ_ERR_INVALID, "circuit batch: no circuits");
+  auto B = std::make_unique<CBatch>();
+  B->dt = dt;
+  B->ncirc = ncirc;
+  const size_t item = itemsize(dt);
+  CBInput in;
+  in.matrices = matrices;
+  in.plans.resize(ncirc);
+  in.nt.resize(ncirc);
+  in.toff.resize(ncirc);
+  in.moff.resize(ncirc);
+  size_t gi = 0, ti = 0, mi = 0;
+  uint32_t maxg = 0;
+  uint64_t amp = 0;
+  for (uint32_t j = 0; j < ncirc; ++j) {
+    if (nq[j] < 1 || nq[j] > 30)
+      return fail(SQ_ERR_INVALID, "circuit batch: qubit counts must be in [1, 30]");
+    in.plans[j].resize(ng[j]);
+    for (uint32_t g = 0; g < ng[j]; ++g, ++gi) {
+      const int k = (int)nt[gi];
+      if (k < 1 || k > kMaxK || k > (int)nq[j])
+        return fail(SQ_ERR_INVALID, "circuit batch: circuit " + std::to_string(j) + ", gate " +
+                                        std::to_string(g) + ": 1 to 5 targets, at most the qubit count");
+      SQ_TRY(make_plan(matrices + mi, targets + ti, k, (int)nq[j], (int)nq[j], &in.plans[j][g],
+                       kPlanDense | kPlanExact));
+      if (in.plans[j][g].kind != Kind::DENSE || in.plans[j][g].kk != k)
+        return fail(SQ_ERR_INVALID, "circuit batch: internal: gate not planned dense");
+      in.nt[j].push_back(k);
+      in.toff[j].push_back(ti);
+      in.moff[j].push_back(mi);
+      ti += (size_t)k;
+      mi += 2ull << (2 * k);
+    }
+    maxg = std::max(maxg, ng[j]);
+    B->nq.push_back(nq[j]);
+    B->host_psi.push_back(amp);
+    amp += 1ull << nq[j];
+    B->state_bytes += std::ldexp(1.0, (int)nq[j]) * (double)item;
+  }
+  in.targets.assign(targets, targets + ti);
+  B->nelems = amp;
+  // the gate-by-gate step count (stats): 5-target blocks (4 targets from 15
+  // qubits on) in one launch, the others in another
+  for (uint32_t s = 0; s < maxg; ++s) {
+    bool big = false, small = false;
+    for (uint32_t j = 0; j < ncirc; ++j) {
+      if (s >= ng[j]) continue;
+      B->traffic_bytes += 2.0 * std::ldexp(1.0, (int)nq[j]) * (double)item;
+      const int k = in.plans[j][s].kk;
+      const bool five = k == 5 ? (int)nq[j] >= pass_min_bits(dt) : k == 4 && nq[j] >= 15;
+      (five ? big : small) = true;
+    }
+    B->gate_launches += (uint64_t)big + (uint64_t)small;
+  }
+  B->traffic_bytes += (double)amp * (double)item;  // the initial state
+  // (the passes' matrices, 6 KiB or more a block, can be what does not fit)
+  int rc = cbatch_build(B.get(), in, true);
+  if (rc == SQ_ERR_OOM) rc = cbatch_build(B.get(), in, false);
+  if (rc != SQ_OK) return rc;
   *handle = B.release();
   return SQ_OK;
 }

@@ -172,13 +172,14 @@ def test_gates_with_ordinary_accesses(C, dtype, n):
 
 @pytest.fixture
 def little_memory(C):
-    """Device memory taken until 64 MiB or less are left."""
+    """take(mib): device memory taken until that many MiB or less are left."""
     L = _library(C)
     L.sq_malloc.argtypes = [ctypes.POINTER(P), ctypes.c_size_t]
     L.sq_free.argtypes = [P]
-    left, held = 64 << 20, []
+    held = []
 
-    def take():
+    def take(mib):
+        left = mib << 20
         size = C.core.cuda.mem_info()[0] - left
         while size >= 1 << 20:
             p = P()
@@ -208,7 +209,7 @@ def test_program_without_room_for_passes(C, little_memory):
     n = 10
     ops = _small_gates(n, 60000, 1)
     sv = device_state(C, n, "complex128")
-    little_memory()
+    little_memory(64)
     prog = C.functionals.Program(n, ops, dtype="complex128")
     prog.run(sv)
     # 60,000 roundings of 2^-53 on a unit vector, in the same order as the oracle
@@ -224,7 +225,7 @@ def test_batch_without_room_for_passes(C, little_memory, dtype):
     n, sets, gates = 10, 2048, 120
     different = [_small_gates(n, gates, seed) for seed in range(3)]
     states = StateBatch(sets, n, dtype=dtype)
-    little_memory()
+    little_memory(64)
     b = BatchProgram(n, [different[y % 3] for y in range(sets)], dtype=dtype)
     for first in (0, 1):
         if first:
@@ -236,3 +237,20 @@ def test_batch_without_room_for_passes(C, little_memory, dtype):
                 got = np.array(states.state(y).cpu(), copy=True).astype(np.complex128)
                 ref = run_oracle(n, different[(y + first) % 3])
                 assert np.abs(got - ref).max() <= TOL[dtype], (y, use_graph)
+
+
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+def test_circuit_batch_without_room_for_passes(C, little_memory, dtype):
+    """2,048 circuits of 120 gates on 10 qubits: some 300 MB of pass matrices,
+    where the states, matrices and tables are 75 to 115."""
+    from snuqs_amd.cbatch import circuit_batch
+
+    n, circuits, gates = 10, 2048, 120
+    different = [_small_gates(n, gates, seed) for seed in range(3)]
+    little_memory(160)
+    b = circuit_batch([(n, different[y % 3]) for y in range(circuits)], dtype=dtype, fuse=False)
+    for use_graph in (False, True):
+        b.run(use_graph=use_graph)
+        for y in (0, 1, 2, circuits - 1):
+            got = b.state(y).astype(np.complex128)
+            assert np.abs(got - run_oracle(n, different[y % 3])).max() <= TOL[dtype], (y, use_graph)

@@ -334,8 +334,6 @@ static int cbatch_build(CBatch *B, const CBInput &in, bool with_passes) try {
         P.blocks += chunks;
         entries.push_back(e);
       }
-      if (P.blocks > (1ull << 22))
-        return fail(SQ_ERR_INVALID, "circuit batch: too many circuits for one launch per step");
       if (P.blocks) B->launches.push_back(P);
     }
   }

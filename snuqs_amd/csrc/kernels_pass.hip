@@ -29,8 +29,8 @@
 
 namespace sq {
 
-// Workgroups of a pass in x (one chunk each); the rest go to z (a dimension
-// holds fewer than 2^32 work-items).
+// Workgroups of a pass in x (one chunk each), since a dimension holds fewer than
+// 2^32 work-items; the rest go to z, or to further launches (circuit batches).
 constexpr uint64_t kPassGrid = 1ull << 22;
 
 // 16 bytes of a state, which starts at any of its elements' boundaries (the
@@ -444,15 +444,17 @@ __global__ void SQ_PASS_BOUNDS
     pass_chunk<R, CB, STREAM>(sv + blockIdx.y * sstride, c, geom, blocks, nblocks, G, false, lds);
 }
 
-// Circuit batches: workgroup w takes chunk w - first of its entry.
+// Circuit batches: workgroup w of a step takes chunk w - first of its entry
+// (this launch's are w0, w0 + 1, ...).
 template <typename R, int CB, bool STREAM>
 __global__ void SQ_PASS_BOUNDS
     k_pass_entries(typename CV<R>::T *__restrict__ states, const PassEntry *__restrict__ entries,
-                   const uint32_t *__restrict__ entry, const PassBlock *__restrict__ blocks,
-                   const char *__restrict__ images) {
+                   const uint32_t *__restrict__ entry, uint64_t w0,
+                   const PassBlock *__restrict__ blocks, const char *__restrict__ images) {
   __shared__ PassLds<R, CB> lds;
-  const PassEntry &e = entries[__builtin_amdgcn_readfirstlane(entry[blockIdx.x])];
-  pass_chunk<R, CB, STREAM>(states + e.psi, blockIdx.x - e.first, e.geom, blocks + e.blocks, e.nblocks,
+  const uint64_t w = w0 + blockIdx.x;
+  const PassEntry &e = entries[__builtin_amdgcn_readfirstlane(entry[w])];
+  pass_chunk<R, CB, STREAM>(states + e.psi, w - e.first, e.geom, blocks + e.blocks, e.nblocks,
                         reinterpret_cast<const nt_f4 *>(images + e.image), e.initial != 0, lds);
 }
 
@@ -500,11 +502,14 @@ int launch_pass_entries(int cb, sq_dtype_t dt, void *states, const PassEntry *en
   const bool cached = pass_cached((nwg << cb) * itemsize(dt));
 #define SQ_PASS(R, CB)                                                                          \
   hipLaunchKernelGGL((cached ? k_pass_entries<R, CB, false> : k_pass_entries<R, CB, true>),     \
-                     dim3((unsigned)nwg), dim3(PassShape<R, CB>::NT), 0, st,                    \
-                     (typename CV<R>::T *)states, entries, entry, blocks, (const char *)images)
-  SQ_PASS_SWITCH(cb)
+                     dim3((unsigned)std::min(nwg - w0, kPassGrid)), dim3(PassShape<R, CB>::NT), \
+                     0, st, (typename CV<R>::T *)states, entries, entry, w0, blocks,            \
+                     (const char *)images)
+  for (uint64_t w0 = 0; w0 < nwg; w0 += kPassGrid) {
+    SQ_PASS_SWITCH(cb)
+    SQ_HIP(hipGetLastError());
+  }
 #undef SQ_PASS
-  SQ_HIP(hipGetLastError());
   return SQ_OK;
 }
 

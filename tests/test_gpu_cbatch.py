@@ -91,6 +91,23 @@ def test_cbatch_uneven_gate_counts_and_large_offsets(C):
         assert abs(np.vdot(got, got).real - 1.0) < 1e-12, (j, n)
 
 
+def test_cbatch_more_chunks_than_one_launch(C):
+    """32 circuits of 30 qubits between two of 20 (256 GiB): 2^22 + 256 chunks
+    in a step, more than one launch holds."""
+    from snuqs_amd.cbatch import circuit_batch
+
+    if C.core.cuda.mem_info()[0] < (257 << 30):
+        pytest.skip("needs 257 GiB of free device memory")
+    g = C.operation.gate_operations
+    small = [g.RotY([3], 0.4), g.Hadamard([19])]
+    batch = circuit_batch([(20, small)] + [(30, [g.Hadamard([5])])] * 32 + [(20, small)],
+                          dtype="complex64", fuse=False)
+    batch.run(use_graph=False)
+    ref = run_oracle(20, small)
+    for j in (0, 33):
+        assert np.abs(batch.state(j).astype(np.complex128) - ref).max() < 1e-6, j
+
+
 def test_cbatch_copy_state_checks(C):
     from snuqs_amd.cbatch import circuit_batch
 

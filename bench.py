@@ -630,9 +630,9 @@ def main():
                                         if flops else None),
         },
         "passes": passes,
-        # `value` counts gate sweeps; the program and batch legs below run several
-        # blocks to a pass, so their bytes per second can exceed the HBM peak
-        "leg_bytes": "GB/s of the program and batch legs: 2 x touched amplitudes x itemsize of "
+        # `value` counts gate sweeps; the program and parameter batch legs below run
+        # several blocks to a pass, so their bytes per second can exceed the HBM peak
+        "leg_bytes": "GB/s of the program and parameter batch legs: 2 x touched amplitudes x itemsize of "
                      "every fused block / time, though a pass moves them once for several blocks",
         "kernel_ms_per_step": kernel_ms / args.steps,
         # the same bytes over the summed kernel times (HIP events), without launch gaps

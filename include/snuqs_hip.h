@@ -428,9 +428,7 @@ int sq_cbatch_run(void *batch, int use_graph, void *stream);
  * 2^num_qubits[j] elements of the batch's dtype), ordered on `stream`. */
 int sq_cbatch_copy_state(void *batch, uint32_t circuit, void *dst,
                          uint64_t num_elems, void *stream);
-/* Launches per run and HBM bytes when each step is one gate of every circuit
- * (upper bounds of what sq_cbatch_run takes with passes), bytes of all
- * states. */
+/* Kernel launches per run, bytes of all states, HBM bytes one run moves. */
 int sq_cbatch_stats(void *batch, uint64_t *launches, double *state_bytes,
                     double *traffic_bytes);
 int sq_cbatch_destroy(void *batch);

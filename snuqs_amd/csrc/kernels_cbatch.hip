@@ -204,8 +204,7 @@ struct CBatch {
     uint64_t blocks;
   };
   std::vector<Launch> launches;
-  bool zero_first = false;     // some circuit starts from a state in memory
-  uint64_t gate_launches = 0;  // launches when every step is one gate per circuit
+  bool zero_first = false;  // some circuit starts from a state in memory
   hipGraphExec_t exec = nullptr;
   hipGraph_t graph = nullptr;
   double state_bytes = 0, traffic_bytes = 0;
@@ -252,6 +251,7 @@ static int cbatch_build(CBatch *B, const CBInput &in, bool with_passes) try {
   const auto &plans = in.plans;
   B->launches.clear();
   B->zero_first = false;
+  B->traffic_bytes = 0.0;
   // Steps of the circuits that run in passes.  Chunks are chosen by the batch's
   // amplitudes: together the circuits fill the chip as one state of that size
   // would.
@@ -304,6 +304,7 @@ static int cbatch_build(CBatch *B, const CBInput &in, bool with_passes) try {
       e.nblocks = std::min<uint64_t>((e.nfree + kBlock - 1) / kBlock, kCBMaxBlocksPerGate);
       L.blocks += e.nblocks;
       L.count++;
+      B->traffic_bytes += 2.0 * std::ldexp(1.0, (int)nq[j]) * (double)item;
       tabs.push_back(e);
     }
     if (L.blocks > (uint64_t)INT32_MAX)
@@ -332,11 +333,14 @@ static int cbatch_build(CBatch *B, const CBInput &in, bool with_passes) try {
         const uint64_t chunks = 1ull << (nq[j] - cb);
         wgs.insert(wgs.end(), chunks, (uint32_t)entries.size());
         P.blocks += chunks;
+        // the first pass writes the state, the others read it too
+        B->traffic_bytes += (e.initial ? 1.0 : 2.0) * std::ldexp(1.0, (int)nq[j]) * (double)item;
         entries.push_back(e);
       }
       if (P.blocks) B->launches.push_back(P);
     }
   }
+  if (B->zero_first) B->traffic_bytes += (double)B->nelems * (double)item;
   std::vector<char> pimg;
   auto put = [&](const void *src, size_t bytes) {
     const size_t off = (pimg.size() + 255) / 256 * 256;
@@ -398,7 +402,6 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
   in.toff.resize(ncirc);
   in.moff.resize(ncirc);
   size_t gi = 0, ti = 0, mi = 0;
-  uint32_t maxg = 0;
   uint64_t amp = 0;
   for (uint32_t j = 0; j < ncirc; ++j) {
     if (nq[j] < 1 || nq[j] > 30)
@@ -419,7 +422,6 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
       ti += (size_t)k;
       mi += 2ull << (2 * k);
     }
-    maxg = std::max(maxg, ng[j]);
     B->nq.push_back(nq[j]);
     B->host_psi.push_back(amp);
     amp += 1ull << nq[j];
@@ -427,20 +429,6 @@ int cbatch_create(void **handle, sq_dtype_t dt, uint32_t ncirc, const uint32_t *
   }
   in.targets.assign(targets, targets + ti);
   B->nelems = amp;
-  // the gate-by-gate step count (stats): 5-target blocks (4 targets from 15
-  // qubits on) in one launch, the others in another
-  for (uint32_t s = 0; s < maxg; ++s) {
-    bool big = false, small = false;
-    for (uint32_t j = 0; j < ncirc; ++j) {
-      if (s >= ng[j]) continue;
-      B->traffic_bytes += 2.0 * std::ldexp(1.0, (int)nq[j]) * (double)item;
-      const int k = in.plans[j][s].kk;
-      const bool five = k == 5 ? (int)nq[j] >= pass_min_bits(dt) : k == 4 && nq[j] >= 15;
-      (five ? big : small) = true;
-    }
-    B->gate_launches += (uint64_t)big + (uint64_t)small;
-  }
-  B->traffic_bytes += (double)amp * (double)item;  // the initial state
   // (the passes' matrices, 6 KiB or more a block, can be what does not fit)
   int rc = cbatch_build(B.get(), in, true);
   if (rc == SQ_ERR_OOM) rc = cbatch_build(B.get(), in, false);
@@ -519,7 +507,10 @@ int cbatch_copy_state(void *handle, uint32_t circuit, void *dst, uint64_t nelems
 
 int cbatch_stats(void *handle, uint64_t *launches, double *state_bytes, double *traffic_bytes) {
   CBatch *B = (CBatch *)handle;
-  if (launches) *launches = B->gate_launches + 2;  // + the two initial-state kernels
+  if (launches) {
+    *launches = B->zero_first ? 2 : 0;  // the two initial-state kernels
+    for (const auto &L : B->launches) *launches += L.cb ? pass_entry_launches(L.blocks) : 1;
+  }
   if (state_bytes) *state_bytes = B->state_bytes;
   if (traffic_bytes) *traffic_bytes = B->traffic_bytes;
   return SQ_OK;

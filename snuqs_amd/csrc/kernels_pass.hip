@@ -496,6 +496,8 @@ static void launch_pass_cb(const PassGeom &geom, void *sv, uint64_t nelems, uint
     default: return fail(SQ_ERR_INVALID, "internal: pass chunk size");          \
   }
 
+uint64_t pass_entry_launches(uint64_t nwg) { return (nwg + kPassGrid - 1) / kPassGrid; }
+
 int launch_pass_entries(int cb, sq_dtype_t dt, void *states, const PassEntry *entries,
                         const uint32_t *entry, const PassBlock *blocks, const void *images,
                         uint64_t nwg, hipStream_t st) {

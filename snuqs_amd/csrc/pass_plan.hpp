@@ -102,6 +102,8 @@ struct PassEntry {
 int launch_pass_entries(int cb, sq_dtype_t dt, void *states, const PassEntry *entries,
                         const uint32_t *entry, const PassBlock *blocks, const void *images,
                         uint64_t nwg, hipStream_t stream);
+// The launches that takes.
+uint64_t pass_entry_launches(uint64_t nwg);
 
 // Launch a pass over nsets states of nelems amplitudes (state y at
 // sv + y * nelems, its matrices at image + y * gstride bytes).

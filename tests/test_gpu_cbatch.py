@@ -38,8 +38,14 @@ def test_cbatch_vs_oracle_and_programs(C, dtype, tol, fuse):
     batch = circuit_batch(circs, dtype=dtype, fuse=fuse)
     batch.run(use_graph=False)
     st = batch.stats()
-    nblocks = [len(fuse_operations(ops, 5)) if fuse else len(ops) for _, ops in circs]
-    assert max(nblocks) + 2 <= st["launches"] <= 2 * max(nblocks) + 2
+    nblocks = {n: len(fuse_operations(ops, 5)) if fuse else len(ops) for n, ops in circs}
+    # one launch a step for the circuits below 10 / 9 qubits, and one a step and
+    # chunk size (the qubit counts from there to 12 / 11) for the others' passes
+    least = 10 if dtype == "complex64" else 9
+    alone = max(b for n, b in nblocks.items() if n < least)
+    chunks = len({min(n, least + 2) for n in sizes if n >= least})
+    passes = max(b for n, b in nblocks.items() if n >= least)
+    assert 2 + alone + chunks <= st["launches"] <= 2 + alone + chunks * passes
     for j, (n, ops) in enumerate(circs):
         got = batch.state(j).astype(np.complex128)
         ref = run_oracle(n, ops)
@@ -151,28 +157,53 @@ def test_cbatch_many_circuits(C, dtype, tol):
         assert np.array_equal(batch.state(j), first[j]), j
 
 
-def test_cbatch_tiles_per_wave_bitwise(C):
-    """Steps whose 5-target entries hold enough tiles for 4 tiles per wave
-    (40 circuits of 20 qubits) give the same bits as 1 tile per wave, and
-    agree with Programs run alone."""
+@pytest.mark.parametrize("dtype,sizes,launches", [
+    # below the smallest chunk; every chunk size (2^13 amplitudes of complex64
+    # from 2^20 in all, 2^12 of complex128 from 2^21); two circuits of one size;
+    # no gates
+    ("complex64", [8, 10, 11, 12, 13, 20, 3, 11], 2 + 1 + 4),
+    ("complex128", [8, 9, 10, 11, 12, 21, 3, 10], 2 + 1 + 4),
+    # passes only: nothing to zero
+    ("complex64", [12, 12, 14], 1), ("complex128", [11, 13], 1)])
+def test_cbatch_chunk_sizes(C, dtype, sizes, launches):
+    """One batch of circuits of every chunk size: launches and bytes of a run
+    of one gate each, and the states of longer circuits against the oracle."""
+    from snuqs_amd.cbatch import circuit_batch
+    from snuqs_amd.circuits import random_layered
+
+    g = C.operation.gate_operations
+    item = 8 if dtype == "complex64" else 16
+    least = 10 if dtype == "complex64" else 9
+    one = [(n, [] if n == 3 else [g.RotX([n - 2], 0.3)]) for n in sizes]
+    batch = circuit_batch(one, dtype=dtype)
+    batch.run()
+    st = batch.stats()
+    assert st["launches"] == launches
+    amps = sum(1 << n for n in sizes)
+    zeroed = amps if min(sizes) < least else 0
+    # a first pass writes its state, a gate alone reads and writes it
+    moved = sum((0 if n == 3 else 2 if n < least else 1) << n for n in sizes)
+    assert st["traffic_bytes"] == item * (zeroed + moved)
+    deep = [(n, [] if n == 3 else random_layered(n, 3, seed=40 + j)) for j, n in enumerate(sizes)]
+    tol = 2e-5 if dtype == "complex64" else 1e-12
+    for circs in (one, deep):
+        batch = circuit_batch(circs, dtype=dtype)
+        batch.run()
+        for j, (n, ops) in enumerate(circs):
+            got = batch.state(j).astype(np.complex128)
+            assert np.abs(got - run_oracle(n, ops)).max() < tol, (j, n)
+
+
+def test_cbatch_of_large_circuits(C):
+    """40 circuits of 20 qubits agree with Programs run alone."""
     from snuqs_amd.cbatch import circuit_batch
     from snuqs_amd.circuits import random_layered
     from snuqs_amd.transpile import fuse_operations
 
     circs = [(20, random_layered(20, 3, seed=700 + j)) for j in range(40)]
-    saved = C.core.tune_get("mfma_tiles_per_wave")
-    states = {}
-    try:
-        for tiles in (1, 4):
-            C.core.tune_set("mfma_tiles_per_wave", tiles)
-            batch = circuit_batch(circs, dtype="complex64")
-            batch.run()
-            states[tiles] = [batch.state(j) for j in (0, 13, 39)]
-            del batch
-    finally:
-        C.core.tune_set("mfma_tiles_per_wave", saved)
-    for j, a, b in zip((0, 13, 39), states[1], states[4]):
-        assert np.array_equal(a, b), j
+    batch = circuit_batch(circs, dtype="complex64")
+    batch.run()
+    for j in (0, 13, 39):
         sv = device_state(C, 20, "complex64")
         C.functionals.Program(20, fuse_operations(circs[j][1], 5), dtype="complex64").run(sv)
-        assert np.abs(b.astype(np.complex128) - to_np(C, sv)).max() < 2e-5, j
+        assert np.abs(batch.state(j).astype(np.complex128) - to_np(C, sv)).max() < 2e-5, j

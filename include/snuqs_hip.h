@@ -162,7 +162,8 @@ int sq_program_stats(void *program, uint64_t *num_launches,
 /* Apply every gate (asynchronous on `stream`).  Gates are grouped at creation
  * into passes: the gates of a pass act inside chunks of up to 2^13 amplitudes
  * held on chip, so the state is read and written once per pass.  Gates are
- * reordered only past gates they share no target with. */
+ * reordered only past gates they share no target with.  A pass whose gates, with
+ * their present matrices, touch no more than the state once runs gate by gate. */
 int sq_program_run(void *program, void *sv, uint64_t num_elems, void *stream);
 /* sq_program_run through a hipGraph (no reference counterpart; the reference
  * launches one kernel per Python call, simulation.py:274-284): the launch

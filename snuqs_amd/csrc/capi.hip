@@ -297,28 +297,44 @@ int sq_apply(void *sv, sq_dtype_t dt, uint64_t n, uint32_t num_qubits,
 // ---- programs -----------------------------------------------------------------
 namespace sq {
 
-// The steps of a program or batch (plan_passes) and where each pass's device
-// data sits: descriptors at `desc`, set y's matrices at `image + y * stride`.
+// The steps of a program or batch (plan_passes), and the passes' device data:
+// pass i's descriptors at dev + desc[i], set y's matrices at dev + image[i] + y *
+// stride[i].  Steps and layout depend on the targets alone and stand from creation
+// on; use[i]: whether pass i runs, or its gates on their own, is decided for the
+// matrices at hand.
 struct PassSet {
   std::vector<Step> steps;
   std::vector<PassPlan> plans;
   std::vector<PassGeom> geoms;
   std::vector<std::vector<PassBlock>> blocks;
+  std::vector<char> use;
   std::vector<size_t> desc, image, stride;  // bytes
   size_t total = 0;                         // bytes of descriptors and nsets images
+  void *dev = nullptr;
 };
 
-// Plan the passes of a gate list.  The plan depends on the targets and on
-// the plans' touched fractions at creation; later matrices of the same gates
-// run on the same steps.
+static void free_passes(PassSet *ps) {
+  if (ps->dev) (void)hipFree(ps->dev);
+  ps->dev = nullptr;
+}
+
+// Every gate on its own kernel.
+static void without_passes(size_t ngates, PassSet *ps) {
+  free_passes(ps);
+  *ps = PassSet{};
+  for (size_t g = 0; g < ngates; ++g) ps->steps.push_back({(int)g, -1});
+}
+
+// Plan the steps of a gate list and take the memory for its passes; gate by gate
+// if that is not to be had.
 static void plan_pass_set(int nq, sq_dtype_t dt, uint32_t nsets, const std::vector<int> &nt,
                           const std::vector<size_t> &toff, const std::vector<uint32_t> &targets,
-                          const std::vector<double> &touched, PassSet *ps) {
+                          PassSet *ps) {
   std::vector<uint64_t> masks(nt.size(), 0);
   for (size_t g = 0; g < nt.size(); ++g)
     for (int t = 0; t < nt[g]; ++t) masks[g] |= 1ull << (nq - 1 - (int)targets[toff[g] + t]);
   *ps = PassSet{};
-  plan_passes(nq, pass_chunk_bits(dt, nq), dt, masks, touched.data(), &ps->steps, &ps->plans);
+  plan_passes(nq, pass_chunk_bits(dt, nq), dt, masks, true, &ps->steps, &ps->plans);
   for (const PassPlan &p : ps->plans) {
     size_t bytes;
     ps->geoms.push_back(pass_geom(p));
@@ -329,33 +345,40 @@ static void plan_pass_set(int nq, sq_dtype_t dt, uint32_t nsets, const std::vect
     ps->stride.push_back(bytes);
     ps->total += nsets * bytes;
   }
+  if (ps->total && hipMalloc(&ps->dev, ps->total) != hipSuccess) {
+    (void)hipGetLastError();
+    ps->dev = nullptr;
+    without_passes(nt.size(), ps);
+  }
 }
 
-// Every gate on its own kernel.
-static void without_passes(size_t ngates, PassSet *ps) {
-  *ps = PassSet{};
-  for (size_t g = 0; g < ngates; ++g) ps->steps.push_back({(int)g, -1});
+// Choose the passes that run.
+static void choose_passes(const std::vector<double> &touched, PassSet *ps) {
+  ps->use.clear();
+  for (const PassPlan &p : ps->plans) ps->use.push_back(pass_pays(p, touched));
 }
 
-// Write the descriptors and matrices of a pass set to `dev` (ps.total bytes):
-// `gates.matrices` is set 0's matrices, set y's lie set_doubles further on.  The
-// image goes through a host buffer of a bounded size, in order; returns when the
-// last copy is done.  SQ_ERR_OOM: no room for the buffer.
+// Write the descriptors and matrices of the passes that run to their device
+// memory: `gates.matrices` is set 0's matrices, set y's lie set_doubles further on.
+// They go through a host buffer of a bounded size, in order; returns when the last
+// copy is done.  SQ_ERR_OOM: no room for the buffer.
 static int upload_pass_set(const PassSet &ps, sq_dtype_t dt, uint32_t nsets, PassGates gates,
-                           size_t set_doubles, void *dev, hipStream_t st) {
+                           size_t set_doubles, hipStream_t st) {
   constexpr size_t kStage = (size_t)64 << 20;
   size_t largest = 0;
   for (size_t i = 0; i < ps.plans.size(); ++i)
-    largest = std::max({largest, ps.image[i] - ps.desc[i], ps.stride[i]});
+    if (ps.use[i]) largest = std::max({largest, ps.image[i] - ps.desc[i], ps.stride[i]});
+  if (!largest) return SQ_OK;
   std::vector<char> buf;
   try {
     buf.resize(std::min(ps.total, std::max(kStage, largest)));
   } catch (const std::bad_alloc &) {
     return fail(SQ_ERR_OOM, "passes: no host memory for their matrices");
   }
-  size_t used = 0, done = 0;
+  size_t used = 0, done = 0;  // bytes in `buf`, and where on the device they go
   auto flush = [&]() -> int {
-    SQ_HIP(hipMemcpyAsync((char *)dev + done, buf.data(), used, hipMemcpyHostToDevice, st));
+    if (!used) return SQ_OK;
+    SQ_HIP(hipMemcpyAsync((char *)ps.dev + done, buf.data(), used, hipMemcpyHostToDevice, st));
     SQ_HIP(hipStreamSynchronize(st));
     done += used;
     used = 0;
@@ -364,7 +387,9 @@ static int upload_pass_set(const PassSet &ps, sq_dtype_t dt, uint32_t nsets, Pas
   const double *m0 = gates.matrices;
   for (size_t i = 0; i < ps.plans.size(); ++i) {
     const size_t desc = ps.image[i] - ps.desc[i];
-    if (used + desc > buf.size()) SQ_TRY(flush());
+    if (!ps.use[i]) continue;
+    if (done + used != ps.desc[i] || used + desc > buf.size()) SQ_TRY(flush());
+    done = ps.desc[i] - used;
     std::memcpy(buf.data() + used, ps.blocks[i].data(), ps.blocks[i].size() * sizeof(PassBlock));
     used += desc;
     for (uint32_t y = 0; y < nsets; ++y) {
@@ -374,12 +399,12 @@ static int upload_pass_set(const PassSet &ps, sq_dtype_t dt, uint32_t nsets, Pas
       used += ps.stride[i];
     }
   }
-  return used ? flush() : SQ_OK;
+  return flush();
 }
 
 static int launch_pass_step(const PassSet &ps, int i, sq_dtype_t dt, void *sv, uint64_t nelems,
-                            uint32_t nsets, const void *dev, hipStream_t st) {
-  const char *d = (const char *)dev;
+                            uint32_t nsets, hipStream_t st) {
+  const char *d = (const char *)ps.dev;
   return launch_pass(ps.plans[i], ps.geoms[i], dt, sv, nelems, nsets,
                      (const PassBlock *)(d + ps.desc[i]), (int)ps.blocks[i].size(),
                      d + ps.image[i], ps.stride[i], st);
@@ -402,7 +427,6 @@ struct Program {
   uint64_t launches = 0;
   double bytes = 0.0;
   PassSet passes;                      // the forward run's steps
-  void *dev_pass = nullptr;            // pass descriptors and matrices
   // hipGraph of the forward launch sequence on one state (sq_program_run_graph)
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
@@ -520,21 +544,30 @@ static std::vector<char> program_image(Program *p) {
   return img;
 }
 
-// The passes' descriptors and matrices, from the program's matrices.
-static int upload_passes(Program *p, hipStream_t st) {
-  if (!p->dev_pass) return SQ_OK;
-  return upload_pass_set(p->passes, p->dt, 1,
-                         PassGates{p->mats.data(), &p->moffs, &p->toff, &p->targets, &p->nt, p->nq},
-                         0, p->dev_pass, st);
+// The passes that run, and their descriptors and matrices, from the program's
+// matrices.
+static int build_passes(Program *p, hipStream_t st) {
+  std::vector<double> touched;
+  for (const GatePlan &g : p->fwd) touched.push_back(g.touched);
+  choose_passes(touched, &p->passes);
+  const int rc = upload_pass_set(
+      p->passes, p->dt, 1,
+      PassGates{p->mats.data(), &p->moffs, &p->toff, &p->targets, &p->nt, p->nq}, 0, st);
+  if (rc != SQ_ERR_OOM) return rc;
+  without_passes(p->nt.size(), &p->passes);
+  return SQ_OK;
 }
 
 // The program's forward launches: its steps.
 static int program_launches(Program *p, void *sv, uint64_t n, hipStream_t st) {
+  auto gate = [&](int g) { return launch_plan(p->fwd[g], sv, p->dt, n, st, p->fwd_dev[g]); };
   for (const Step &s : p->passes.steps) {
-    if (s.pass >= 0)
-      SQ_TRY(launch_pass_step(p->passes, s.pass, p->dt, sv, n, 1, p->dev_pass, st));
+    if (s.pass < 0)
+      SQ_TRY(gate(s.gate));
+    else if (p->passes.use[s.pass])
+      SQ_TRY(launch_pass_step(p->passes, s.pass, p->dt, sv, n, 1, st));
     else
-      SQ_TRY(launch_plan(p->fwd[s.gate], sv, p->dt, n, st, p->fwd_dev[s.gate]));
+      for (int g : p->passes.plans[s.pass].gates) SQ_TRY(gate(g));
   }
   return SQ_OK;
 }
@@ -582,26 +615,12 @@ int sq_program_create(void **program, sq_dtype_t dt, uint32_t nq, uint32_t ng,
       return fail(SQ_ERR_HIP, "program matrices: upload failed");
     }
   }
-  std::vector<double> touched;
-  for (const GatePlan &g : prog->fwd) touched.push_back(g.touched);
-  plan_pass_set(prog->nq, dt, 1, prog->nt, prog->toff, prog->targets, touched, &prog->passes);
-  if (prog->passes.total) {
-    int rc = SQ_ERR_OOM;
-    if (hipMalloc(&prog->dev_pass, prog->passes.total) == hipSuccess) {
-      rc = upload_passes(prog.get(), nullptr);
-    } else {
-      (void)hipGetLastError();
-      prog->dev_pass = nullptr;
-    }
-    if (rc != SQ_OK) {
-      if (prog->dev_pass) (void)hipFree(prog->dev_pass);
-      prog->dev_pass = nullptr;
-      if (rc != SQ_ERR_OOM) {
-        if (prog->dev_mats) (void)hipFree(prog->dev_mats);
-        return rc;
-      }
-      without_passes(ng, &prog->passes);  // no room for the passes' matrices: gate by gate
-    }
+  plan_pass_set(prog->nq, dt, 1, prog->nt, prog->toff, prog->targets, &prog->passes);
+  const int rc = build_passes(prog.get(), nullptr);
+  if (rc != SQ_OK) {
+    free_passes(&prog->passes);
+    if (prog->dev_mats) (void)hipFree(prog->dev_mats);
+    return rc;
   }
   *program = prog.release();
   return SQ_OK;
@@ -621,14 +640,14 @@ int sq_program_set_matrices(void *program, const double *matrices, void *stream)
     SQ_HIP(hipMemcpyAsync(p->dev_mats, img.data(), p->dev_cap, hipMemcpyHostToDevice, st));
     SQ_HIP(hipStreamSynchronize(st));
   }
-  return upload_passes(p, st);
+  return build_passes(p, st);
 }
 
 int sq_program_destroy(void *program) {
   Program *p = (Program *)program;
   if (!p) return SQ_OK;
   drop_graph(p);
-  if (p->dev_pass) SQ_HIP(hipFree(p->dev_pass));
+  free_passes(&p->passes);
   if (p->dev_mats) SQ_HIP(hipFree(p->dev_mats));
   delete p;
   return SQ_OK;
@@ -2163,8 +2182,7 @@ struct Batch {
     uint64_t gstride = 0;         // elements between two sets' blocks
   };
   std::vector<Gate> gates;
-  PassSet passes;             // planned once, at creation
-  void *dev_pass = nullptr;   // their descriptors and matrices
+  PassSet passes;
   std::vector<char> in_pass;  // gates that run inside a pass: no tables of their own
   void *dev = nullptr;        // tables and block matrices of the other gates
   size_t dev_cap = 0;
@@ -2299,60 +2317,48 @@ static int upload_batch(Batch *b, const std::vector<char> &img, hipStream_t st) 
   return SQ_OK;
 }
 
-// The gates that passes hold.
-static void batch_in_pass(Batch *b) {
-  b->in_pass.assign(b->nt.size(), 1);
-  for (const Step &s : b->passes.steps)
-    if (s.gate >= 0) b->in_pass[s.gate] = 0;
-}
-
-// Plan the batch's passes and take the memory for them, if it is to be had.
-static void plan_batch_passes(Batch *b) {
-  std::vector<double> touched(b->nt.size(), 0.0);
-  for (size_t g = 0; g < touched.size(); ++g)
+// The passes that run and the device data of all steps; gate by gate where there
+// is no room for the passes' matrices (6 KiB or more a block and set) beside the
+// rest.
+static int build_batch_steps(Batch *b, const double *matrices, hipStream_t st) {
+  const size_t ng = b->nt.size();
+  // (one structure for all sets: set 0's plan stands for every set's)
+  std::vector<double> touched(ng, 0.0);
+  for (size_t g = 0; g < ng; ++g)
     if (!b->gates[g].plans.empty()) touched[g] = b->gates[g].plans[0].touched;
-  plan_pass_set(b->nq, b->dt, b->nsets, b->nt, b->toff, b->targets, touched, &b->passes);
-  if (b->passes.total && hipMalloc(&b->dev_pass, b->passes.total) != hipSuccess) {
-    (void)hipGetLastError();
-    b->dev_pass = nullptr;
-    without_passes(b->nt.size(), &b->passes);
-  }
-  batch_in_pass(b);
-}
-
-// The device data of a batch's steps; gate by gate where there is no room for
-// the passes' matrices (6 KiB or more a block and set) beside the rest.
-static int upload_batch_steps(Batch *b, const double *matrices, hipStream_t st) {
   while (true) {
-    int rc = SQ_OK;
-    if (b->dev_pass)
-      rc = upload_pass_set(b->passes, b->dt, b->nsets,
-                           PassGates{matrices, &b->moffs, &b->toff, &b->targets, &b->nt, b->nq},
-                           b->set_doubles, b->dev_pass, st);
+    choose_passes(touched, &b->passes);
+    b->in_pass.assign(ng, 0);
+    for (size_t i = 0; i < b->passes.plans.size(); ++i)
+      if (b->passes.use[i])
+        for (int g : b->passes.plans[i].gates) b->in_pass[g] = 1;
+    int rc = upload_pass_set(b->passes, b->dt, b->nsets,
+                             PassGates{matrices, &b->moffs, &b->toff, &b->targets, &b->nt, b->nq},
+                             b->set_doubles, st);
     std::vector<char> img;
     if (rc == SQ_OK) rc = batch_tables(b, &img);
     if (rc == SQ_OK) rc = upload_batch(b, img, st);
-    if (rc != SQ_ERR_OOM || !b->dev_pass) return rc;
-    SQ_HIP(hipFree(b->dev_pass));
-    b->dev_pass = nullptr;
-    without_passes(b->nt.size(), &b->passes);
-    batch_in_pass(b);
+    if (rc != SQ_ERR_OOM || !b->passes.total) return rc;
+    without_passes(ng, &b->passes);
   }
 }
 
 static int batch_launches(Batch *b, void *states, hipStream_t st) {
   const uint64_t n = 1ull << b->nq;
   const char *d = (const char *)b->dev;
+  auto gate = [&](int g) -> int {
+    const Batch::Gate &gt = b->gates[g];
+    if (gt.plans.empty()) return SQ_OK;
+    return launch_batch_gate(gt.plans[0], b->dt, n, b->nsets, states, d + gt.tab_off,
+                             gt.blk_off == (size_t)-1 ? nullptr : d + gt.blk_off, gt.gstride, st);
+  };
   for (const Step &s : b->passes.steps) {
-    if (s.pass >= 0) {
-      SQ_TRY(launch_pass_step(b->passes, s.pass, b->dt, states, n, b->nsets, b->dev_pass, st));
-      continue;
-    }
-    const Batch::Gate &gt = b->gates[s.gate];
-    if (gt.plans.empty()) continue;
-    SQ_TRY(launch_batch_gate(gt.plans[0], b->dt, n, b->nsets, states, d + gt.tab_off,
-                             gt.blk_off == (size_t)-1 ? nullptr : d + gt.blk_off, gt.gstride,
-                             st));
+    if (s.pass < 0)
+      SQ_TRY(gate(s.gate));
+    else if (b->passes.use[s.pass])
+      SQ_TRY(launch_pass_step(b->passes, s.pass, b->dt, states, n, b->nsets, st));
+    else
+      for (int g : b->passes.plans[s.pass].gates) SQ_TRY(gate(g));
   }
   return SQ_OK;
 }
@@ -2397,10 +2403,10 @@ int sq_batch_create(void **batch, sq_dtype_t dt, uint32_t nq, uint32_t nsets, ui
   }
   b->set_doubles = moff;
   SQ_TRY(plan_batch(b.get(), matrices));
-  plan_batch_passes(b.get());
-  const int rc = upload_batch_steps(b.get(), matrices, nullptr);
+  plan_pass_set(b->nq, dt, nsets, b->nt, b->toff, b->targets, &b->passes);
+  const int rc = build_batch_steps(b.get(), matrices, nullptr);
   if (rc != SQ_OK) {
-    if (b->dev_pass) (void)hipFree(b->dev_pass);
+    free_passes(&b->passes);
     if (b->dev) (void)hipFree(b->dev);
     return rc;
   }
@@ -2416,7 +2422,7 @@ int sq_batch_set_matrices(void *batch, const double *matrices, void *stream) {
   drop_batch_graph(b);
   // work already queued on `stream` may still read the old tables: the new
   // ones are copied behind it
-  return upload_batch_steps(b, matrices, (hipStream_t)stream);
+  return build_batch_steps(b, matrices, (hipStream_t)stream);
 }
 
 int sq_batch_run(void *batch, void *states, uint64_t n, void *stream) {
@@ -2468,7 +2474,7 @@ int sq_batch_destroy(void *batch) {
   Batch *b = (Batch *)batch;
   if (!b) return SQ_OK;
   drop_batch_graph(b);
-  if (b->dev_pass) SQ_HIP(hipFree(b->dev_pass));
+  free_passes(&b->passes);
   if (b->dev) SQ_HIP(hipFree(b->dev));
   delete b;
   return SQ_OK;

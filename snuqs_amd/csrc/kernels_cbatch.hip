@@ -270,7 +270,7 @@ static int cbatch_build(CBatch *B, const CBInput &in, bool with_passes) try {
     for (size_t g = 0; g < ng; ++g)
       for (int b = 0; b < plans[j][g].kk; ++b) masks[g] |= 1ull << plans[j][g].tbit[b];
     std::vector<Step> st;
-    plan_passes((int)nq[j], cb, dt, masks, nullptr, &st, &passes[j]);
+    plan_passes((int)nq[j], cb, dt, masks, false, &st, &passes[j]);
     steps = std::max(steps, passes[j].size());
   }
   // matrices in the state's precision, tables per launch

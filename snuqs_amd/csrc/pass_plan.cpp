@@ -119,8 +119,8 @@ int pass_chunk_bits(sq_dtype_t dt, int nbits) {
   return std::min(nbits, nbits >= (dt == SQ_COMPLEX64 ? 20 : 21) ? cmax : cmax - 1);
 }
 
-void plan_passes(int nq, int cb, sq_dtype_t dt, const std::vector<uint64_t> &masks,
-                 const double *touched, std::vector<Step> *steps, std::vector<PassPlan> *passes) {
+void plan_passes(int nq, int cb, sq_dtype_t dt, const std::vector<uint64_t> &masks, bool alone,
+                 std::vector<Step> *steps, std::vector<PassPlan> *passes) {
   steps->clear();
   passes->clear();
   const int ng = (int)masks.size();
@@ -142,7 +142,6 @@ void plan_passes(int nq, int cb, sq_dtype_t dt, const std::vector<uint64_t> &mas
     ++left;
     for (uint64_t m = masks[g]; m; m &= m - 1) pl.perbit[__builtin_ctzll(m)].push_back(g);
   }
-  bool phases_placed = phases.empty();
   std::vector<int> t2, btaken;
   while (left) {
     // seed: the earliest ready gate
@@ -183,29 +182,37 @@ void plan_passes(int nq, int cb, sq_dtype_t dt, const std::vector<uint64_t> &mas
       ptr = bptr;
       taken.insert(taken.end(), btaken.begin(), btaken.end());
     }
-    double sweeps = 0.0;
-    if (touched)
-      for (int g : taken) sweeps += touched[g];
-    if (!touched || (taken.size() >= 2 && sweeps > 1.0)) {
+    if (!alone || taken.size() >= 2) {
       PassPlan p;
       for (int b = 0; b < nq && __builtin_popcountll(set) < cb; ++b) set |= 1ull << b;
       p.local = set;
       p.cb = cb;
       make_blocks(taken, masks, set, &p.blocks);
-      if (!phases_placed) {
-        p.blocks[0].gates.insert(p.blocks[0].gates.end(), phases.begin(), phases.end());
-        phases_placed = true;
-      }
+      p.gates = taken;
       steps->push_back({-1, (int)passes->size()});
       passes->push_back(std::move(p));
     } else {
-      for (int g : taken) steps->push_back({g, -1});
+      steps->push_back({taken[0], -1});
     }
     pl.ptr = ptr;
     left -= (int)taken.size();
   }
-  if (!phases_placed)
+  if (passes->empty()) {
     for (int g : phases) steps->push_back({g, -1});
+    return;
+  }
+  // global phases ride in the pass of most gates
+  PassPlan &most = *std::max_element(
+      passes->begin(), passes->end(),
+      [](const PassPlan &a, const PassPlan &b) { return a.gates.size() < b.gates.size(); });
+  most.gates.insert(most.gates.end(), phases.begin(), phases.end());
+  most.blocks[0].gates.insert(most.blocks[0].gates.end(), phases.begin(), phases.end());
+}
+
+bool pass_pays(const PassPlan &p, const std::vector<double> &touched) {
+  double sweeps = 0.0;
+  for (int g : p.gates) sweeps += touched[g];
+  return sweeps > 1.0;
 }
 
 PassGeom pass_geom(const PassPlan &p) {

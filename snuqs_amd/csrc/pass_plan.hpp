@@ -28,6 +28,7 @@ struct PassBlockPlan {
 struct PassPlan {
   uint64_t local = 0;  // state bits that vary inside a chunk
   int cb = 0;          // their number
+  std::vector<int> gates;  // in an order that gives the same product
   std::vector<PassBlockPlan> blocks;
 };
 
@@ -44,12 +45,15 @@ int pass_chunk_bits(sq_dtype_t dt, int nbits);
 
 // Steps of a gate list on an nq-bit state in chunks of 2^cb amplitudes (cb <=
 // nq; every step is one gate when cb < pass_min_bits).  masks[g]: the state
-// bits gate g acts on (0 for a global phase); touched[g]: the fraction of the
-// amplitudes it changes, or nullptr where gates have no kernels of their own
-// and every step is to be a pass.  Gates are reordered only past gates they
-// share no bit with.
-void plan_passes(int nq, int cb, sq_dtype_t dt, const std::vector<uint64_t> &masks,
-                 const double *touched, std::vector<Step> *steps, std::vector<PassPlan> *passes);
+// bits gate g acts on (0 for a global phase).  alone: gates have kernels of their
+// own, and a gate that no other joins is a step of one gate instead of a pass.
+// Gates are reordered only past gates they share no bit with.
+void plan_passes(int nq, int cb, sq_dtype_t dt, const std::vector<uint64_t> &masks, bool alone,
+                 std::vector<Step> *steps, std::vector<PassPlan> *passes);
+
+// Whether a pass moves less than its gates would on their own kernels, gate g
+// changing the fraction touched[g] of the amplitudes.
+bool pass_pays(const PassPlan &p, const std::vector<double> &touched);
 
 // Device form of one block: byte offsets in the chunk's LDS image that the
 // block's column (group), wave and row (amplitude) index bits stand for; an

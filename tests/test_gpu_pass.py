@@ -79,6 +79,65 @@ def _library(C):
     return L
 
 
+def _rotations(C, n, th):
+    """Gates that are the identity at angle 0."""
+    g = C.operation.gate_operations
+    ops = [g.RotX([q], float(th[q])) for q in range(n)]
+    ops += [g.XX([q, q + 1], float(th[n + q])) for q in range(n - 1)]
+    return ops + [g.RotZ([q], float(th[q] * th[n - 1 - q])) for q in range(n)]
+
+
+# rounding tells a plan from another, so equal bits are equal steps
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+def test_steps_follow_the_matrices(C, dtype):
+    """A program's steps are those of a program made with its present matrices,
+    whatever it was made with (angles of 0 and others)."""
+    n = 12
+    th = [np.zeros(2 * n)] + list(np.random.default_rng(5).uniform(0.1, 3, (2, 2 * n)))
+    fresh = []
+    for t in th:
+        sv = device_state(C, n, dtype)
+        C.functionals.Program(n, _rotations(C, n, t), dtype=dtype).run(sv)
+        fresh.append(to_np(C, sv))
+    for order in ((0, 1, 2), (1, 0, 2, 1)):
+        prog = C.functionals.Program(n, _rotations(C, n, th[order[0]]), dtype=dtype)
+        for i in order:
+            prog.set_gates(_rotations(C, n, th[i]))
+            for use_graph in (False, True):
+                sv = device_state(C, n, dtype)
+                prog.run(sv, use_graph=use_graph)
+                assert np.array_equal(to_np(C, sv), fresh[i]), (order, i, use_graph)
+
+
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+def test_batch_steps_follow_the_matrices(C, dtype):
+    from snuqs_amd.batch import BatchProgram, StateBatch
+
+    n, sets = 12, 3
+    rng = np.random.default_rng(6)
+    zero = np.zeros((sets, 2 * n))
+    some = rng.uniform(0.1, 3, (sets, 2 * n))
+    mixed = some * (np.arange(sets) % 2)[:, None]  # set 0 (and 2) at zero beside another
+    states = StateBatch(sets, n, dtype=dtype)
+
+    def run(b, use_graph=False):
+        states.initialize_basis_z()
+        b.run(states, use_graph=use_graph)
+        return np.array(states.cpu(), copy=True)
+
+    def circuits(th):
+        return [_rotations(C, n, t) for t in th]
+
+    fresh = {name: run(BatchProgram(n, circuits(th), dtype=dtype))
+             for name, th in (("zero", zero), ("some", some), ("mixed", mixed))}
+    th = {"zero": zero, "some": some, "mixed": mixed}
+    b = BatchProgram(n, circuits(zero), dtype=dtype)
+    for name in ("some", "zero", "mixed", "zero", "some"):
+        b.set_gates(circuits(th[name]))
+        for use_graph in (False, True):
+            assert np.array_equal(run(b, use_graph), fresh[name]), (name, use_graph)
+
+
 def _gate_arrays(ops):
     return (np.array([len(op.targets) for op in ops], np.uint32),
             np.array([q for op in ops for q in op.targets], np.uint32),

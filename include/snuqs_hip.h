@@ -151,7 +151,9 @@ int sq_program_destroy(void *program);
  * copy is ordered after the work already queued on `stream` and the call
  * returns when it is done; work on other streams that runs this program must
  * have finished.  A captured hipGraph is dropped (recaptured on the next
- * sq_program_run_graph); tuned launch shapes are kept. */
+ * sq_program_run_graph); tuned launch shapes are kept.  The passes of
+ * sq_program_run get their matrices in the next run, which returns when they are
+ * copied; while a caller captures that run's stream, it runs gate by gate. */
 int sq_program_set_matrices(void *program, const double *matrices, void *stream);
 /* Number of gate sweeps of a run (one kernel launch each when the gates run
  * one by one, as in sq_program_run_timed; sq_program_run applies several gates

@@ -7,6 +7,7 @@
 // The reference exits the process on any CUDA error (utils_cuda.h:8-17); here
 // every entry point returns a status and records a message instead.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -427,6 +428,8 @@ struct Program {
   uint64_t launches = 0;
   double bytes = 0.0;
   PassSet passes;                      // the forward run's steps
+  std::atomic<bool> stale{false};      // `passes` is of earlier matrices
+  std::mutex build_mutex;              // of the run that brings it up to date
   // hipGraph of the forward launch sequence on one state (sq_program_run_graph)
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
@@ -558,9 +561,35 @@ static int build_passes(Program *p, hipStream_t st) {
   return SQ_OK;
 }
 
-// The program's forward launches: its steps.
+// Bring the passes up to the program's matrices, in the first run after they
+// changed: programs that only the adjoint runs on never need them.  *capturing:
+// not done, since `st` is being captured.
+static int update_passes(Program *p, hipStream_t st, bool *capturing) {
+  *capturing = false;
+  if (!p->stale.load(std::memory_order_acquire)) return SQ_OK;
+  std::lock_guard<std::mutex> lk(p->build_mutex);
+  if (!p->stale.load(std::memory_order_relaxed)) return SQ_OK;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (st) SQ_HIP(hipStreamIsCapturing(st, &cs));
+  if (cs != hipStreamCaptureStatusNone) {
+    *capturing = true;
+    return SQ_OK;
+  }
+  SQ_TRY(build_passes(p, st));
+  p->stale.store(false, std::memory_order_release);
+  return SQ_OK;
+}
+
+// The program's forward launches: its steps (gate by gate where a caller captures
+// the first run after new matrices).
 static int program_launches(Program *p, void *sv, uint64_t n, hipStream_t st) {
   auto gate = [&](int g) { return launch_plan(p->fwd[g], sv, p->dt, n, st, p->fwd_dev[g]); };
+  bool capturing;
+  SQ_TRY(update_passes(p, st, &capturing));
+  if (capturing) {
+    for (size_t g = 0; g < p->fwd.size(); ++g) SQ_TRY(gate((int)g));
+    return SQ_OK;
+  }
   for (const Step &s : p->passes.steps) {
     if (s.pass < 0)
       SQ_TRY(gate(s.gate));
@@ -634,13 +663,17 @@ int sq_program_set_matrices(void *program, const double *matrices, void *stream)
   // the blocks may still be read by work queued on `stream`; the new image is
   // copied behind it, and the call returns once the copy is done
   SQ_TRY(plan_program(p, matrices));
+  const bool was_stale = p->stale.exchange(true);
   drop_graph(p);  // kernel arguments (1-3 target matrices) changed
   std::vector<char> img = program_image(p);
   if (p->dev_cap) {
     SQ_HIP(hipMemcpyAsync(p->dev_mats, img.data(), p->dev_cap, hipMemcpyHostToDevice, st));
     SQ_HIP(hipStreamSynchronize(st));
   }
-  return build_passes(p, st);
+  // the next run writes the passes' matrices, on any stream: what reads the old
+  // ones now has to be done
+  if (!was_stale && p->passes.dev) SQ_HIP(hipStreamSynchronize(st));
+  return SQ_OK;
 }
 
 int sq_program_destroy(void *program) {
@@ -847,6 +880,8 @@ int sq_program_run_graph(void *program, void *sv, uint64_t n, void *stream) {
     // capture on a private stream (thread-local mode: other threads' work is
     // not pulled in); the graph holds only kernel launches
     drop_graph(p);
+    bool capturing;
+    SQ_TRY(update_passes(p, (hipStream_t)stream, &capturing));
     hipStream_t cs;
     SQ_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
     int rc = SQ_OK;

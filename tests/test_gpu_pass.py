@@ -138,6 +138,57 @@ def test_batch_steps_follow_the_matrices(C, dtype):
             assert np.array_equal(run(b, use_graph), fresh[name]), (name, use_graph)
 
 
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+def test_new_matrices_then_a_callers_capture(C, dtype):
+    """The first run after set_gates inside a graph that the caller captures,
+    and later runs on two streams at once."""
+    import threading
+
+    n = 14
+    th = np.random.default_rng(9).uniform(0, 3, (2, 2 * n))
+    prog = C.functionals.Program(n, _rotations(C, n, th[0]), dtype=dtype)
+    ref = run_oracle(n, _rotations(C, n, th[1]))
+    sv = device_state(C, n, dtype)
+    prog.run(sv)
+    prog.set_gates(_rotations(C, n, th[1]))
+    L = _library(C)  # (finds the HIP runtime that the engine runs on)
+    L.hipStreamBeginCapture.argtypes = [P, ctypes.c_int]
+    L.hipStreamEndCapture.argtypes = [P, ctypes.POINTER(P)]
+    L.hipGraphInstantiate.argtypes = [ctypes.POINTER(P), P, P, P, ctypes.c_size_t]
+    L.hipGraphLaunch.argtypes = [P, P]
+    L.hipGraphExecDestroy.argtypes = L.hipGraphDestroy.argtypes = [P]
+    stream = C.stream.Stream.create_nonblocking()
+    graph, executable = P(), P()
+    C.core.cuda.device_synchronize()
+    assert L.hipStreamBeginCapture(stream.get(), 0) == 0  # global mode
+    C.functionals.initialize_basis_z(sv, stream=stream)
+    prog.run(sv, stream=stream)
+    assert L.hipStreamEndCapture(stream.get(), ctypes.byref(graph)) == 0
+    assert L.hipGraphInstantiate(ctypes.byref(executable), graph, None, None, 0) == 0
+    for _ in range(3):
+        assert L.hipGraphLaunch(executable, stream.get()) == 0
+        C.core.cuda.device_synchronize()
+        assert np.abs(to_np(C, sv) - ref).max() <= TOL[dtype]
+        C.functionals.norm2(sv)
+    L.hipGraphExecDestroy(executable)
+    L.hipGraphDestroy(graph)
+    # eager again, from two threads at once
+    svs = [device_state(C, n, dtype) for _ in range(2)]
+    C.core.cuda.device_synchronize()
+    streams = [C.stream.Stream.create() for _ in svs]
+    threads = [threading.Thread(target=prog.run, args=(s,), kwargs={"stream": st})
+               for s, st in zip(svs, streams)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    C.core.cuda.device_synchronize()
+    fresh = device_state(C, n, dtype)
+    C.functionals.Program(n, _rotations(C, n, th[1]), dtype=dtype).run(fresh)
+    for s in svs:
+        assert np.array_equal(to_np(C, s), to_np(C, fresh))
+
+
 def _gate_arrays(ops):
     return (np.array([len(op.targets) for op in ops], np.uint32),
             np.array([q for op in ops for q in op.targets], np.uint32),

@@ -165,7 +165,10 @@ int sq_program_stats(void *program, uint64_t *num_launches,
  * into passes: the gates of a pass act inside chunks of up to 2^13 amplitudes
  * held on chip, so the state is read and written once per pass.  Gates are
  * reordered only past gates they share no target with.  A pass whose gates, with
- * their present matrices, touch no more than the state once runs gate by gate. */
+ * their present matrices, touch no more than the state once runs gate by gate.
+ * A pass mixes all amplitudes of a block: an infinite or NaN amplitude, or in
+ * complex64 a part above 3.396e38, spreads over the amplitudes that it shares
+ * blocks with as NaN, and complex64 amplitudes below 2^-108 lose bits. */
 int sq_program_run(void *program, void *sv, uint64_t num_elems, void *stream);
 /* sq_program_run through a hipGraph (no reference counterpart; the reference
  * launches one kernel per Python call, simulation.py:274-284): the launch

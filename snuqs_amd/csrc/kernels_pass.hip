@@ -69,9 +69,13 @@ __device__ __forceinline__ uint32_t xor_lane(const uint16_t *w, uint32_t v) {
 }
 
 // complex64 products run on the bf16 matrix instructions (16 times the FP32
-// rate) with every FP32 operand split in three bf16 parts, x = x0 + x1 + x2 to
-// 2^-27 of x: the six products of parts i + j <= 2 are summed in FP32, and the
-// dropped ones are below 2^-26 of |g x|, under the rounding of an FP32 product.
+// rate) with every FP32 operand split in three bf16 parts: the six products of
+// parts i + j <= 2 are summed in FP32.  Each part is a nearest 8-bit value, so |x1|
+// <= 2^-8 |x0| and |x2| <= 2^-17 |x0|: x0 + x1 + x2 is x (24 bits), or the FP64
+// matrix entry to 2^-26, and a sum of six products is within 2^-24 of g x (the
+// bound of an FP32 product's rounding), 2^-27 root mean square over random
+// operands.  Parts are exact for |x| from 2^-108 (below, x2 is subnormal) to
+// 3.396e38 (above, x0 is infinite).
 // The matrix parts come from its FP64 entries (pass_image).  Error of a layered
 // circuit against 64 bits (2-norm): 14 qubits 6.3e-7 -> 3.6e-7, 23 qubits 7.4e-7
 // -> 4.3e-7, 30 qubits 7.9e-7 -> 4.7e-7 against the FP32 instructions with three

@@ -364,3 +364,53 @@ def test_circuit_batch_without_room_for_passes(C, little_memory, dtype):
         for y in (0, 1, 2, circuits - 1):
             got = b.state(y).astype(np.complex128)
             assert np.abs(got - run_oracle(n, different[y % 3])).max() <= TOL[dtype], (y, use_graph)
+
+
+def _phases_and_permutations(C, n, rng, gates=25):
+    """Gates that move and turn amplitudes without mixing them."""
+    g = C.operation.gate_operations
+    ops = []
+    for _ in range(gates):
+        q = [int(x) for x in rng.permutation(n)[:3]]
+        a = float(rng.uniform(0.1, 3))
+        ops.append([lambda: g.PauliX(q[:1]), lambda: g.S(q[:1]), lambda: g.T(q[:1]),
+                    lambda: g.RotZ(q[:1], a), lambda: g.CX(q[:2]), lambda: g.CPhaseShift(q[:2], a),
+                    lambda: g.Swap(q[:2]), lambda: g.ISwap(q[:2]), lambda: g.ZZ(q[:2], a),
+                    lambda: g.CCNot(q)][int(rng.integers(10))]())
+    return ops
+
+
+# every chunk size of both types
+@pytest.mark.parametrize("dtype,n", [("complex64", 10), ("complex64", 11), ("complex64", 14),
+                                     ("complex64", 20), ("complex128", 9), ("complex128", 10),
+                                     ("complex128", 14), ("complex128", 21)])
+def test_large_amplitudes(C, dtype, n):
+    """Amplitudes up to bf16's largest value (complex64) and to the largest
+    double keep their values beside ordinary ones."""
+    rng = np.random.default_rng(n)
+    ops = _phases_and_permutations(C, n, rng)
+    init = random_state(n, rng, np.dtype(dtype))
+    init[rng.permutation(1 << n)[:4]] = np.array([1, -1, 1j, -1j]) * (
+        3.38e38 if dtype == "complex64" else 1.7e308)
+    alone = device_state(C, n, dtype, init)
+    for op in ops:
+        C.functionals.apply(alone, op, n, op.targets)
+    together = device_state(C, n, dtype, init)
+    C.functionals.Program(n, ops, dtype=dtype).run(together)
+    got, ref = to_np(C, together) * 2.0 ** -10, to_np(C, alone) * 2.0 ** -10
+    # 25 products of an amplitude with a number of modulus 1
+    tol = (1e-5 if dtype == "complex64" else 1e-13) * np.abs(ref).clip(2.0 ** (-n / 2 - 10))
+    assert (np.abs(got - ref) <= tol).all()
+
+
+def test_small_complex64_amplitudes(C):
+    """The three bf16 parts of an amplitude hold its 24 bits down to 2^-108."""
+    n = 12
+    rng = np.random.default_rng(n)
+    ops = _small_gates(n, 20, 3)
+    init = (random_state(n, rng) * 2.0 ** -100).astype(np.complex64)  # 2^-106 each
+    sv = device_state(C, n, "complex64", init)
+    C.functionals.Program(n, ops, dtype="complex64").run(sv)
+    ref = run_oracle(n, ops, init.astype(np.complex128))
+    # 20 roundings of 2^-24, as at any other scale
+    assert np.linalg.norm(to_np(C, sv) - ref) <= 20 * 2.0 ** -24 * np.linalg.norm(ref)

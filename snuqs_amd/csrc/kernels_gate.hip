@@ -1593,16 +1593,22 @@ uint64_t mfma_wave_tiles(uint64_t total_tiles) {
   return t;
 }
 
-// Ordinary instead of non-temporal accesses where the state stays in the 256 MiB
-// Infinity Cache from one gate to the next (28 and more one-gate calls on one
-// state, us): 16 MiB complex128 207 against 200 non-temporal, 32 MiB complex64
-// 328 / 354, 64 MiB 519 / 650, 128 MiB 1044 / 1260, 256 MiB complex128 1863 /
-// 2351, 512 MiB complex64 4330 / 4652, 1 GiB complex128 11878 / 11569.
-static bool sweep_cached(uint64_t bytes) { return bytes >= 32ull << 20 && bytes <= 512ull << 20; }
+// Ordinary instead of non-temporal accesses for a gate that touches no more than
+// the 256 MiB of the Infinity Cache on a state larger than the L2s hold (8 x 4
+// MiB).  Non-temporal against ordinary, calls of a rotation, a dense two-qubit and
+// a CX gate on random qubits: 32 MiB states 1.29-1.35, 1.24-1.31 and 1.05-1.11
+// times as long, 256 MiB 1.16-1.18, 1.15-1.34 and 1.29-1.35; 512 MiB 0.92-0.95,
+// 0.91-0.93 and (a CX touches half) 0.92-1.11, a rotated qubit entangled with all
+// others 1.08-1.15 by this rule and 1.02-1.09 with all gates ordinary; 1 GiB
+// 0.90-0.95 for all.  Below 32 MiB: 16 MiB 0.93 (complex64) and 0.99 (complex128),
+// 8 MiB and less 1.00-1.02.
+static bool sweep_cached(uint64_t bytes, double touched) {
+  return bytes >= 32ull << 20 && touched * (double)bytes <= (double)(256ull << 20);
+}
 
 int launch_plan(const GatePlan &p, void *sv, sq_dtype_t dt, uint64_t nelems,
                 hipStream_t stream, const void *dev_matrix) {
-  const bool cached = sweep_cached(nelems * itemsize(dt));
+  const bool cached = sweep_cached(nelems * itemsize(dt), p.touched);
   if (dt == SQ_COMPLEX64) {
     const auto launch = cached ? launch_plan_t<float, false> : launch_plan_t<float, true>;
     return launch(p, (float2 *)sv, nelems, stream, (const float *)dev_matrix);

@@ -280,6 +280,32 @@ def test_gates_with_ordinary_accesses(C, dtype, n):
     assert np.abs(to_np(C, sv) - run_oracle(n, ops, init.astype(np.complex128))).max() <= TOL[dtype]
 
 
+# 512 MiB: gates that touch half of it or less are read with ordinary accesses,
+# full sweeps are not
+@pytest.mark.parametrize("dtype,n", [("complex128", 25), ("complex64", 26)])
+def test_gates_on_a_state_beyond_the_caches(C, dtype, n):
+    from snuqs_amd._C.operation import gate_operations as g
+
+    small = 6  # the same gates on the qubits that they touch
+    where = [0, 3, 10, n - 9, n - 2, n - 1]
+    rng = np.random.default_rng(n)
+    gates = [lambda q: g.RotY(q[:1], 0.7), lambda q: g.CX(q[:2]), lambda q: g.CZ(q[:2]),
+             lambda q: g.RotZ(q[:1], 0.3), lambda q: g.Swap(q[:2]), lambda q: g.CCNot(q[:3])]
+    sv = device_state(C, n, dtype)
+    ops = []
+    for i in range(36):
+        q = [int(x) for x in rng.permutation(small)]
+        ops.append(gates[i % 6](q))
+        op = gates[i % 6]([where[x] for x in q])
+        C.functionals.apply(sv, op, n, op.targets)
+    ref = run_oracle(small, ops)
+    index = [sum(((i >> (small - 1 - j)) & 1) << (n - 1 - where[j]) for j in range(small))
+             for i in range(1 << small)]
+    got = np.array(C.functionals.amplitudes(sv, index))
+    assert np.abs(got - ref).max() <= TOL[dtype]
+    assert abs(C.functionals.norm2(sv) - 1) <= TOL[dtype]
+
+
 @pytest.fixture
 def little_memory(C):
     """take(mib): device memory taken until that many MiB or less are left."""

@@ -462,15 +462,23 @@ __global__ void SQ_PASS_BOUNDS
                         reinterpret_cast<const nt_f4 *>(images + e.image), e.initial != 0, lds);
 }
 
-// Ordinary instead of non-temporal accesses: states of up to 1 MiB (the L2s:
-// 16 qubits complex64 70.8 against 74.3 us a circuit) and of 64-256 MiB (the
-// Infinity Cache: 23, 24 and 25 qubits complex64 426 / 427, 809 / 850 and 1597 /
-// 1695 us); between them and above they are slower (8 MiB 122 / 120, 16 MiB
-// 174 / 158 and complex128 235 / 184, 32 MiB 268 / 262, 512 MiB 4925 / 4880).
+// Ordinary instead of non-temporal accesses: states of up to 2 MiB, half of what
+// each XCD's L2 holds, and those above what the eight L2s hold together (32 MiB)
+// that fit the Infinity Cache (256 MiB).  (In between, a chunk's lines presumably lie
+// in the L2 of another XCD, which had them in the last pass.)  Non-temporal over
+// ordinary time,
+// layered circuits as programs, complex64 / complex128: 128 KiB 1.03-1.04 / 1.04-1.05,
+// 1 MiB 1.03-1.04 / 1.02-1.04, 2 MiB 1.03 / 1.03, 4 MiB 1.00-1.01 / 1.00-1.01, 8 MiB
+// 0.98-1.00 / 0.96-0.97, 16 MiB 0.94 / 0.86-0.88, 32 MiB 1.01-1.10 / 0.98-0.99, 64 MiB
+// 1.02 / 0.98-1.00, 128 MiB 1.06-1.08 / 1.03-1.04, 256 MiB 1.07-1.08 / 1.05-1.07, 512
+// MiB 0.99 / 0.98-0.99.  Parameter batches by all their states: up to 2 MiB 1.00, 4-16
+// MiB 0.85-0.96, 64-256 MiB 1.01-1.07 / 1.02, 512 MiB 0.98 / 0.99.  Circuit batches: up
+// to 2 MiB 1.00-1.02, 8-32 MiB 0.79-0.99, 64-128 MiB 1.02-1.05 / 0.98-0.99, 256 MiB
+// 0.99 / 0.99: complex128 ones stay non-temporal above 2 MiB.
 // The choice is a template argument: the compiler merges accesses that differ
 // in this hint alone.
 static bool pass_cached(uint64_t bytes) {
-  return bytes <= 1ull << 20 || (bytes >= 64ull << 20 && bytes <= 256ull << 20);
+  return bytes <= 2ull << 20 || (bytes > 32ull << 20 && bytes <= 256ull << 20);
 }
 
 template <typename R, int CB>
@@ -505,7 +513,8 @@ uint64_t pass_entry_launches(uint64_t nwg) { return (nwg + kPassGrid - 1) / kPas
 int launch_pass_entries(int cb, sq_dtype_t dt, void *states, const PassEntry *entries,
                         const uint32_t *entry, const PassBlock *blocks, const void *images,
                         uint64_t nwg, hipStream_t st) {
-  const bool cached = pass_cached((nwg << cb) * itemsize(dt));
+  const uint64_t bytes = (nwg << cb) * itemsize(dt);
+  const bool cached = pass_cached(bytes) && (dt == SQ_COMPLEX64 || bytes <= 2ull << 20);
 #define SQ_PASS(R, CB)                                                                          \
   hipLaunchKernelGGL((cached ? k_pass_entries<R, CB, false> : k_pass_entries<R, CB, true>),     \
                      dim3((unsigned)std::min(nwg - w0, kPassGrid)), dim3(PassShape<R, CB>::NT), \

@@ -31,7 +31,7 @@ def _circuit(n, rng, gates):
 
 
 # 8 / 9: below the smallest chunk of complex128 / complex64; 9-13: the state is
-# one chunk; 20 / 21: the largest chunk starts at 21 qubits
+# one chunk; 20 / 21: the largest chunk starts at 20 (complex64) and 21 qubits
 @pytest.mark.parametrize("dtype", ["complex128", "complex64"])
 @pytest.mark.parametrize("n", [8, 9, 10, 11, 12, 13, 14, 17, 20, 21])
 def test_program_passes_vs_oracle(C, dtype, n):
@@ -249,7 +249,7 @@ def test_unaligned_batch_states(C, dtype, at):
     L.sq_batch_destroy(batch)
 
 
-# 64 MiB: the smallest state above 1 MiB that passes read with ordinary accesses
+# 64 MiB: the smallest state above 2 MiB that passes read with ordinary accesses
 @pytest.mark.parametrize("dtype,n", [("complex128", 22), ("complex64", 23)])
 def test_passes_with_ordinary_accesses(C, dtype, n):
     rng = np.random.default_rng(n)

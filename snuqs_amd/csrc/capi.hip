@@ -2197,7 +2197,7 @@ int sq_cbatch_destroy(void *batch) { return cbatch_destroy(batch); }
 // ---- parameter batches ---------------------------------------------------------
 // One circuit structure, many parameter sets: nsets states of 2^nq amplitudes
 // in one device allocation (state y at y * 2^nq), each evolved by the same
-// gates with its own matrices, one launch per gate for the whole batch.
+// gates with its own matrices, one launch per pass or gate for the whole batch.
 namespace sq {
 
 struct Batch {

@@ -1093,7 +1093,7 @@ PYBIND11_MODULE(_C, m) {
            "One gate list per parameter set (same gates and targets, own matrices).")
       .def("run", &BatchProgram::run, py::arg("states"), py::kw_only(),
            py::arg("use_graph") = false, py::arg("stream") = nullptr,
-           "Apply every gate to every state, one launch per gate for the whole batch.")
+           "Apply every gate to every state, one launch per pass of gates for the whole batch.")
       .def("set_gates", &BatchProgram::set_gates, py::arg("parameter_sets"), py::kw_only(),
            py::arg("stream") = nullptr)
       .def("stats", &BatchProgram::stats)
@@ -1126,7 +1126,7 @@ PYBIND11_MODULE(_C, m) {
            "Circuits of uneven qubit counts, [(num_qubits, gates), ...], as one launch sequence.")
       .def("run", &CircuitBatch::run, py::kw_only(), py::arg("use_graph") = true,
            py::arg("stream") = nullptr,
-           "Every state <- |0...0>, then every circuit's gates (launch s: gate s of each circuit).")
+           "Every state <- |0...0>, then every circuit's gates (step s: pass s of each circuit).")
       .def("copy_state", &CircuitBatch::copy_state, py::arg("circuit"), py::arg("sv"),
            py::kw_only(), py::arg("stream") = nullptr,
            "Copy circuit j's state into a device StateVector of its qubit count and dtype.")

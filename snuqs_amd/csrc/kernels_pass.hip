@@ -17,7 +17,7 @@
 // 0-3, 6, 10, 12, ..., 28: no block 3.5 ms, 1 block 3.6, 2 blocks 3.9, 3 blocks
 // 4.9, 4 blocks 6.1 (FP32 instructions: 3.4, 3.6, 4.7, 5.9, 7.4), where one
 // block per launch takes 3.1 ms each.  Layered 30-qubit circuit of depth 10 in
-// 48 blocks: 148 -> 69 ms; 25-qubit mixed circuit of 175 gates unfused: 12.4 ->
+// 48 blocks: 148 -> 71-80 ms by box; 25-qubit mixed circuit of 175 gates unfused: 12.4 ->
 // 1.1 ms.  A loop over several chunks per workgroup with the next chunk's loads
 // issued ahead of the products (4 waves, 2 tiles each) measured 5-10% slower
 // than one chunk per workgroup: the two workgroups of a CU already overlap

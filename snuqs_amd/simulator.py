@@ -10,8 +10,9 @@ program as a JSON dict (or string), or an OpenQASM 3 program (an object or dict
 with ``source`` and ``inputs``, or the source text; read by
 ``snuqs_amd.openqasm``, run_openqasm at simulator.py:380-437), and returns a
 ``TaskResult`` with the same fields as GateModelTaskResult.  Extra keyword arguments: ``precision``
-("complex64" / "complex128"), ``fuse`` (largest fused block, 0 = off) and
-``exact_sampling``.
+("complex64" / "complex128"), ``fuse`` (largest fused block, 0 = off; states of
+10 qubits and more run several gates to a pass over the state whatever it is)
+and ``exact_sampling``.
 
 Differences from the reference, by design: the engine runs on the GPU
 (accelerator None / "cuda" / "hip"); accelerator "hybrid" or offload "cpu"

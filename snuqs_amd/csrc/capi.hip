@@ -1270,20 +1270,31 @@ static int sample_from(const double *probs, const void *sv, sq_dtype_t dt, int n
   const size_t red_b = (kRedBlocks + 64) * sizeof(double) + 256;
   hipStream_t st = (hipStream_t)stream;
   Workspace *w;
+  // the state's probabilities where a route stores them: as large as the state, so
+  // not kept in the workspace
+  struct Probs {
+    double *p = nullptr;
+    ~Probs() {
+      if (p) (void)hipFree(p);
+    }
+  } pr;
   // route 0: exact samples by tiles; 1: a cdf over all elements (fast mode, and
   // exact mode on entries that are negative or not finite)
   for (int route = exact ? 0 : 1; route < 2; ++route) {
     const size_t scr_b =
         (route ? sample_scratch_bytes(n, exact != 0) : sample_exact_scratch_bytes(n)) + 256;
     const size_t cdf_b = route ? n * sizeof(double) + 256 : 0;
-    const size_t prob_b = route && sv ? n * sizeof(double) + 256 : 0;
-    SQ_TRY(ws_reserve(dev, cdf_b + scr_b + red_b + prob_b + io_b + 1024, io_b, &w));
+    if (route && sv && hipMalloc((void **)&pr.p, n * sizeof(double)) != hipSuccess) {
+      (void)hipGetLastError();
+      pr.p = nullptr;
+      return fail(SQ_ERR_OOM, "sampling: device allocation of the probabilities failed");
+    }
+    SQ_TRY(ws_reserve(dev, cdf_b + scr_b + red_b + io_b + 1024, io_b, &w));
     char *d = (char *)w->dev;
     double *cdf = (double *)d;
     char *scr = al(d + cdf_b);
     double *red = (double *)al(scr + scr_b);
-    double *pr = (double *)al((char *)red + red_b);
-    double *du = (double *)al((char *)pr + prob_b);
+    double *du = (double *)al((char *)red + red_b);
     int64_t *dout = (int64_t *)al((char *)du + shots * 8);
     int bad = 0;
     std::memcpy(w->host, uniforms, shots * 8);
@@ -1298,9 +1309,9 @@ static int sample_from(const double *probs, const void *sv, sq_dtype_t dt, int n
         SQ_TRY(sample_exact(probs, n, du, shots, dout, scr, &bad_dev, st));
       SQ_HIP(hipMemcpyAsync(&bad, bad_dev, sizeof(int), hipMemcpyDeviceToHost, st));
     } else {
-      if (sv && normalize) SQ_TRY(launch_probabilities_div(sv, dt, n, pr, red, st));
-      else if (sv) SQ_TRY(launch_probabilities(sv, dt, n, pr, st));
-      SQ_TRY(sample_cdf(sv ? pr : probs, n, cdf, exact != 0, scr, scr_b, st));
+      if (sv && normalize) SQ_TRY(launch_probabilities_div(sv, dt, n, pr.p, red, st));
+      else if (sv) SQ_TRY(launch_probabilities(sv, dt, n, pr.p, st));
+      SQ_TRY(sample_cdf(sv ? pr.p : probs, n, cdf, exact != 0, scr, scr_b, st));
       SQ_TRY(launch_search(cdf, n, du, shots, dout, st));
     }
     SQ_HIP(hipMemcpyAsync(w->host, dout, shots * 8, hipMemcpyDeviceToHost, st));

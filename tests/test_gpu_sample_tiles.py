@@ -143,3 +143,22 @@ def test_negative_entries_through_the_c_abi(C):
     fast = out.copy()
     assert L.sq_sample(buf.data_ptr, 1 << n, u.ctypes.data, 500, 1, out.ctypes.data, None) == 0
     assert np.abs(out - fast).max() <= 1
+
+
+def test_probabilities_are_given_back(C):
+    """Fast sampling from a state keeps the cdf (8 bytes an element) and some
+    scratch in the workspace, and not the probabilities."""
+    n = 28
+    sv = device_state(C, n, "complex64")
+    u = np.random.default_rng(3).random(100)
+    C.functionals.sample(sv, u, exact=True)
+
+    def free():
+        # (the runtime returns memory with the next allocation and release)
+        other = C.result_types.StateVector(C.DeviceType.CUDA, n, dtype="complex64")
+        del other
+        return C.core.cuda.mem_info()[0]
+
+    before = free()
+    assert (C.functionals.sample(sv, u, exact=False) == 0).all()
+    assert before - free() < 12 << n

@@ -412,7 +412,7 @@ def _phases_and_permutations(C, n, rng, gates=25):
                                      ("complex128", 14), ("complex128", 21)])
 def test_large_amplitudes(C, dtype, n):
     """Amplitudes up to bf16's largest value (complex64) and to the largest
-    double keep their values beside ordinary ones."""
+    double (blocks of 4 targets) keep their values beside ordinary ones."""
     rng = np.random.default_rng(n)
     ops = _phases_and_permutations(C, n, rng)
     init = random_state(n, rng, np.dtype(dtype))
